@@ -179,7 +179,9 @@ PK_API int launch_quantize_int8_per_channel(const uint16_t *W, int8_t *Wq, float
 
 /* Config-2 MLP block: y = add(bias(matmul(gelu(bias(matmul(rmsnorm(x, gamma),
  * W1), b1)), W2), b2), x).  x [M,d], W1 [d,F], W2 [F,d].  `workspace` must
- * hold pk_mlp_block_workspace_size(M, d, F) bytes. */
+ * hold pk_mlp_block_workspace_size(M, d, F) bytes (the normalised rows and the
+ * hidden activations, 2 M (d + F) bytes in 256-byte units, are required; the
+ * split partials behind them are used where the workspace holds them). */
 PK_API size_t pk_mlp_block_workspace_size(int M, int d, int F);
 PK_API int launch_mlp_block(const uint16_t *x, const uint16_t *gamma, const uint16_t *W1,
                      const uint16_t *b1, const uint16_t *W2, const uint16_t *b2, uint16_t *out,

@@ -143,7 +143,25 @@ int gelu_table(const uint16_t **table) {
   return PK_OK;
 }
 
-int library_workspace(size_t bytes, void *st, WorkspaceLease &lease) {
+namespace {
+// Whether memory can't be allocated now because `st` is being captured (or its
+// state can't be told, as on the null stream beside a capturing one).
+bool capturing(void *st) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(static_cast<hipStream_t>(st), &s) == hipSuccess) return s != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+size_t ws_round(size_t bytes) {
+  size_t n = size_t(1) << 20;
+  while (n < bytes) n <<= 1;
+  return n;
+}
+}  // namespace
+
+int library_workspace(size_t bytes, void *st, WorkspaceLease &lease) { return library_workspace(bytes, bytes, st, lease); }
+
+int library_workspace(size_t need, size_t want, void *st, WorkspaceLease &lease) {
   int dev = 0;
   PK_HIP(hipGetDevice(&dev));
   if (dev < 0 || dev >= kMaxDevices) {
@@ -164,15 +182,19 @@ int library_workspace(size_t bytes, void *st, WorkspaceLease &lease) {
     if (!slot->released) break;
     lk.unlock();  // released between the lookup and the lock: take the slot that replaced it
   }
-  if (slot->bytes < bytes) {
-    size_t want = size_t(1) << 20;
-    while (want < bytes) want <<= 1;
+  auto grow = [&](size_t bytes) -> hipError_t {
     void *p = nullptr;
-    PK_HIP(hipMalloc(&p, want));
+    const hipError_t e = hipMalloc(&p, ws_round(bytes));
+    if (e != hipSuccess) return e;
     if (slot->ptr) slot->retired.push_back(slot->ptr);
     slot->ptr = p;
-    slot->bytes = want;
-  }
+    slot->bytes = ws_round(bytes);
+    return e;
+  };
+  // beyond `need` only where it can be had: not during a capture, not when memory is short
+  if (want > need && slot->bytes < want && !capturing(st) && grow(want) != hipSuccess) (void)hipGetLastError();
+  if (slot->bytes < need) PK_HIP(grow(need));
+  lease.bytes = slot->bytes;
   lease.ptr = slot->ptr;
   lease.keep = slot;
   lease.lock = std::move(lk);

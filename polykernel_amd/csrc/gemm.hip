@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "gemm_kernels.hpp"
+#include "gemm_stream.hpp"
 
 namespace pk {
 
@@ -40,6 +41,17 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_kernel(GemmArgs g) {
 template <int EPI, int STAGES, int W = G2_WAVES, int WNN = G2_WAVES_N>
 __global__ __launch_bounds__(W * 64, 1) void gemm_dma_kernel(GemmArgs g) {
   gemm_dma_body<EPI, STAGES, W, WNN>(g);
+}
+
+template <int NT, int MT, int WK, int STAGES, int EPI>
+__global__ __launch_bounds__(WK * 64) void gemm_stream_kernel(GemmStreamArgs a) {
+  gemm_stream_body<NT, MT, WK, STAGES, EPI>(a);
+}
+
+constexpr int GS_REDUCE_THREADS = 128;
+template <int EPI>
+__global__ __launch_bounds__(GS_REDUCE_THREADS) void gemm_reduce_kernel(GemmArgs g, const float *partial, int splits) {
+  gemm_reduce_body<EPI>(g, partial, splits);
 }
 
 template <int BM, int BN, int WM, int WN, int EPI>
@@ -66,14 +78,19 @@ int tile_grid_ok(int M, int N, int K, int bm, int bn, const char *name) {
   return PK_ERR_UNSUPPORTED;
 }
 
+// Whether every operand and every row of it can be read and written in 16-byte
+// vectors.
+bool gemm_vec_ok(const GemmArgs &g) {
+  return (g.K % 8 == 0) && (g.N % 8 == 0) && aligned16(g.A) && aligned16(g.B) && aligned16(g.C) &&
+         (!g.R || aligned16(g.R)) && (!g.bias || aligned16(g.bias));
+}
+
 // Whether tile 0 runs the direct-to-LDS 256x256 kernel for these operands
 // (otherwise the register-staged one).
 bool gemm_dma_fits(const GemmArgs &g) {
-  const bool aligned = (g.K % 8 == 0) && (g.N % 8 == 0) && aligned16(g.A) && aligned16(g.B);
   const bool offsets32 = (size_t)g.K * g.N * 2 < (size_t(1) << 31) &&
                          (size_t)G2_BM * g.K * 2 < (size_t(1) << 31);
-  const bool ep_aligned = aligned16(g.C) && (!g.R || aligned16(g.R)) && (!g.bias || aligned16(g.bias));
-  return aligned && ep_aligned && offsets32 && g.K % G2_BK == 0 && g.N >= 8;
+  return gemm_vec_ok(g) && offsets32 && g.K % G2_BK == 0 && g.N >= 8;
 }
 
 template <int EPI>
@@ -138,6 +155,109 @@ int gemm_launch_variant(const GemmArgs &g, int v, bool vec, hipStream_t st) {
   }
 }
 
+// ---- decode-sized calls (gemm_stream.hpp) -----------------------------------
+// The streaming kernel's variants, by slice width (16 * nt columns) and rows
+// (16 * mt): WK waves and STAGES ring stages, chosen so that two workgroups
+// fit a CU's LDS where the width allows it.  `rate` is the weight bytes per ns
+// one workgroup draws, fitted to [16, N, K] for N 512-16384, K 768-16384
+// (narrow slices read short runs: 32 bytes per weight row at nt 1).
+struct StreamVariant {
+  int nt, mt;
+  double rate;
+  void (*fn[4])(dim3, hipStream_t, const GemmStreamArgs &);
+};
+template <int NT, int MT, int WK, int STAGES, int EPI>
+void stream_launch(dim3 grid, hipStream_t st, const GemmStreamArgs &a) {
+  gemm_stream_kernel<NT, MT, WK, STAGES, EPI><<<grid, WK * 64, 0, st>>>(a);
+}
+#define PK_GS(NT, MT, WK, S, RATE)                                                                    \
+  {                                                                                                   \
+    NT, MT, RATE, {                                                                                   \
+      stream_launch<NT, MT, WK, S, EPI_NONE>, stream_launch<NT, MT, WK, S, EPI_BIAS_GELU>,            \
+          stream_launch<NT, MT, WK, S, EPI_BIAS_RESID>, stream_launch<NT, MT, WK, S, EPI_RESID>       \
+    }                                                                                                 \
+  }
+const StreamVariant kStream[] = {
+    PK_GS(4, 1, 4, 3, 28.0), PK_GS(8, 1, 4, 2, 40.0), PK_GS(2, 1, 8, 3, 15.5), PK_GS(1, 1, 8, 8, 8.3),
+    PK_GS(4, 2, 4, 3, 24.0), PK_GS(8, 2, 4, 3, 36.0), PK_GS(2, 2, 8, 3, 13.0), PK_GS(1, 2, 8, 4, 7.0),
+    PK_GS(4, 4, 4, 3, 19.0), PK_GS(8, 4, 2, 4, 30.0), PK_GS(2, 4, 8, 3, 10.0), PK_GS(1, 4, 8, 4, 6.0),
+};
+#undef PK_GS
+constexpr int kStreamRows = 64;
+
+struct StreamPlan {
+  const StreamVariant *v = nullptr;
+  int splits = 1, split_steps = 0, slices = 0;
+};
+
+// Whether the streaming kernel takes the shape (operands 16-byte aligned).
+bool stream_shape_ok(int M, int N, int K) {
+  return M <= kStreamRows && N % 8 == 0 && K % 8 == 0 && (size_t)K * N * 2 < (size_t(1) << 31);
+}
+
+// Slice width and K splits by a time model (us) fitted to the same sweep: 3
+// for the launch, the larger of the HBM time of all weights (5.7 TB/s; A's own
+// loads cost 0.35 of the weights' per byte) and of the busiest CU's units, and
+// for a split 2.5 for the reduction's launch plus its partials at 5 TB/s.
+// Rows of N * 2 bytes that do not start on 128-byte lines share lines between
+// slices: the wide slice then streams at 0.9, the others at 0.72 ([8, 50256,
+// 2048]: 44.9 us with 128 columns, 60.0 with 64).  Splits use at most
+// `scratch` bytes of partials.
+bool stream_plan(int M, int N, int K, size_t scratch, StreamPlan &best) {
+  if (!stream_shape_ok(M, N, K)) return false;
+  const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+  const int ksteps = (K + GS_KSTEP - 1) / GS_KSTEP;
+  double best_us = 0;
+  for (const StreamVariant &v : kStream) {
+    if (v.mt != mt) continue;
+    const int nb = 16 * v.nt, slices = (N + nb - 1) / nb;
+    const double a_share = 1.0 + 0.35 * (v.mt - 1) / v.nt;
+    const double line = N % 64 == 0 ? 1.0 : v.nt == 8 ? 0.9 : 0.72;
+    const double hbm = (double)N * K * 2 * a_share / (5.7e6 * line);
+    for (int s : {1, 2, 3, 4, 6, 8, 12, 14, 16}) {
+      const int steps = (ksteps + s - 1) / s;
+      if (s > 1 && steps < 8) break;
+      const int splits = (ksteps + steps - 1) / steps;
+      const size_t part = splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
+      if (part > scratch) break;
+      const double rounds = std::ceil((double)slices * splits / 256);
+      double us = 3.0 + std::max(hbm, rounds * steps * GS_KSTEP * nb * 2 / (v.rate * 1e3 * line));
+      if (splits > 1) us += 2.5 + 2.0 * part / 5e6;
+      if (!best.v || us < best_us * (1 - 1e-9)) {
+        best_us = us;
+        best = StreamPlan{&v, splits, steps, slices};
+      }
+    }
+  }
+  return best.v != nullptr;
+}
+
+int stream_run(int epi, const GemmArgs &g, const StreamPlan &p, void *scratch, hipStream_t st) {
+  const GemmStreamArgs a{g, static_cast<float *>(scratch), p.splits, p.split_steps, p.slices};
+  p.v->fn[epi](dim3(p.slices * p.splits, (g.M + 16 * p.v->mt - 1) / (16 * p.v->mt)), st, a);
+  PK_LAUNCH_CHECK("gemm_stream_kernel");
+  if (p.splits == 1) return PK_OK;
+  const int64_t items = (int64_t)g.M * g.N / 8;
+  const int blocks = (int)std::min<int64_t>((items + GS_REDUCE_THREADS - 1) / GS_REDUCE_THREADS, 4096);
+  switch (epi) {
+    case EPI_NONE: gemm_reduce_kernel<EPI_NONE><<<blocks, GS_REDUCE_THREADS, 0, st>>>(g, a.partial, p.splits); break;
+    case EPI_BIAS_GELU: gemm_reduce_kernel<EPI_BIAS_GELU><<<blocks, GS_REDUCE_THREADS, 0, st>>>(g, a.partial, p.splits); break;
+    case EPI_BIAS_RESID: gemm_reduce_kernel<EPI_BIAS_RESID><<<blocks, GS_REDUCE_THREADS, 0, st>>>(g, a.partial, p.splits); break;
+    default: gemm_reduce_kernel<EPI_RESID><<<blocks, GS_REDUCE_THREADS, 0, st>>>(g, a.partial, p.splits); break;
+  }
+  PK_LAUNCH_CHECK("gemm_reduce_kernel");
+  return PK_OK;
+}
+
+// Bytes of split partials the built-in choice wants for aligned operands (0:
+// none); a caller with less scratch gets the best choice within it.
+constexpr size_t kStreamScratchMax = size_t(64) << 20;
+size_t gemm_scratch_bytes(int M, int N, int K) {
+  StreamPlan p;
+  if (M <= 0 || N <= 0 || K <= 0 || !stream_plan(M, N, K, kStreamScratchMax, p) || p.splits == 1) return 0;
+  return (size_t)p.splits * M * N * sizeof(float);
+}
+
 // Largest tile that still gives at least ~one workgroup per CU.
 // With the direct-to-LDS kernel (`dma`), 256x256 from 72 tiles up: even one
 // round that leaves most CUs idle beats the 128x128 kernel's rounds (K 4096:
@@ -173,7 +293,9 @@ int gemm_configs(int M, int N, int K, pk_config *out, int cap) {
   return n;
 }
 
-// What gemm_run picks for 16-byte aligned operands.
+// The tile gemm_run picks for 16-byte aligned operands above kStreamRows rows.
+// Fewer rows take the streaming kernel, which is no configuration of the
+// tuning cache: the tile returned here is then the one a cache entry serves.
 bool gemm_default(int M, int N, int K, pk_config *out) {
   if (M <= 0 || N <= 0 || K <= 0) return false;
   const int vw = (K % 8 == 0 && N % 8 == 0) ? 8 : 1;
@@ -226,12 +348,17 @@ int gemm_run_config(int epi, const uint16_t *A, const uint16_t *B, uint16_t *C, 
 }
 
 int gemm_run(int epi, const uint16_t *A, const uint16_t *B, uint16_t *C, const uint16_t *bias,
-             const uint16_t *R, int M, int N, int K, hipStream_t st, int tile = -1) {
+             const uint16_t *R, int M, int N, int K, hipStream_t st, int tile = -1, void *scratch = nullptr,
+             size_t scratch_bytes = 0) {
   if (int rc = tile_grid_ok(M, N, K, 64, 64, "matmul")) return rc;
   GemmArgs g{A, B, C, bias, R, nullptr, M, N, K};
   if (epi == EPI_BIAS_GELU) {
     int rc = gelu_table(&g.gelu_tab);
     if (rc) return rc;
+  }
+  if (tile < 0 && M <= kStreamRows && gemm_vec_ok(g)) {
+    StreamPlan p;
+    if (stream_plan(M, N, K, aligned16(scratch) ? scratch_bytes : 0, p)) return stream_run(epi, g, p, scratch, st);
   }
   if (tile < 0) tile = pick_tile(M, N, gemm_dma_fits(g));
   switch (epi) {
@@ -292,14 +419,18 @@ int fused_rmsnorm_matmul(const uint16_t *x, const uint16_t *gamma, const uint16_
     PK_LAUNCH_CHECK(name);
     return PK_OK;
   }
-  // Otherwise: normalise once into library workspace, then the plain GEMM.
+  // Otherwise: normalise once into library workspace, then the plain GEMM, its
+  // split partials behind the rows where the workspace can hold them too.
   WorkspaceLease lease;  // held until the GEMM that reads the panel is queued
-  int rc = library_workspace((size_t)M * K * 2, st, lease);
+  const size_t row_bytes = ((size_t)M * K * 2 + 255) & ~size_t(255);
+  const size_t part = gemm_scratch_bytes(M, N, K);
+  int rc = library_workspace((size_t)M * K * 2, part ? row_bytes + part : (size_t)M * K * 2, st, lease);
   if (rc) return rc;
   uint16_t *a = static_cast<uint16_t *>(lease.ptr);
   rc = rmsnorm_launch(x, gamma, a, M, K, eps, st);
   if (rc) return rc;
-  return gemm_run(EPI_NONE, a, W, out, nullptr, nullptr, M, N, K, st);
+  return gemm_run(EPI_NONE, a, W, out, nullptr, nullptr, M, N, K, st, -1, static_cast<char *>(lease.ptr) + row_bytes,
+                  lease.bytes >= row_bytes + part ? part : 0);
 }
 
 }  // namespace pk
@@ -347,10 +478,16 @@ int launch_fused_rmsnorm_matmul_gamma(const uint16_t *x, const uint16_t *gamma, 
                               "launch_fused_rmsnorm_matmul_gamma");
 }
 
-size_t pk_mlp_block_workspace_size(int M, int d, int F) {
-  if (M <= 0 || d <= 0 || F <= 0) return 0;  // no launch takes a workspace
+// The normalised rows and the hidden activations: what launch_mlp_block cannot
+// do without.  Workspace beyond it holds split partials.
+static size_t mlp_rows_bytes(int M, int d, int F) {
   auto up = [](size_t v) { return (v + 255) & ~size_t(255); };
   return up((size_t)M * d * 2) + up((size_t)M * F * 2);
+}
+
+size_t pk_mlp_block_workspace_size(int M, int d, int F) {
+  if (M <= 0 || d <= 0 || F <= 0) return 0;  // no launch takes a workspace
+  return mlp_rows_bytes(M, d, F) + std::max(gemm_scratch_bytes(M, F, d), gemm_scratch_bytes(M, d, F));
 }
 
 int launch_mlp_block(const uint16_t *x, const uint16_t *gamma, const uint16_t *W1,
@@ -361,7 +498,7 @@ int launch_mlp_block(const uint16_t *x, const uint16_t *gamma, const uint16_t *W
   PK_CHECK_ARG(M >= 0 && d > 0 && F > 0, "launch_mlp_block: invalid shape");
   if (M == 0) return PK_OK;
   if (int rc = tile_grid_ok(M, std::max(d, F), std::max(d, F), 64, 64, "launch_mlp_block")) return rc;  // before any launch
-  const size_t need = pk_mlp_block_workspace_size(M, d, F);
+  const size_t need = mlp_rows_bytes(M, d, F);
   if (!workspace || workspace_bytes < need) {
     set_error("launch_mlp_block: workspace of %zu bytes required, got %zu", need, workspace_bytes);
     return PK_ERR_WORKSPACE;
@@ -371,9 +508,10 @@ int launch_mlp_block(const uint16_t *x, const uint16_t *gamma, const uint16_t *W
   uint16_t *h = a + (((size_t)M * d * 2 + 255) & ~size_t(255)) / 2;
   int rc = rmsnorm_launch(x, gamma, a, M, d, eps, st);
   if (rc) return rc;
-  rc = gemm_run(EPI_BIAS_GELU, a, W1, h, b1, nullptr, M, F, d, st);
+  void *scratch = static_cast<char *>(workspace) + need;
+  rc = gemm_run(EPI_BIAS_GELU, a, W1, h, b1, nullptr, M, F, d, st, -1, scratch, workspace_bytes - need);
   if (rc) return rc;
-  return gemm_run(EPI_BIAS_RESID, h, W2, out, b2, x, M, d, F, st);
+  return gemm_run(EPI_BIAS_RESID, h, W2, out, b2, x, M, d, F, st, -1, scratch, workspace_bytes - need);
 }
 
 // Test/tuning hook: run one GEMM epilogue variant with an explicit tile choice

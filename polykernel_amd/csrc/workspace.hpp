@@ -25,6 +25,7 @@ namespace pk {
 // streams call it before destroying one.
 struct WorkspaceLease {
   void *ptr = nullptr;
+  size_t bytes = 0;                    // of the whole buffer
   std::shared_ptr<void> keep;          // keeps the slot alive while the lock is held
   std::unique_lock<std::mutex> lock;   // destroyed first (members unwind in reverse)
 };
@@ -32,6 +33,10 @@ struct WorkspaceLease {
 // `stream` is the hipStream_t the caller will launch on (nullptr: the null
 // stream).  Returns a PK_* status.
 int library_workspace(size_t bytes, void *stream, WorkspaceLease &lease);
+// The same for a caller that works with `need` bytes and better with `want`:
+// the buffer grows to `want` unless the stream is being captured or memory is
+// short (lease.bytes tells), and is refused only where `need` would be.
+int library_workspace(size_t need, size_t want, void *stream, WorkspaceLease &lease);
 
 // Frees the calling device's slot of `stream` after hipStreamSynchronize on
 // it; the next call on that stream allocates again.  PK_OK when there is no

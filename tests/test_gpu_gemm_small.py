@@ -1,0 +1,113 @@
+"""GEMMs of at most 64 rows (the weight-streaming kernel): every slice width,
+row block and epilogue at ragged edges, with and without K splits."""
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+
+from polykernel_amd import synth
+from tests.bounds import _gate_bad
+from tests.helpers import bf, from_dev, int_bf16, rng_bf16, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+# rows at the edges of the 16-row blocks; K a multiple of 32 or only of 8 (40,
+# 520: a last step with 8 rows); N within one slice, ragged, and with whole
+# slices of 128, 64, 32 and 16 columns (50256, 16384, 8192, 3072)
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
+@pytest.mark.parametrize("N,Kd", [(8, 8), (8, 40), (264, 512), (1000, 520), (3072, 768), (8192, 1032),
+                                  (16384, 256), (50256, 40)])
+def test_small_m_gemm_integer_bit_exact(gpu, oracle, M, N, Kd):
+    from polykernel_amd import kernels
+
+    print(f"small gemm {M}x{N}x{Kd}", flush=True)
+    a, b = int_bf16((M, Kd), 114), int_bf16((Kd, N), 115)
+    bias, r = bf(np.random.default_rng(116).integers(-4, 5, size=N)), rng_bf16((M, N), 117)
+    da, db, dbias, dr = map(to_dev, (a, b, bias, r))
+    assert np.array_equal(from_dev(kernels.matmul(da, db)), oracle.matmul(a, b))
+    assert np.array_equal(from_dev(kernels.fused_matmul_bias_gelu(da, db, dbias)),
+                          oracle.fused_matmul_bias_gelu(a, b, bias))
+    for bb, dbb in ((bias, dbias), (None, None)):
+        assert np.array_equal(from_dev(kernels.fused_matmul_bias_residual(da, db, dbb, dr)),
+                              oracle.fused_matmul_bias_residual(a, b, bb, r))
+
+
+def test_small_m_gemm_rows_past_k_do_not_leak(gpu, oracle):
+    """K = 40 leaves 24 rows of the last 32-row step past K; the memory a
+    clamped load repeats there holds infinities, which must not reach a sum."""
+    from polykernel_amd import kernels
+
+    M, N, Kd = 5, 72, 40
+    a, b = int_bf16((M, Kd), 118), int_bf16((Kd, N), 119)
+    b[Kd - 1] = 0x7F80  # +inf weights in the last valid row, against zero and nonzero activations
+    a[:, Kd - 1] = 0x3F80
+    a[2, Kd - 1] = 0  # 0 * inf = NaN
+    got, want = from_dev(kernels.matmul(to_dev(a), to_dev(b))), oracle.matmul(a, b)
+    assert np.array_equal(got[[0, 1, 3, 4]], want[[0, 1, 3, 4]])
+    assert np.all((got[2] & 0x7F80) == 0x7F80) and np.all(got[2] & 0x7F)
+
+
+# (M, d, F): K splits in both products, in one of them, ragged widths and K
+@pytest.mark.parametrize("M,d,F", [(1, 512, 2048), (16, 1024, 4096), (17, 768, 3072), (33, 520, 2056),
+                                   (64, 2048, 1000), (5, 4096, 512), (64, 4096, 4096)])
+def test_small_m_mlp_block_stages(gpu, M, d, F):
+    """launch_mlp_block's two GEMMs, each held to the fp32 error model on the
+    operands it read (from the workspace), with the whole workspace and with
+    only the rows (no room for split partials)."""
+    import torch
+
+    from polykernel_amd import _lib, kernels
+
+    lib = _lib.load()
+    x = to_dev(synth.normal_bf16((M, d), 140))
+    g = to_dev(synth.normal_bf16((d,), 141, 0.1, 1.0))
+    w1, w2 = (to_dev(synth.normal_bf16(s, 142 + i, 1 / np.sqrt(s[0]))) for i, s in enumerate(((d, F), (F, d))))
+    b1, b2 = to_dev(synth.normal_bf16((F,), 144, 0.02)), to_dev(synth.normal_bf16((d,), 145, 0.02))
+    up = lambda v: (v + 255) & ~255  # noqa: E731
+    rows = up(2 * M * d) + up(2 * M * F)
+    assert lib.pk_mlp_block_workspace_size(M, d, F) >= rows
+    for size in (lib.pk_mlp_block_workspace_size(M, d, F), rows):
+        ws = torch.full((size,), 0xFF, dtype=torch.uint8, device="cuda")
+        out = torch.empty_like(x)
+        _lib.check(lib.launch_mlp_block(x.data_ptr(), g.data_ptr(), w1.data_ptr(), b1.data_ptr(), w2.data_ptr(),
+                                        b2.data_ptr(), out.data_ptr(), M, d, F, ctypes.c_float(1e-6), ws.data_ptr(),
+                                        size, torch.cuda.current_stream().cuda_stream), "launch_mlp_block")
+        a = ws[:2 * M * d].view(torch.bfloat16).view(M, d)
+        h = ws[up(2 * M * d):up(2 * M * d) + 2 * M * F].view(torch.bfloat16).view(M, F)
+        assert torch.equal(a, kernels.rmsnorm(x, g, 1e-6))
+        assert _gate_bad(1, a.contiguous(), w1, h.contiguous(), bias=b1) == 0, (M, d, F, size)
+        assert _gate_bad(2, h.contiguous(), w2, out, bias=b2, r=x) == 0, (M, d, F, size)
+    assert lib.launch_mlp_block(x.data_ptr(), g.data_ptr(), w1.data_ptr(), b1.data_ptr(), w2.data_ptr(),
+                                b2.data_ptr(), out.data_ptr(), M, d, F, ctypes.c_float(1e-6), ws.data_ptr(),
+                                rows - 1, None) == _lib.PK_ERR_WORKSPACE
+
+
+@pytest.mark.parametrize("M,N,Kd", [(16, 768, 3072), (33, 2048, 4096), (7, 512, 1032)])
+def test_small_m_rmsnorm_matmul_split(gpu, M, N, Kd):
+    """RMSNorm -> MatMul with the split partials behind the normalised rows in
+    the library workspace, eager and captured (the replay keeps the eager bits)."""
+    import torch
+
+    from polykernel_amd import kernels
+
+    x = to_dev(synth.normal_bf16((M, Kd), 150))
+    g = to_dev(synth.normal_bf16((Kd,), 151, 0.1, 1.0))
+    w = to_dev(synth.normal_bf16((Kd, N), 152, 1 / np.sqrt(Kd)))
+    got = kernels.fused_rmsnorm_matmul(x, w, g, 1e-6)
+    assert _gate_bad(0, kernels.rmsnorm(x, g, 1e-6), w, got) == 0
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        kernels.fused_rmsnorm_matmul(x, w, g, 1e-6)
+        torch.cuda.synchronize()
+        gr = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(gr, stream=s):
+            out = kernels.fused_rmsnorm_matmul(x, w, g, 1e-6)
+    for _ in range(3):
+        out.fill_(0)
+        gr.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), got.view(torch.int16))
+        assert torch.equal(kernels.fused_rmsnorm_matmul(x, w, g, 1e-6).view(torch.int16), got.view(torch.int16))
