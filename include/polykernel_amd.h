@@ -247,7 +247,9 @@ typedef struct pk_config {
  * PK_ERR_INVALID_ARG for an unknown op.  No device is needed. */
 PK_API int pk_op_configs(const char *op, long long M, long long N, long long K, pk_config *out, int cap);
 /* The configuration the op's plain entry point chooses for 16-byte aligned
- * operands (PK_ERR_UNSUPPORTED when it takes a generic fallback kernel). */
+ * operands (PK_ERR_UNSUPPORTED when it takes a generic fallback kernel).
+ * GEMMs of few rows or few tiles run kernels that are no configuration (K
+ * split over waves and workgroups): for those it is the nearest tile. */
 PK_API int pk_op_default_config(const char *op, long long M, long long N, long long K, pk_config *out);
 
 /* The configuration launch_matmul_int8 would use for this shape (returns

@@ -23,7 +23,7 @@
 #include <type_traits>
 
 #include "gemm_kernels.hpp"
-#include "gemm_stream.hpp"
+#include "gemm_ring.hpp"
 
 namespace pk {
 
@@ -46,6 +46,11 @@ __global__ __launch_bounds__(W * 64, 1) void gemm_dma_kernel(GemmArgs g) {
 template <int NT, int MT, int WK, int STAGES, int EPI>
 __global__ __launch_bounds__(WK * 64) void gemm_stream_kernel(GemmStreamArgs a) {
   gemm_stream_body<NT, MT, WK, STAGES, EPI>(a);
+}
+
+template <int FM, int WN, int STAGES, int EPI>
+__global__ __launch_bounds__(GR_THREADS, 1) void gemm_ring_kernel(GemmRingArgs a) {
+  gemm_ring_body<FM, WN, STAGES, EPI>(a);
 }
 
 constexpr int GS_REDUCE_THREADS = 128;
@@ -232,30 +237,127 @@ bool stream_plan(int M, int N, int K, size_t scratch, StreamPlan &best) {
   return best.v != nullptr;
 }
 
-int stream_run(int epi, const GemmArgs &g, const StreamPlan &p, void *scratch, hipStream_t st) {
-  const GemmStreamArgs a{g, static_cast<float *>(scratch), p.splits, p.split_steps, p.slices};
-  p.v->fn[epi](dim3(p.slices * p.splits, (g.M + 16 * p.v->mt - 1) / (16 * p.v->mt)), st, a);
-  PK_LAUNCH_CHECK("gemm_stream_kernel");
-  if (p.splits == 1) return PK_OK;
+int reduce_run(int epi, const GemmArgs &g, const float *partial, int splits, hipStream_t st) {
   const int64_t items = (int64_t)g.M * g.N / 8;
   const int blocks = (int)std::min<int64_t>((items + GS_REDUCE_THREADS - 1) / GS_REDUCE_THREADS, 4096);
   switch (epi) {
-    case EPI_NONE: gemm_reduce_kernel<EPI_NONE><<<blocks, GS_REDUCE_THREADS, 0, st>>>(g, a.partial, p.splits); break;
-    case EPI_BIAS_GELU: gemm_reduce_kernel<EPI_BIAS_GELU><<<blocks, GS_REDUCE_THREADS, 0, st>>>(g, a.partial, p.splits); break;
-    case EPI_BIAS_RESID: gemm_reduce_kernel<EPI_BIAS_RESID><<<blocks, GS_REDUCE_THREADS, 0, st>>>(g, a.partial, p.splits); break;
-    default: gemm_reduce_kernel<EPI_RESID><<<blocks, GS_REDUCE_THREADS, 0, st>>>(g, a.partial, p.splits); break;
+    case EPI_NONE: gemm_reduce_kernel<EPI_NONE><<<blocks, GS_REDUCE_THREADS, 0, st>>>(g, partial, splits); break;
+    case EPI_BIAS_GELU: gemm_reduce_kernel<EPI_BIAS_GELU><<<blocks, GS_REDUCE_THREADS, 0, st>>>(g, partial, splits); break;
+    case EPI_BIAS_RESID: gemm_reduce_kernel<EPI_BIAS_RESID><<<blocks, GS_REDUCE_THREADS, 0, st>>>(g, partial, splits); break;
+    default: gemm_reduce_kernel<EPI_RESID><<<blocks, GS_REDUCE_THREADS, 0, st>>>(g, partial, splits); break;
   }
   PK_LAUNCH_CHECK("gemm_reduce_kernel");
   return PK_OK;
 }
 
+int stream_run(int epi, const GemmArgs &g, const StreamPlan &p, void *scratch, hipStream_t st) {
+  const GemmStreamArgs a{g, static_cast<float *>(scratch), p.splits, p.split_steps, p.slices};
+  p.v->fn[epi](dim3(p.slices * p.splits, (g.M + 16 * p.v->mt - 1) / (16 * p.v->mt)), st, a);
+  PK_LAUNCH_CHECK("gemm_stream_kernel");
+  return p.splits > 1 ? reduce_run(epi, g, a.partial, p.splits, st) : PK_OK;
+}
+
+// ---- prompt-sized calls (gemm_ring.hpp) -------------------------------------
+// Tiles of 32 fm x 64 wn; `us` is the time of one 64-deep k-tile with a tile
+// on every CU.
+struct RingVariant {
+  int fm, wn;
+  double us;
+  void (*fn[4])(dim3, hipStream_t, const GemmRingArgs &);
+};
+template <int FM, int WN, int STAGES, int EPI>
+void ring_launch(dim3 grid, hipStream_t st, const GemmRingArgs &a) {
+  gemm_ring_kernel<FM, WN, STAGES, EPI><<<grid, GR_THREADS, 0, st>>>(a);
+}
+#define PK_GR(FM, WN, S, US)                                                                \
+  {                                                                                         \
+    FM, WN, US, {                                                                           \
+      ring_launch<FM, WN, S, EPI_NONE>, ring_launch<FM, WN, S, EPI_BIAS_GELU>,              \
+          ring_launch<FM, WN, S, EPI_BIAS_RESID>, ring_launch<FM, WN, S, EPI_RESID>         \
+    }                                                                                       \
+  }
+const RingVariant kRing[] = {PK_GR(2, 2, 4, 0.27), PK_GR(3, 2, 4, 0.375), PK_GR(4, 2, 4, 0.44),
+                             PK_GR(3, 4, 3, 0.67), PK_GR(4, 4, 3, 0.75),  PK_GR(5, 4, 3, 0.925)};
+#undef PK_GR
+
+struct RingPlan {
+  const RingVariant *v = nullptr;
+  int splits = 1, split_tiles = 0, units = 0;
+  double us = 0;
+};
+
+// Tile and K splits by a time model (us) fitted to 60 shapes of 65-3850 rows,
+// N 512-16384 and K 512-16384 (its choice is within 0.7 % of the best variant
+// in the geometric mean, 10 % at worst): 3.6 for the launch and first loads,
+// 1.7 per round of 256 workgroups, per k-tile the variant's time (up to 1.2
+// of it in long launches, where the clock falls), at least the operands'
+// memory time at 9.5 TB/s of a full grid, and for a split 2.8 and its partials
+// written and read at 4.6 TB/s.
+bool ring_plan(int M, int N, int K, size_t scratch, RingPlan &best) {
+  if (N % 8 != 0 || K % 8 != 0 || (size_t)K * N * 2 >= (size_t(1) << 31) || (size_t)160 * K * 2 >= (size_t(1) << 31))
+    return false;
+  const int ktiles = (K + GR_BK - 1) / GR_BK;
+  const double bytes = 2.0 * ((double)N * K + (double)M * K + (double)M * N);
+  for (const RingVariant &v : kRing) {
+    const int64_t tiles = (int64_t)((M + 32 * v.fm - 1) / (32 * v.fm)) * ((N + 64 * v.wn - 1) / (64 * v.wn));
+    for (int s : {1, 2, 3, 4, 6, 8}) {
+      const int steps = (ktiles + s - 1) / s;
+      if (s > 1 && steps < 4) break;
+      const int splits = (ktiles + steps - 1) / steps;
+      const size_t part = splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
+      const int64_t units = tiles * splits;
+      if (part > scratch || units > INT32_MAX / 2 || (splits > 1 && units > 1024)) break;
+      const double rounds = std::ceil(units / 256.0);
+      const double slow = 1.0 + 0.2 * std::min(1.0, (rounds - 1) / 2);
+      double us = 3.6 + 1.7 * rounds +
+                  std::max(rounds * steps * v.us * slow, bytes / (9.5e6 * std::min(1.0, units / 256.0)));
+      if (splits > 1) us += 2.8 + 2.0 * part / 4.6e6;
+      if (!best.v || us < best.us * (1 - 1e-9)) best = RingPlan{&v, splits, steps, (int)units, us};
+    }
+  }
+  return best.v != nullptr;
+}
+
+// The same model of the 256 x 256 kernel: 5.8 us, 2 per round and 0.5 per
+// 32-deep k-tile, up to half as much again in launches of three rounds or more.
+double dma_us(int M, int N, int K) {
+  const double rounds = std::ceil((double)(((int64_t)M + 255) / 256) * (((int64_t)N + 255) / 256) / 256);
+  return 5.8 + rounds * (2.0 + K / 32.0 * 0.5 * (1.0 + 0.5 * std::min(1.0, (rounds - 1) / 2)));
+}
+
+int ring_run(int epi, const GemmArgs &g, const RingPlan &p, void *scratch, hipStream_t st) {
+  const GemmRingArgs a{g, static_cast<float *>(scratch), p.splits, p.split_tiles};
+  p.v->fn[epi](dim3(p.units), st, a);
+  PK_LAUNCH_CHECK("gemm_ring_kernel");
+  return p.splits > 1 ? reduce_run(epi, g, a.partial, p.splits, st) : PK_OK;
+}
+
+// The kernel of the built-in choice for vector-aligned operands and at most
+// `scratch` bytes of partials: the streaming kernel up to kStreamRows rows,
+// above it the ring kernel or, where its model is no slower, the 256 x 256 one
+// (`dma`: it takes these operands).  Neither plan set: the tiles of pick_tile.
+struct GemmPlan {
+  StreamPlan stream;
+  RingPlan ring;
+  size_t part(int M, int N) const {
+    const int s = stream.v ? stream.splits : ring.v ? ring.splits : 1;
+    return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
+  }
+};
+GemmPlan gemm_plan(int M, int N, int K, bool dma, size_t scratch) {
+  GemmPlan p;
+  if (M <= kStreamRows && stream_plan(M, N, K, scratch, p.stream)) return p;
+  if (ring_plan(M, N, K, scratch, p.ring) && dma && dma_us(M, N, K) <= p.ring.us) p.ring = RingPlan{};
+  return p;
+}
+
 // Bytes of split partials the built-in choice wants for aligned operands (0:
 // none); a caller with less scratch gets the best choice within it.
-constexpr size_t kStreamScratchMax = size_t(64) << 20;
+constexpr size_t kGemmScratchMax = size_t(64) << 20;
 size_t gemm_scratch_bytes(int M, int N, int K) {
-  StreamPlan p;
-  if (M <= 0 || N <= 0 || K <= 0 || !stream_plan(M, N, K, kStreamScratchMax, p) || p.splits == 1) return 0;
-  return (size_t)p.splits * M * N * sizeof(float);
+  constexpr int most = INT32_MAX - 1023;  // as tile_grid_ok
+  if (M <= 0 || N <= 0 || K <= 0 || M > most || N > most || K > most) return 0;
+  return gemm_plan(M, N, K, gemm_dma_shape_ok(N, K), kGemmScratchMax).part(M, N);
 }
 
 // Largest tile that still gives at least ~one workgroup per CU.
@@ -293,9 +395,10 @@ int gemm_configs(int M, int N, int K, pk_config *out, int cap) {
   return n;
 }
 
-// The tile gemm_run picks for 16-byte aligned operands above kStreamRows rows.
-// Fewer rows take the streaming kernel, which is no configuration of the
-// tuning cache: the tile returned here is then the one a cache entry serves.
+// The configuration of the tuning cache nearest to what gemm_run picks for
+// 16-byte aligned operands: the streaming and ring kernels are no
+// configurations, so where gemm_plan takes one this is the tile that a cache
+// entry without a sweep would serve.
 bool gemm_default(int M, int N, int K, pk_config *out) {
   if (M <= 0 || N <= 0 || K <= 0) return false;
   const int vw = (K % 8 == 0 && N % 8 == 0) ? 8 : 1;
@@ -356,11 +459,12 @@ int gemm_run(int epi, const uint16_t *A, const uint16_t *B, uint16_t *C, const u
     int rc = gelu_table(&g.gelu_tab);
     if (rc) return rc;
   }
-  if (tile < 0 && M <= kStreamRows && gemm_vec_ok(g)) {
-    StreamPlan p;
-    if (stream_plan(M, N, K, aligned16(scratch) ? scratch_bytes : 0, p)) return stream_run(epi, g, p, scratch, st);
+  if (tile < 0 && gemm_vec_ok(g)) {
+    const GemmPlan p = gemm_plan(M, N, K, gemm_dma_fits(g), aligned16(scratch) ? std::min(scratch_bytes, kGemmScratchMax) : 0);
+    if (p.stream.v) return stream_run(epi, g, p.stream, scratch, st);
+    if (p.ring.v) return ring_run(epi, g, p.ring, scratch, st);
   }
-  if (tile < 0) tile = pick_tile(M, N, gemm_dma_fits(g));
+  if (tile < 0) tile = gemm_dma_fits(g) ? 0 : pick_tile(M, N, false);
   switch (epi) {
     case EPI_NONE: return gemm_dispatch<EPI_NONE>(g, tile, st);
     case EPI_BIAS_GELU: return gemm_dispatch<EPI_BIAS_GELU>(g, tile, st);

@@ -61,9 +61,11 @@ __device__ __forceinline__ int gs_xor(int s) {
   else return s & 7;
 }
 
-// Epilogue of 8 consecutive outputs of row m from their fp32 sums.
+// Epilogue of 8 consecutive outputs of row m from their fp32 sums; `tab` is the
+// GELU table (global or LDS).
 template <int EPI>
-__device__ __forceinline__ void gemm_finish8(const f32x4 v0, const f32x4 v1, int m, int n, const GemmArgs &g) {
+__device__ __forceinline__ void gemm_finish8(const f32x4 v0, const f32x4 v1, int m, int n, const GemmArgs &g,
+                                             const uint16_t *tab) {
 #pragma clang fp contract(off)
   u32x4 t = {pack_bf(v0[0], v0[1]), pack_bf(v0[2], v0[3]), pack_bf(v1[0], v1[1]), pack_bf(v1[2], v1[3])};
   if constexpr (EPI == EPI_BIAS_GELU || EPI == EPI_BIAS_RESID) {
@@ -74,7 +76,7 @@ __device__ __forceinline__ void gemm_finish8(const f32x4 v0, const f32x4 v1, int
   if constexpr (EPI == EPI_BIAS_GELU) {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      t[e] = gelu_bits(t[e] & 0xFFFFu, g.gelu_tab) | (gelu_bits(t[e] >> 16, g.gelu_tab) << 16);
+      t[e] = gelu_pair_exact(t[e], tab);
   }
   if constexpr (EPI == EPI_BIAS_RESID || EPI == EPI_RESID) {
     const u32x4 r = *reinterpret_cast<const u32x4 *>(g.R + (size_t)m * g.N + n);
@@ -99,7 +101,7 @@ __device__ __forceinline__ void gemm_reduce_body(const GemmArgs &g, const float 
       s0 += *reinterpret_cast<const f32x4 *>(q);
       s1 += *reinterpret_cast<const f32x4 *>(q + 4);
     }
-    gemm_finish8<EPI>(s0, s1, (int)(e / g.N), (int)(e % g.N), g);
+    gemm_finish8<EPI>(s0, s1, (int)(e / g.N), (int)(e % g.N), g, g.gelu_tab);
   }
 }
 
@@ -261,7 +263,7 @@ __device__ __forceinline__ void gemm_stream_body(const GemmStreamArgs &a) {
       *reinterpret_cast<f32x4 *>(o) = v0;
       *reinterpret_cast<f32x4 *>(o + 4) = v1;
     } else {
-      gemm_finish8<EPI>(v0, v1, m, n, g);
+      gemm_finish8<EPI>(v0, v1, m, n, g, g.gelu_tab);
     }
   }
 }

@@ -1,5 +1,6 @@
-"""GEMMs of at most 64 rows (the weight-streaming kernel): every slice width,
-row block and epilogue at ragged edges, with and without K splits."""
+"""GEMMs of decode and prompt size (the weight-streaming and the ring kernel):
+every slice width, tile, row block and epilogue at ragged edges, with and
+without K splits."""
 from __future__ import annotations
 
 import ctypes
@@ -21,9 +22,22 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("N,Kd", [(8, 8), (8, 40), (264, 512), (1000, 520), (3072, 768), (8192, 1032),
                                   (16384, 256), (50256, 40)])
 def test_small_m_gemm_integer_bit_exact(gpu, oracle, M, N, Kd):
+    _check_integer(oracle, M, N, Kd)
+
+
+# the ring kernel's six tiles (64 x 128 ... 160 x 256), one row over a tile,
+# K below, at and above a k-tile of 64 with tails of 8 to 56, one and several
+# rounds of a ring slot
+@pytest.mark.parametrize("M,N,Kd", [(65, 8, 8), (97, 136, 72), (129, 264, 520), (272, 6592, 40), (391, 6680, 64),
+                                    (514, 6744, 120), (879, 6456, 72), (1060, 7184, 200), (161, 2056, 1336)])
+def test_ring_gemm_integer_bit_exact(gpu, oracle, M, N, Kd):
+    _check_integer(oracle, M, N, Kd)
+
+
+def _check_integer(oracle, M, N, Kd):
     from polykernel_amd import kernels
 
-    print(f"small gemm {M}x{N}x{Kd}", flush=True)
+    print(f"gemm {M}x{N}x{Kd}", flush=True)
     a, b = int_bf16((M, Kd), 114), int_bf16((Kd, N), 115)
     bias, r = bf(np.random.default_rng(116).integers(-4, 5, size=N)), rng_bf16((M, N), 117)
     da, db, dbias, dr = map(to_dev, (a, b, bias, r))
@@ -35,25 +49,27 @@ def test_small_m_gemm_integer_bit_exact(gpu, oracle, M, N, Kd):
                               oracle.fused_matmul_bias_residual(a, b, bb, r))
 
 
-def test_small_m_gemm_rows_past_k_do_not_leak(gpu, oracle):
-    """K = 40 leaves 24 rows of the last 32-row step past K; the memory a
-    clamped load repeats there holds infinities, which must not reach a sum."""
+@pytest.mark.parametrize("M,N,Kd", [(5, 72, 40), (70, 72, 40), (70, 72, 200)])
+def test_gemm_rows_past_k_do_not_leak(gpu, oracle, M, N, Kd):
+    """The last k-step of a ragged K reaches past it; the memory a clamped load
+    repeats there holds infinities, which must not reach a sum."""
     from polykernel_amd import kernels
 
-    M, N, Kd = 5, 72, 40
     a, b = int_bf16((M, Kd), 118), int_bf16((Kd, N), 119)
     b[Kd - 1] = 0x7F80  # +inf weights in the last valid row, against zero and nonzero activations
     a[:, Kd - 1] = 0x3F80
     a[2, Kd - 1] = 0  # 0 * inf = NaN
     got, want = from_dev(kernels.matmul(to_dev(a), to_dev(b))), oracle.matmul(a, b)
-    assert np.array_equal(got[[0, 1, 3, 4]], want[[0, 1, 3, 4]])
+    rest = np.arange(M) != 2
+    assert np.array_equal(got[rest], want[rest])
     assert np.all((got[2] & 0x7F80) == 0x7F80) and np.all(got[2] & 0x7F)
 
 
 # (M, d, F): K splits in both products, in one of them, ragged widths and K
 @pytest.mark.parametrize("M,d,F", [(1, 512, 2048), (16, 1024, 4096), (17, 768, 3072), (33, 520, 2056),
-                                   (64, 2048, 1000), (5, 4096, 512), (64, 4096, 4096)])
-def test_small_m_mlp_block_stages(gpu, M, d, F):
+                                   (64, 2048, 1000), (5, 4096, 512), (64, 4096, 4096), (65, 512, 2048),
+                                   (100, 768, 3072), (333, 520, 2056), (501, 1024, 4096), (777, 2048, 4096)])
+def test_mlp_block_stages(gpu, M, d, F):
     """launch_mlp_block's two GEMMs, each held to the fp32 error model on the
     operands it read (from the workspace), with the whole workspace and with
     only the rows (no room for split partials)."""
@@ -85,8 +101,8 @@ def test_small_m_mlp_block_stages(gpu, M, d, F):
                                 rows - 1, None) == _lib.PK_ERR_WORKSPACE
 
 
-@pytest.mark.parametrize("M,N,Kd", [(16, 768, 3072), (33, 2048, 4096), (7, 512, 1032)])
-def test_small_m_rmsnorm_matmul_split(gpu, M, N, Kd):
+@pytest.mark.parametrize("M,N,Kd", [(16, 768, 3072), (33, 2048, 4096), (7, 512, 1032), (130, 768, 3072)])
+def test_rmsnorm_matmul_split(gpu, M, N, Kd):
     """RMSNorm -> MatMul with the split partials behind the normalised rows in
     the library workspace, eager and captured (the replay keeps the eager bits)."""
     import torch
