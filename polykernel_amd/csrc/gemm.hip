@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "gemm_kernels.hpp"
+#include "gemm_plan.hpp"
 #include "gemm_ring.hpp"
 
 namespace pk {
@@ -258,64 +259,26 @@ int stream_run(int epi, const GemmArgs &g, const StreamPlan &p, void *scratch, h
 }
 
 // ---- prompt-sized calls (gemm_ring.hpp) -------------------------------------
-// Tiles of 32 fm x 64 wn; `us` is the time of one 64-deep k-tile with a tile
-// on every CU.
-struct RingVariant {
-  int fm, wn;
-  double us;
-  void (*fn[4])(dim3, hipStream_t, const GemmRingArgs &);
-};
+using RingLaunch = void (*)(dim3, hipStream_t, const GemmRingArgs &);
 template <int FM, int WN, int STAGES, int EPI>
 void ring_launch(dim3 grid, hipStream_t st, const GemmRingArgs &a) {
   gemm_ring_kernel<FM, WN, STAGES, EPI><<<grid, GR_THREADS, 0, st>>>(a);
 }
-#define PK_GR(FM, WN, S, US)                                                                \
-  {                                                                                         \
-    FM, WN, US, {                                                                           \
-      ring_launch<FM, WN, S, EPI_NONE>, ring_launch<FM, WN, S, EPI_BIAS_GELU>,              \
-          ring_launch<FM, WN, S, EPI_BIAS_RESID>, ring_launch<FM, WN, S, EPI_RESID>         \
-    }                                                                                       \
+#define PK_GR(FM, WN, S)                                                            \
+  {                                                                                 \
+    ring_launch<FM, WN, S, EPI_NONE>, ring_launch<FM, WN, S, EPI_BIAS_GELU>,        \
+        ring_launch<FM, WN, S, EPI_BIAS_RESID>, ring_launch<FM, WN, S, EPI_RESID>   \
   }
-const RingVariant kRing[] = {PK_GR(2, 2, 4, 0.27), PK_GR(3, 2, 4, 0.375), PK_GR(4, 2, 4, 0.44),
-                             PK_GR(3, 4, 3, 0.67), PK_GR(4, 4, 3, 0.75),  PK_GR(5, 4, 3, 0.925)};
+const RingTile kRing[] = {{2, 2, 0.27}, {3, 2, 0.375}, {4, 2, 0.44}, {3, 4, 0.67}, {4, 4, 0.75}, {5, 4, 0.925}};
+const RingLaunch kRingFn[][4] = {PK_GR(2, 2, 4), PK_GR(3, 2, 4), PK_GR(4, 2, 4),
+                                 PK_GR(3, 4, 3), PK_GR(4, 4, 3), PK_GR(5, 4, 3)};
 #undef PK_GR
 
-struct RingPlan {
-  const RingVariant *v = nullptr;
-  int splits = 1, split_tiles = 0, units = 0;
-  double us = 0;
-};
-
-// Tile and K splits by a time model (us) fitted to 60 shapes of 65-3850 rows,
-// N 512-16384 and K 512-16384 (its choice is within 0.7 % of the best variant
-// in the geometric mean, 10 % at worst): 3.6 for the launch and first loads,
-// 1.7 per round of 256 workgroups, per k-tile the variant's time (up to 1.2
-// of it in long launches, where the clock falls), at least the operands'
-// memory time at 9.5 TB/s of a full grid, and for a split 2.8 and its partials
-// written and read at 4.6 TB/s.
-bool ring_plan(int M, int N, int K, size_t scratch, RingPlan &best) {
-  if (N % 8 != 0 || K % 8 != 0 || (size_t)K * N * 2 >= (size_t(1) << 31) || (size_t)160 * K * 2 >= (size_t(1) << 31))
-    return false;
-  const int ktiles = (K + GR_BK - 1) / GR_BK;
-  const double bytes = 2.0 * ((double)N * K + (double)M * K + (double)M * N);
-  for (const RingVariant &v : kRing) {
-    const int64_t tiles = (int64_t)((M + 32 * v.fm - 1) / (32 * v.fm)) * ((N + 64 * v.wn - 1) / (64 * v.wn));
-    for (int s : {1, 2, 3, 4, 6, 8}) {
-      const int steps = (ktiles + s - 1) / s;
-      if (s > 1 && steps < 4) break;
-      const int splits = (ktiles + steps - 1) / steps;
-      const size_t part = splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
-      const int64_t units = tiles * splits;
-      if (part > scratch || units > INT32_MAX / 2 || (splits > 1 && units > 1024)) break;
-      const double rounds = std::ceil(units / 256.0);
-      const double slow = 1.0 + 0.2 * std::min(1.0, (rounds - 1) / 2);
-      double us = 3.6 + 1.7 * rounds +
-                  std::max(rounds * steps * v.us * slow, bytes / (9.5e6 * std::min(1.0, units / 256.0)));
-      if (splits > 1) us += 2.8 + 2.0 * part / 4.6e6;
-      if (!best.v || us < best.us * (1 - 1e-9)) best = RingPlan{&v, splits, steps, (int)units, us};
-    }
-  }
-  return best.v != nullptr;
+// Fitted to 60 shapes of 65-3850 rows, N 512-16384 and K 512-16384: its choice
+// is within 0.7 % of the best variant in the geometric mean, 10 % at worst.
+constexpr RingModel kRingModel{3.6, 1.7, 0.2, 9.5e6, 2.8, 4.6e6};
+RingChoice ring_plan(int M, int N, int K, size_t scratch) {
+  return ring_choose(kRing, (int)(sizeof kRing / sizeof kRing[0]), kRingModel, M, N, K, 2, scratch);
 }
 
 // The same model of the 256 x 256 kernel: 5.8 us, 2 per round and 0.5 per
@@ -325,9 +288,9 @@ double dma_us(int M, int N, int K) {
   return 5.8 + rounds * (2.0 + K / 32.0 * 0.5 * (1.0 + 0.5 * std::min(1.0, (rounds - 1) / 2)));
 }
 
-int ring_run(int epi, const GemmArgs &g, const RingPlan &p, void *scratch, hipStream_t st) {
-  const GemmRingArgs a{g, static_cast<float *>(scratch), p.splits, p.split_tiles};
-  p.v->fn[epi](dim3(p.units), st, a);
+int ring_run(int epi, const GemmArgs &g, const RingChoice &p, void *scratch, hipStream_t st) {
+  const GemmRingArgs a{g, static_cast<float *>(scratch), p.splits, p.split_tiles, nullptr, nullptr};
+  kRingFn[p.tile][epi](dim3(p.units), st, a);
   PK_LAUNCH_CHECK("gemm_ring_kernel");
   return p.splits > 1 ? reduce_run(epi, g, a.partial, p.splits, st) : PK_OK;
 }
@@ -338,16 +301,17 @@ int ring_run(int epi, const GemmArgs &g, const RingPlan &p, void *scratch, hipSt
 // (`dma`: it takes these operands).  Neither plan set: the tiles of pick_tile.
 struct GemmPlan {
   StreamPlan stream;
-  RingPlan ring;
+  RingChoice ring;
   size_t part(int M, int N) const {
-    const int s = stream.v ? stream.splits : ring.v ? ring.splits : 1;
+    const int s = stream.v ? stream.splits : ring.tile >= 0 ? ring.splits : 1;
     return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
   }
 };
 GemmPlan gemm_plan(int M, int N, int K, bool dma, size_t scratch) {
   GemmPlan p;
   if (M <= kStreamRows && stream_plan(M, N, K, scratch, p.stream)) return p;
-  if (ring_plan(M, N, K, scratch, p.ring) && dma && dma_us(M, N, K) <= p.ring.us) p.ring = RingPlan{};
+  p.ring = ring_plan(M, N, K, scratch);
+  if (dma && dma_us(M, N, K) <= p.ring.us) p.ring = RingChoice{};
   return p;
 }
 
@@ -462,7 +426,7 @@ int gemm_run(int epi, const uint16_t *A, const uint16_t *B, uint16_t *C, const u
   if (tile < 0 && gemm_vec_ok(g)) {
     const GemmPlan p = gemm_plan(M, N, K, gemm_dma_fits(g), aligned16(scratch) ? std::min(scratch_bytes, kGemmScratchMax) : 0);
     if (p.stream.v) return stream_run(epi, g, p.stream, scratch, st);
-    if (p.ring.v) return ring_run(epi, g, p.ring, scratch, st);
+    if (p.ring.tile >= 0) return ring_run(epi, g, p.ring, scratch, st);
   }
   if (tile < 0) tile = gemm_dma_fits(g) ? 0 : pick_tile(M, N, false);
   switch (epi) {

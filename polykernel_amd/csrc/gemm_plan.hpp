@@ -1,0 +1,62 @@
+// gemm_plan.hpp -- tile and K-split choice of the ring kernel (gemm_ring.hpp)
+// for the bf16 and the int8 GEMM.  Host only.
+#pragma once
+
+#include <algorithm>
+#include <cmath>
+#include <cstddef>
+#include <cstdint>
+
+namespace pk {
+
+// A tile of 32 fm x 64 wn outputs; `us` is the time of one 64-deep k-tile with
+// a tile on every CU.
+struct RingTile {
+  int fm, wn;
+  double us;
+};
+
+// Coefficients of the time model (us, bytes per us): launch and first loads,
+// each round of 256 workgroups, the slowdown of k-tiles in launches of three
+// rounds or more (the clock falls), the memory rate of a full grid, and the
+// launch and rate of the split reduction.
+struct RingModel {
+  double launch, round, slow, mem, reduce, reduce_rate;
+};
+
+struct RingChoice {
+  int tile = -1;  // index, or -1: the kernel does not take the shape
+  int splits = 1, split_tiles = 0, units = 0;
+  double us = 0;
+};
+
+// Splits use at most `scratch` bytes of fp32 partials.
+inline RingChoice ring_choose(const RingTile *tiles, int ntiles, const RingModel &c, int M, int N, int K,
+                              int weight_bytes, size_t scratch) {
+  RingChoice best;
+  if (N % (16 / weight_bytes) != 0 || K % 8 != 0 || (size_t)K * N * weight_bytes >= (size_t(1) << 31) ||
+      (size_t)160 * K * 2 >= (size_t(1) << 31))
+    return best;
+  const int ktiles = (K + 63) / 64;
+  const double bytes = (double)N * K * weight_bytes + 2.0 * ((double)M * K + (double)M * N);
+  for (int i = 0; i < ntiles; ++i) {
+    const RingTile &v = tiles[i];
+    const int64_t grid = (((int64_t)M + 32 * v.fm - 1) / (32 * v.fm)) * (((int64_t)N + 64 * v.wn - 1) / (64 * v.wn));
+    for (int s : {1, 2, 3, 4, 6, 8}) {
+      const int steps = (ktiles + s - 1) / s;
+      if (s > 1 && steps < 4) break;
+      const int splits = (ktiles + steps - 1) / steps;
+      const size_t part = splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
+      const int64_t units = grid * splits;
+      if (part > scratch || units > INT32_MAX / 2 || (splits > 1 && units > 1024)) break;
+      const double rounds = std::ceil(units / 256.0);
+      const double k_us = steps * v.us * (1.0 + c.slow * std::min(1.0, (rounds - 1) / 2));
+      double us = c.launch + rounds * c.round + std::max(rounds * k_us, bytes / (c.mem * std::min(1.0, units / 256.0)));
+      if (splits > 1) us += c.reduce + 2.0 * part / c.reduce_rate;
+      if (best.tile < 0 || us < best.us * (1 - 1e-9)) best = RingChoice{i, splits, steps, (int)units, us};
+    }
+  }
+  return best;
+}
+
+}  // namespace pk

@@ -29,12 +29,13 @@
 // first loads and epilogue.
 //
 // Like the streaming kernel it can split K over workgroups (fp32 partials,
-// gemm_reduce_body).  Needs K % 8 == 0, N % 8 == 0, 16-byte aligned A and B;
+// gemm_reduce_body, or int8_stream.hpp's reduction).  Needs K % 8 == 0, N % 8 == 0, 16-byte aligned A and B;
 // rows, columns and k past the end are clamped onto valid memory, and the k
 // past K zeroed in registers.
 #pragma once
 
 #include "gemm_stream.hpp"
+#include "int8_stream.hpp"
 
 namespace pk {
 namespace gk {
@@ -46,6 +47,8 @@ struct GemmRingArgs {
   float *partial;   // [splits][M][N] fp32, splits > 1
   int splits;
   int split_tiles;  // k-tiles per split
+  const int8_t *W8;    // INT8: weights [K][N] and their per-column scale [N]
+  const float *scale;  // (g.B and g.bias are then unused)
 };
 
 // Workgroup -> (split, tile row, tile column): each XCD (workgroup b runs on
@@ -63,14 +66,26 @@ __device__ __forceinline__ void ring_unit(int bid, int total, int tm, int tn, in
   nt = in / rows;
 }
 
-template <int FM, int WN, int STAGES, int EPI>
+// 32-byte-unit XOR of int8 weight row k: the 8 rows of 32 columns that one
+// 32-lane pass of ds_read_b64_tr_b8 reads then cover all 64 banks once.
+template <int BN>
+__device__ __forceinline__ int swz_w8(int k) {
+  return BN == 128 ? (k >> 1) & 3 : k & 7;
+}
+
+// INT8: the weights are int8, widened exactly to bf16 in registers; EPI is then
+// an Int8Epi, applied to the sums times the column's scale.
+template <int FM, int WN, int STAGES, int EPI, bool INT8 = false>
 __device__ __forceinline__ void gemm_ring_body(const GemmRingArgs &a) {
   constexpr int KG = GR_WAVES / WN;          // k groups
   constexpr int SUB = 4 / KG;                // 16-k substeps of a k-tile per wave
   static_assert(KG * WN == GR_WAVES && SUB * KG == 4, "waves split N and K");
   constexpr int BM = 32 * FM, BN = 64 * WN;
-  constexpr int A_BYTES = BM * GR_BK * 2, STAGE = A_BYTES + GR_BK * BN * 2;
-  constexpr int NA = BM / 8, NB = BN / 8;    // 1 KiB loads per k-tile
+  constexpr int WB1 = INT8 ? 1 : 2;          // bytes of a weight
+  constexpr int BCH = BN * WB1 / 16;         // 16-byte chunks of a weight row
+  constexpr int A_BYTES = BM * GR_BK * 2, STAGE = A_BYTES + GR_BK * BN * WB1;
+  constexpr int NA = BM / 8, NB = BCH;       // 1 KiB loads per k-tile
+  constexpr bool GELU = INT8 ? EPI == I8_GELU : EPI == EPI_BIAS_GELU;
   constexpr int HI = (NA + NB + 7) / 8, LO = (NA + NB) / 8;  // per wave: the first waves may have one more
   constexpr int HEAVY = (NA + NB) % 8;       // waves with HI loads (0: all have LO)
   constexpr int NM = 2 * FM, NU = FM + 2;    // MFMAs and fragment-read units per substep
@@ -94,8 +109,13 @@ __device__ __forceinline__ void gemm_ring_body(const GemmRingArgs &a) {
   // to wave i % 8 as its load i / 8, with a loop-invariant lane offset and the
   // k-tile in the scalar offset
   const pk_u32x4 a_rsrc = rsrc_words(g.A + (size_t)m0 * g.K, (uint32_t)((size_t)min(g.M - m0, BM) * g.K * 2));
-  const pk_u32x4 b_rsrc = rsrc_words(g.B + n0, (uint32_t)(((size_t)g.K * g.N - n0) * 2));
-  constexpr int BROWS = 512 / BN;  // rows of B per load
+  const void *w_base = INT8 ? static_cast<const void *>(a.W8 + n0) : static_cast<const void *>(g.B + n0);
+  const pk_u32x4 b_rsrc = rsrc_words(w_base, (uint32_t)(((size_t)g.K * g.N - n0) * WB1));
+  constexpr int BROWS = 64 / BCH;  // rows of B per load
+  const auto w_col = [](int r, int p) {  // column of physical chunk p of row r
+    if constexpr (INT8) return 32 * ((p >> 1) ^ swz_w8<BN>(r)) + 16 * (p & 1);
+    else return 8 * (p ^ swz_b<BN>(r));
+  };
   uint32_t off[HI];
 #pragma unroll
   for (int j = 0; j < HI; ++j) {
@@ -104,8 +124,8 @@ __device__ __forceinline__ void gemm_ring_body(const GemmRingArgs &a) {
       const int r = 8 * i + (lane >> 3);
       off[j] = (uint32_t)(min(r, g.M - 1 - m0) * g.K + 8 * ((lane & 7) ^ swz_a64(r))) * 2u;
     } else {
-      const int r = (i - NA) * BROWS + lane / (BN / 8);
-      off[j] = (uint32_t)(r * g.N + min(8 * ((lane % (BN / 8)) ^ swz_b<BN>(r)), g.N - 8 - n0)) * 2u;
+      const int r = (i - NA) * BROWS + lane / BCH;
+      off[j] = (uint32_t)(r * g.N + min(w_col(r, lane % BCH), g.N - 16 / WB1 - n0)) * WB1;
     }
   }
   auto issue_one = [&](int slot, int t, int j) __attribute__((always_inline)) {
@@ -120,8 +140,8 @@ __device__ __forceinline__ void gemm_ring_body(const GemmRingArgs &a) {
       dma_lds16(a_rsrc, dst, o, (uint32_t)kt * (GR_BK * 2));
     } else {
       uint32_t o = off[j];
-      if (tail) o -= 2u * (uint32_t)g.N * max(0, (i - NA) * BROWS + lane / (BN / 8) - (k_tail - 1));
-      dma_lds16(b_rsrc, dst, o, (uint32_t)kt * (GR_BK * 2) * (uint32_t)g.N);
+      if (tail) o -= WB1 * (uint32_t)g.N * max(0, (i - NA) * BROWS + lane / BCH - (k_tail - 1));
+      dma_lds16(b_rsrc, dst, o, (uint32_t)kt * (GR_BK * WB1) * (uint32_t)g.N);
     }
   };
   auto issue = [&](int slot, int t) __attribute__((always_inline)) {
@@ -144,18 +164,28 @@ __device__ __forceinline__ void gemm_ring_body(const GemmRingArgs &a) {
     a_rd[u] = row * 128 + 16 * ((2 * s + hi) ^ swz_a64(row));
 #pragma unroll
     for (int fn = 0; fn < 2; ++fn) {
-      const int k = 16 * s + 8 * hi + (gi >> 2);
-      const int col = wn * 64 + fn * 32 + 16 * (grp & 1) + 4 * (gi & 3);
-      b_rd[u][fn] = A_BYTES + k * (2 * BN) + 16 * ((col >> 3) ^ swz_b<BN>(k)) + 2 * (col & 7);
+      if constexpr (INT8) {
+        const int k = 16 * s + 8 * hi + (gi >> 1);
+        b_rd[u][fn] = A_BYTES + k * BN + 32 * ((wn * 2 + fn) ^ swz_w8<BN>(k)) + 16 * (grp & 1) + 8 * (gi & 1);
+      } else {
+        const int k = 16 * s + 8 * hi + (gi >> 2);
+        const int col = wn * 64 + fn * 32 + 16 * (grp & 1) + 4 * (gi & 3);
+        b_rd[u][fn] = A_BYTES + k * (2 * BN) + 16 * ((col >> 3) ^ swz_b<BN>(k)) + 2 * (col & 7);
+      }
     }
   }
   struct Frag {
     bf16x8 a[FM], b[2];
+    i8s::v2i32 w[2];  // INT8: the weights as read, widened to b by the substep that uses them
   };
   auto read_unit = [&](Frag &f, int slot, int u, int i) __attribute__((always_inline)) {
     const uint8_t *base = ring + slot * STAGE;
     if (i < 2) {
       const uint8_t *p = base + b_rd[u][i];
+      if constexpr (INT8) {
+        f.w[i] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((i8s::lds_v2i32 *)p);
+        return;
+      }
       const i16x4 h0 = lds_read_tr(reinterpret_cast<const uint16_t *>(p));
       const i16x4 h1 = lds_read_tr(reinterpret_cast<const uint16_t *>(p + 4 * (2 * BN)));
       f.b[i] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -171,9 +201,15 @@ __device__ __forceinline__ void gemm_ring_body(const GemmRingArgs &a) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
   // W as the first operand: lane l holds 4 consecutive columns of output row
-  // 32 fm + l % 32
-  auto mfma_one = [&](const Frag &f, int i) __attribute__((always_inline)) {
-    acc[i >> 1][i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.b[i & 1], f.a[i >> 1], acc[i >> 1][i & 1], 0, 0, 0);
+  // 32 fm + l % 32.  INT8 takes a column block's MFMAs together, so that the
+  // second block is widened between those of the first.
+  auto mfma_one = [&](Frag &f, int i) __attribute__((always_inline)) {
+    const int fm = INT8 ? i % FM : i >> 1, fn = INT8 ? i / FM : i & 1;
+    if constexpr (INT8) {
+      if (i == 0) f.b[0] = i8s::widen8(f.w[0]);
+      if (i == 1) f.b[1] = i8s::widen8(f.w[1]);
+    }
+    acc[fm][fn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.b[fn], f.a[fm], acc[fm][fn], 0, 0, 0);
   };
   // the lane's 8 k of a substep lie past K on the last k-tile: zero both operands
   auto mask_tail = [&](Frag &f, int u, int t) __attribute__((always_inline)) {
@@ -181,15 +217,14 @@ __device__ __forceinline__ void gemm_ring_body(const GemmRingArgs &a) {
       const bf16x8 z = __builtin_bit_cast(bf16x8, u32x4{0, 0, 0, 0});
 #pragma unroll
       for (int i = 0; i < FM; ++i) f.a[i] = z;
-      f.b[0] = z;
-      f.b[1] = z;
+      if constexpr (!INT8) f.b[0] = f.b[1] = z;  // (an int8 weight is finite)
     }
   };
 
   // the GELU table, loaded ahead of the first DMA and copied to LDS at the end
   constexpr int TAB_W = (GELU_TABLE_SIZE + 1) / 2, TAB_PT = (TAB_W + GR_THREADS - 1) / GR_THREADS;
-  uint32_t tab_pre[EPI == EPI_BIAS_GELU ? TAB_PT : 1];
-  if constexpr (EPI == EPI_BIAS_GELU) {
+  uint32_t tab_pre[GELU ? TAB_PT : 1];
+  if constexpr (GELU) {
 #pragma unroll
     for (int j = 0; j < TAB_PT; ++j) {
       const int i = tid + j * GR_THREADS;
@@ -216,7 +251,7 @@ __device__ __forceinline__ void gemm_ring_body(const GemmRingArgs &a) {
   for (int i = 0; i < NU; ++i) read_unit(f0, 0, 0, i);
   // MFMAs of one substep with the reads of the next one spread over them, and
   // loads [j0, j1) of k-tile lt behind every second MFMA
-  auto substep = [&](const Frag &f, Frag &nx, int nslot, int nu, int lslot, int lt, int j0, int j1)
+  auto substep = [&](Frag &f, Frag &nx, int nslot, int nu, int lslot, int lt, int j0, int j1)
       __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < NM; ++i) {
@@ -277,7 +312,7 @@ __device__ __forceinline__ void gemm_ring_body(const GemmRingArgs &a) {
   constexpr int LD = 68, WB = 32 * LD * 4;
   static_assert(GR_WAVES * WB + GELU_TABLE_SIZE * 2 + 16 <= STAGES * STAGE, "staging fits the ring");
   uint16_t *tab = reinterpret_cast<uint16_t *>(ring + GR_WAVES * WB);
-  if constexpr (EPI == EPI_BIAS_GELU) {
+  if constexpr (GELU) {
 #pragma unroll
     for (int j = 0; j < TAB_PT; ++j)
       if (tid + j * GR_THREADS < TAB_W) reinterpret_cast<uint32_t *>(tab)[tid + j * GR_THREADS] = tab_pre[j];
@@ -311,6 +346,8 @@ __device__ __forceinline__ void gemm_ring_body(const GemmRingArgs &a) {
         float *o = a.partial + ((size_t)split * g.M + m) * g.N + n;
         *reinterpret_cast<f32x4 *>(o) = v0;
         *reinterpret_cast<f32x4 *>(o + 4) = v1;
+      } else if constexpr (INT8) {
+        i8s::int8_epilogue8<EPI>(v0, v1, m, n, g.N, a.scale, g.R, tab, g.C);
       } else {
         gemm_finish8<EPI>(v0, v1, m, n, g, tab);
       }

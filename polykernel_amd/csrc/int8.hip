@@ -23,6 +23,8 @@
 // golden's per-stage bf16 rounding.
 #include <mutex>
 
+#include "gemm_plan.hpp"
+#include "gemm_ring.hpp"
 #include "int8_stream.hpp"
 
 namespace pk {
@@ -224,6 +226,41 @@ __global__ __launch_bounds__(WAVES * 64, 1) void int8_stream_kernel(I8sArgs g) {
   stream_body<NT, MT, WAVES, STAGES, EPI>(g);
 }
 
+// ---- prompt-sized calls (gemm_ring.hpp, weights widened in registers) ---------
+template <int FM, int WN, int STAGES, int EPI>
+__global__ __launch_bounds__(gk::GR_THREADS, 1) void int8_ring_kernel(gk::GemmRingArgs a) {
+  gk::gemm_ring_body<FM, WN, STAGES, EPI, true>(a);
+}
+using RingLaunch = void (*)(dim3, hipStream_t, const gk::GemmRingArgs &);
+template <int FM, int WN, int STAGES, int EPI>
+void ring_launch(dim3 grid, hipStream_t st, const gk::GemmRingArgs &a) {
+  int8_ring_kernel<FM, WN, STAGES, EPI><<<grid, gk::GR_THREADS, 0, st>>>(a);
+}
+#define I8R_V(FM, WN, S) \
+  { ring_launch<FM, WN, S, I8_NONE>, ring_launch<FM, WN, S, I8_GELU>, ring_launch<FM, WN, S, I8_RESID> }
+const RingTile kI8Ring[] = {{2, 2, 0.33}, {4, 2, 0.456}, {5, 2, 0.558}, {4, 4, 0.728}, {5, 4, 0.9}};
+const RingLaunch kI8RingFn[][3] = {I8R_V(2, 2, 6), I8R_V(4, 2, 5), I8R_V(5, 2, 5), I8R_V(4, 4, 4), I8R_V(5, 4, 4)};
+#undef I8R_V
+
+// Above 32 rows the streaming kernel's workgroups re-read the weights for each
+// block of rows ([300, 12288, 4096] 87 us with five blocks of 64, 43.8 here) or
+// widen a weight for few MFMAs (M 64: [64, 12288, 4096] 29.0 and 22.0 us, M 33:
+// [33, 12288, 4096] 25.9 and 21); at M 32 it still wins or ties.  The model is
+// fitted to 32 shapes of 33-1000 rows: within 0.6 % of the best variant.  The
+// scratch is capped at the static buffer of launch_matmul_int8_noalloc, so
+// that entry points with and without a workspace of their own split alike.
+constexpr int kI8RingRows = 32;
+constexpr RingModel kI8RingModel{5.4, 1.1, 0.12, 6.4e6, 2.0, 4.4e6};
+constexpr size_t kInt8ScratchBytes = size_t(16) << 20;
+RingChoice i8_ring_plan(int M, int N, int K, size_t scratch) {
+  if (M <= kI8RingRows) return RingChoice{};
+  return ring_choose(kI8Ring, (int)(sizeof kI8Ring / sizeof kI8Ring[0]), kI8RingModel, M, N, K, 1,
+                     std::min(scratch, kInt8ScratchBytes));
+}
+size_t i8_ring_part(const RingChoice &p, int M, int N) {
+  return p.splits > 1 ? (size_t)p.splits * M * N * sizeof(float) : 0;
+}
+
 // Number of K splits: enough workgroups to cover the chip ~4x, each wave
 // keeping at least 8 steps.
 int choose_splits(int M, int N, int K) {
@@ -233,6 +270,19 @@ int choose_splits(int M, int N, int K) {
   int s = 1;
   while (tiles * s < 1024 && kunits / (2 * s) >= 2) s *= 2;
   return s;
+}
+
+// The generic kernel's split partials in bytes; its splits go to *g if given.
+size_t generic_workspace(int M, int N, int K, Int8Args *g) {
+  const int unit = I8_STEP * I8_WAVES;
+  int splits = choose_splits(M, N, K);
+  const int kper = ((K + splits - 1) / splits + unit - 1) / unit * unit;
+  splits = (K + kper - 1) / kper;
+  if (g) {
+    g->splits = splits;
+    g->kper = kper;
+  }
+  return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
 }
 
 // ---- streaming-kernel variants and their selection -------------------------
@@ -423,6 +473,12 @@ size_t int8_workspace_bytes(int M, int N, int K) {
   return std::max(need, s > 1 ? (size_t)s * M * N * sizeof(float) : 0);
 }
 
+static int check_workspace(size_t need, size_t ws_bytes) {
+  if (ws_bytes >= need) return PK_OK;
+  set_error("int8 matmul: workspace of %zu bytes required, got %zu", need, ws_bytes);
+  return PK_ERR_WORKSPACE;
+}
+
 static int use_workspace(size_t need, void *&ws, size_t ws_bytes, hipStream_t st, WorkspaceLease &lease) {
   if (need == 0) return PK_OK;
   if (ws == nullptr) {
@@ -430,10 +486,27 @@ static int use_workspace(size_t need, void *&ws, size_t ws_bytes, hipStream_t st
     ws = lease.ptr;
     return rc;
   }
-  if (ws_bytes < need) {
-    set_error("int8 matmul: workspace of %zu bytes required, got %zu", need, ws_bytes);
-    return PK_ERR_WORKSPACE;
+  return check_workspace(need, ws_bytes);
+}
+
+// Sum of g.splits partials and the epilogue.
+static int reduce_run(int epi, const Int8Args &g, hipStream_t st) {
+  const int64_t total = (int64_t)g.M * g.N;
+  const bool vec = g.N % 8 == 0 && aligned16(g.partial) && aligned16(g.scale) && aligned16(g.C) &&
+                   (epi != I8_RESID || aligned16(g.R));
+  if (vec) {
+    constexpr int T = PK_I8_REDUCE_THREADS;
+    const int blocks = (int)std::min<int64_t>((total / 8 + T - 1) / T, 4096);
+    if (epi == I8_NONE) int8_reduce8_kernel<I8_NONE><<<blocks, T, 0, st>>>(g);
+    else if (epi == I8_GELU) int8_reduce8_kernel<I8_GELU><<<blocks, T, 0, st>>>(g);
+    else int8_reduce8_kernel<I8_RESID><<<blocks, T, 0, st>>>(g);
+  } else {
+    const int blocks = (int)std::min<int64_t>((total + 255) / 256, 4096);
+    if (epi == I8_NONE) int8_reduce_kernel<I8_NONE><<<blocks, 256, 0, st>>>(g);
+    else if (epi == I8_GELU) int8_reduce_kernel<I8_GELU><<<blocks, 256, 0, st>>>(g);
+    else int8_reduce_kernel<I8_RESID><<<blocks, 256, 0, st>>>(g);
   }
+  PK_LAUNCH_CHECK("int8_reduce_kernel");
   return PK_OK;
 }
 
@@ -446,6 +519,31 @@ int int8_run(int epi, const uint16_t *A, const int8_t *W, const float *scale, ui
     if (rc) return rc;
   }
   I8sPlan plan;
+  if (!cfg && aligned16(A) && aligned16(W) && aligned16(scale) && aligned16(C) && (epi != I8_RESID || aligned16(R))) {
+    // a caller's scratch is refused where the streaming or generic kernel's splits would not fit it
+    if (ws && i8_ring_plan(M, N, K, 0).tile >= 0) {
+      if (int rc = check_workspace(i8s_plan(M, N, K, nullptr, device_cus(), plan) ? i8s_workspace(plan, M, N)
+                                                                                  : generic_workspace(M, N, K, nullptr),
+                                   ws_bytes))
+        return rc;
+    }
+    // caller scratch as it is, library scratch as far as it can be had
+    RingChoice p = i8_ring_plan(M, N, K, ws ? (aligned16(ws) ? ws_bytes : 0) : kInt8ScratchBytes);
+    WorkspaceLease lease;
+    if (p.tile >= 0 && p.splits > 1 && !ws) {
+      int rc = library_workspace(0, i8_ring_part(p, M, N), st, lease);
+      if (rc) return rc;
+      if (lease.bytes >= i8_ring_part(p, M, N)) ws = lease.ptr;
+      else p = i8_ring_plan(M, N, K, 0);
+    }
+    if (p.tile >= 0) {
+      const gk::GemmRingArgs a{{A, nullptr, C, nullptr, R, tab, M, N, K}, static_cast<float *>(ws), p.splits,
+                               p.split_tiles, W, scale};
+      kI8RingFn[p.tile][epi](dim3(p.units), st, a);
+      PK_LAUNCH_CHECK("int8_ring_kernel");
+      return p.splits > 1 ? reduce_run(epi, Int8Args{A, W, scale, a.partial, C, R, tab, M, N, K, p.splits, 0}, st) : PK_OK;
+    }
+  }
   const bool fast = aligned16(A) && aligned16(W) && aligned16(scale) && aligned16(C) &&
                     (epi != I8_RESID || aligned16(R)) && i8s_plan(M, N, K, cfg, device_cus(), plan);
   if (cfg && !fast) {
@@ -472,11 +570,8 @@ int int8_run(int epi, const uint16_t *A, const int8_t *W, const float *scale, ui
     g.splits = plan.splits;
     g.partial = a.partial;
   } else {
-    g.splits = choose_splits(M, N, K);
-    const int unit = I8_STEP * I8_WAVES;
-    g.kper = ((K + g.splits - 1) / g.splits + unit - 1) / unit * unit;
-    g.splits = (K + g.kper - 1) / g.kper;
-    int rc = use_workspace(g.splits > 1 ? (size_t)g.splits * M * N * sizeof(float) : 0, ws, ws_bytes, st, lease);
+    const size_t need = generic_workspace(M, N, K, &g);
+    int rc = use_workspace(need, ws, ws_bytes, st, lease);
     if (rc) return rc;
     g.partial = static_cast<float *>(ws);
     const bool aligned = (N % 16 == 0) && (K % 8 == 0) && aligned16(A) && aligned16(W);
@@ -492,25 +587,7 @@ int int8_run(int epi, const uint16_t *A, const int8_t *W, const float *scale, ui
 #undef PK_I8
     PK_LAUNCH_CHECK("int8_gemm_kernel");
   }
-  if (g.splits > 1) {
-    const int64_t total = (int64_t)M * N;
-    const bool vec = N % 8 == 0 && aligned16(g.partial) && aligned16(scale) && aligned16(C) &&
-                     (epi != I8_RESID || aligned16(R));
-    if (vec) {
-      constexpr int T = PK_I8_REDUCE_THREADS;
-      const int blocks = (int)std::min<int64_t>((total / 8 + T - 1) / T, 4096);
-      if (epi == I8_NONE) int8_reduce8_kernel<I8_NONE><<<blocks, T, 0, st>>>(g);
-      else if (epi == I8_GELU) int8_reduce8_kernel<I8_GELU><<<blocks, T, 0, st>>>(g);
-      else int8_reduce8_kernel<I8_RESID><<<blocks, T, 0, st>>>(g);
-    } else {
-      const int blocks = (int)std::min<int64_t>((total + 255) / 256, 4096);
-      if (epi == I8_NONE) int8_reduce_kernel<I8_NONE><<<blocks, 256, 0, st>>>(g);
-      else if (epi == I8_GELU) int8_reduce_kernel<I8_GELU><<<blocks, 256, 0, st>>>(g);
-      else int8_reduce_kernel<I8_RESID><<<blocks, 256, 0, st>>>(g);
-    }
-    PK_LAUNCH_CHECK("int8_reduce_kernel");
-  }
-  return PK_OK;
+  return g.splits > 1 ? reduce_run(epi, g, st) : PK_OK;
 }
 
 // ---- the no-allocation variant of launch_matmul_int8 -------------------------
@@ -520,7 +597,6 @@ int int8_run(int epi, const uint16_t *A, const int8_t *W, const float *scale, ui
 // not device memory: its device address is looked up per device with
 // hipGetSymbolAddress once (int8_scratch_setup) and only that address is
 // passed to kernels.
-constexpr size_t kInt8ScratchBytes = size_t(16) << 20;
 static __device__ __align__(256) float scratch[kInt8ScratchBytes / sizeof(float)];
 
 namespace {

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from polykernel_amd import synth
-from tests.bounds import _gate_bad
+from tests.bounds import _gate_bad, _int8_exact_inputs
 from tests.helpers import bf, from_dev, int_bf16, rng_bf16, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -127,3 +127,28 @@ def test_rmsnorm_matmul_split(gpu, M, N, Kd):
         torch.cuda.synchronize()
         assert torch.equal(out.view(torch.int16), got.view(torch.int16))
         assert torch.equal(kernels.fused_rmsnorm_matmul(x, w, g, 1e-6).view(torch.int16), got.view(torch.int16))
+
+
+# the int8 ring kernel's five tiles (64 x 128 ... 160 x 256), K tails, K splits
+# (512 columns, long K), N with a ragged 16-column chunk
+@pytest.mark.parametrize("M,N,Kd", [(33, 16, 8), (65, 144, 72), (129, 272, 520), (48, 512, 4096), (300, 2064, 1032),
+                                    (391, 6688, 64), (300, 12288, 64), (879, 6464, 72), (1060, 7184, 136),
+                                    (600, 1040, 4104)])
+def test_int8_ring_integer_bit_exact(gpu, oracle, M, N, Kd):
+    from polykernel_amd import _lib, kernels
+
+    print(f"int8 ring {M}x{N}x{Kd}", flush=True)
+    a, wq, s = _int8_exact_inputs(M, N, Kd, 160)
+    r = rng_bf16((M, N), 163)
+    da, dw, ds, dr = to_dev(a), to_dev(wq), to_dev(s), to_dev(r)
+    plain = oracle.matmul_int8(a, wq, s)
+    got = kernels.matmul_int8(da, dw, ds)
+    assert np.array_equal(from_dev(got), plain)
+    assert np.array_equal(from_dev(kernels.matmul_int8_ex(1, da, dw, ds)), oracle.gelu(plain))
+    assert np.array_equal(from_dev(kernels.matmul_int8_ex(2, da, dw, ds, dr)), oracle.add(plain, r))
+    import torch
+
+    out = torch.empty_like(got)
+    rc = _lib.load().launch_matmul_int8_noalloc(da.data_ptr(), dw.data_ptr(), ds.data_ptr(), out.data_ptr(), M, N, Kd,
+                                                torch.cuda.current_stream().cuda_stream)
+    assert rc == _lib.PK_ERR_WORKSPACE or (rc == 0 and torch.equal(out.view(torch.int16), got.view(torch.int16)))
