@@ -52,6 +52,11 @@ __global__ __launch_bounds__(NW > 4 ? NW * 64 : kBlock) void softmax_vec_kernel(
   softmax_vec_body<NW, VPT, MODE>(a);
 }
 
+template <int NW, int VPT, int MODE>
+__global__ __launch_bounds__(NW > 4 ? NW * 64 : kBlock) void softmax_ragged_kernel(RowArgs a) {
+  softmax_ragged_body<NW, VPT, MODE>(a);
+}
+
 template <int MODE>
 __global__ __launch_bounds__(kBlock) void softmax_generic_kernel(RowArgs a) {
   softmax_generic_body<MODE>(a);
@@ -87,7 +92,9 @@ __global__ __launch_bounds__(kPackedLanes) void softmax_packed_kernel(RowArgs a)
 //   65536 columns 491 -> 176 and 622 -> 238 us, [rows, cols] of 2^27 elements);
 //   8193 to 16384 vectors (up to 131072 columns): 16 waves, 16 vectors per
 //   lane as packed bf16 (num_warps 16, unroll 16);
-//   cols % 8 != 0 or longer rows: the generic kernel.
+//   cols % 8 != 0 or longer rows: the generic kernel (where the entry points
+//   have no config and aligned operands, softmax rows of such lengths up to
+//   32754 columns take softmax_ragged_kernel instead).
 int row_vpt(int nvec, int lanes) {
   for (int v : {1, 2, 4, 8, 16})
     if (lanes * v >= nvec) return v;
@@ -216,6 +223,28 @@ int softmax_run(const RowArgs &a, const pk_config &c, hipStream_t st) {
   return PK_ERR_UNSUPPORTED;
 }
 
+// The ragged kernel for rows of up to 32754 columns, the waves per row by length
+// as for the vector kernels (a row may touch one chunk more than its length
+// needs; a third vector per lane between 1010 and 1522 columns, since lengths
+// just over 1024 would idle half of four).  [16336, 1021] masked 63.2 -> 26.9 us
+// (5.0 TB/s).  False: longer rows stay with the generic kernel (8 vectors per
+// lane of 16 waves would spill).
+template <int MODE>
+bool softmax_ragged_run(const RowArgs &a, hipStream_t st) {
+  const unsigned rows = (unsigned)a.rows, grid4 = rows / 4 + (rows % 4 != 0);
+  const int64_t nvec = ((int64_t)a.cols + 14) / 8;
+  if (nvec <= 64) softmax_ragged_kernel<1, 1, MODE><<<grid4, kBlock, 0, st>>>(a);
+  else if (nvec <= 128) softmax_ragged_kernel<1, 2, MODE><<<grid4, kBlock, 0, st>>>(a);
+  else if (nvec <= 192) softmax_ragged_kernel<1, 3, MODE><<<grid4, kBlock, 0, st>>>(a);
+  else if (nvec <= 256) softmax_ragged_kernel<1, 4, MODE><<<grid4, kBlock, 0, st>>>(a);
+  else if (nvec <= 512) softmax_ragged_kernel<4, 2, MODE><<<rows, 256, 0, st>>>(a);
+  else if (nvec <= 1024) softmax_ragged_kernel<8, 2, MODE><<<rows, 512, 0, st>>>(a);
+  else if (nvec <= 2048) softmax_ragged_kernel<8, 4, MODE><<<rows, 512, 0, st>>>(a);
+  else if (nvec <= 4096) softmax_ragged_kernel<16, 4, MODE><<<rows, 1024, 0, st>>>(a);
+  else return false;
+  return true;
+}
+
 // cfg null: the built-in choice (the first candidate, or the generic kernel
 // when the operands are not 16-byte aligned); otherwise a listed config, which
 // must be the generic one when they are not.
@@ -270,6 +299,10 @@ int softmax_dispatch(const void *in, const uint16_t *mask, uint16_t *y, int rows
   } else {
     row_configs(true, rows, cols, &c, 1);
     if (!aligned) c = pk_config{1, cols, 0, 4, 1, 1, 1};
+    if (aligned && cols % 8 != 0 && softmax_ragged_run<MODE>(a, st)) {
+      PK_LAUNCH_CHECK(name);
+      return PK_OK;
+    }
   }
   int rc = softmax_run<MODE>(a, c, st);
   if (rc) return rc;

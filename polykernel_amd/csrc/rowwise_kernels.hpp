@@ -328,6 +328,95 @@ __device__ __forceinline__ void softmax_vec_body(const RowArgs &a) {
   }
 }
 
+// Rows whose length is not a multiple of 8 (16-byte aligned tensors): the row
+// is read in the 8-element chunks of the whole tensor that cover it, which are
+// aligned whatever row * cols is; the elements of its first and last chunk that
+// belong to the neighbouring rows count as -inf and are not written.  The
+// tensor's last chunk may be short and is then read by elements.  HBM-bound
+// like softmax_vec_body: the generic kernel's three passes of 2- and 4-byte
+// accesses took 63 us for [16336, 1021] fp32 + mask (133 MB).
+template <int NW, int VPT, int MODE>
+__device__ __forceinline__ void softmax_ragged_body(const RowArgs &a) {
+#pragma clang fp contract(off)
+  const void *__restrict__ in = a.in;
+  const uint16_t *__restrict__ mask = a.aux;
+  uint16_t *__restrict__ y = a.out;
+  const int rows = a.rows, cols = a.cols;
+  __shared__ float red[NW];
+  constexpr int kLanes = NW * 64;
+  const unsigned row = NW == 1 ? blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6) : blockIdx.x;
+  const int lane = NW == 1 ? (threadIdx.x & 63) : threadIdx.x;
+  if (row >= (unsigned)rows) return;
+  const size_t total = (size_t)rows * cols, base = (size_t)row * cols;
+  const size_t first = base & ~size_t(7);       // of the row's first chunk
+  const int lead = (int)(base - first);         // elements of the previous row in it
+  const int nvec = (lead + cols + 7) >> 3;
+  const int tail = lead + cols - 8 * (nvec - 1);  // elements up to the row's end in its last chunk
+
+  Z8Words<MODE> zw[VPT];
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int c = lane + i * kLanes;
+    const size_t off = first + (size_t)c * 8;
+    if (c < nvec && off + 8 <= total) zw[i] = load_z8_words<MODE>(in, mask, off);
+  }
+  float z[VPT][8];
+  float m = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int c = lane + i * kLanes;
+    const size_t off = first + (size_t)c * 8;
+    if (c < nvec) {
+      if (off + 8 <= total) {
+        z8_of<MODE>(zw[i], z[i]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) z[i][e] = off + e < total ? load_z1<MODE>(in, mask, off + e) : -INFINITY;
+      }
+      if (c == 0 || c == nvec - 1) {
+        const int lo = c == 0 ? lead : 0, hi = c == nvec - 1 ? tail : 8;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (e < lo || e >= hi) z[i][e] = -INFINITY;
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) m = fmaxf(m, z[i][e]);
+    }
+  }
+  m = group_max<NW>(m, red);
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    if (lane + i * kLanes < nvec) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        z[i][e] = expf(z[i][e] - m);  // 0 for the neighbours' elements (NaN with m, and then the sum is NaN anyway)
+        s += z[i][e];
+      }
+    }
+  }
+  s = group_sum<NW>(s, red);
+  const float inv = 1.0f / s;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int c = lane + i * kLanes;
+    if (c < nvec) {
+      float o[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = z[i][e] * inv;
+      uint16_t *out = y + first + (size_t)c * 8;
+      const int lo = c == 0 ? lead : 0, hi = c == nvec - 1 ? tail : 8;
+      if (lo == 0 && hi == 8) {
+        st16(out, pack8(o));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (e >= lo && e < hi) out[e] = (uint16_t)f2bf(o[e]);
+      }
+    }
+  }
+}
+
 template <int MODE>
 __device__ __forceinline__ void softmax_generic_body(const RowArgs &a) {
 #pragma clang fp contract(off)
