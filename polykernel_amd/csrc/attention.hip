@@ -24,9 +24,11 @@
 // queries of one (b,h); K/V tiles are double-buffered in LDS.  When queries
 // alone do not fill the chip the key range is split (flash-decoding style)
 // and att_combine_kernel merges the fp32 partials in split order.  Head dims
-// 64 and 128 with enough query tiles take attention_fa_kernel (below).
+// 64 and 128 take attention_fa_kernel (below), and up to 4 queries of them
+// attention_decode_kernel.
 #include <cstring>
 
+#include "attention_decode.hpp"
 #include "attention_kernels.hpp"
 #include "attention_module.hpp"
 
@@ -60,6 +62,11 @@ __global__ __launch_bounds__(FA_THREADS, 1) void attention_fa_kernel(FaArgs g) {
 template <int DP>
 __global__ __launch_bounds__(256) void fa_combine_kernel(FaArgs g) {
   fa_combine_body<DP>(g);
+}
+
+template <int D, int NQ>
+__global__ __launch_bounds__(AD_THREADS) void attention_decode_kernel(FaArgs g) {
+  att_decode_body<D, NQ>(g);
 }
 
 __global__ __launch_bounds__(256) void kv_append_kernel(pk_kv_append_args a) { kv_append_body(a); }
@@ -284,6 +291,54 @@ int attention_fa(FaArgs a, int D, int qg, hipStream_t st, const AttModule *mod) 
   return PK_OK;
 }
 
+// 1 to 4 queries per head: the streaming kernel, for operands the flash kernel
+// takes (any S_cache, since rows are read one by one) when every query sees a
+// key.  Key splits while the (b, h) alone leave CUs idle, each keeping a batch
+// per wave.
+bool decode_applicable(int S_q, int S_kv, bool causal) {
+  return S_q > 0 && S_q <= AD_MAX_Q && S_kv > 0 && (!causal || S_kv >= S_q);
+}
+int attention_decode(FaArgs a, int D, hipStream_t st) {
+  a.q_tiles = 1;
+  const int batch = AD_U * 512 / D;  // keys of a wave's batch
+  a.splits = 1;
+  while (a.BH * a.splits < 256 && a.S_kv / (a.splits * 2) >= AD_WAVES * batch && a.splits < 64) a.splits *= 2;
+  const size_t rows = (size_t)a.BH * a.S_q;
+  const size_t bytes_o = (size_t)a.splits * rows * D * sizeof(float);
+  WorkspaceLease lease;  // held until the merge kernel is queued
+  if (a.splits > 1) {
+    const size_t bytes = bytes_o + (size_t)a.splits * rows * 2 * sizeof(float);
+    int rc = library_workspace(0, bytes, st, lease);
+    if (rc) return rc;
+    if (lease.bytes >= bytes) {
+      a.part_o = static_cast<float *>(lease.ptr);
+      a.part_ml = reinterpret_cast<float *>(static_cast<char *>(lease.ptr) + bytes_o);
+    } else {
+      a.splits = 1;
+    }
+  }
+  if (int rc = grid_ok(a.BH, 1, a.splits, "attention")) return rc;
+  const int blocks = a.BH * a.splits;
+#define PK_AD_LAUNCH(DV)                                                                     \
+  do {                                                                                       \
+    if (a.S_q == 1) attention_decode_kernel<DV, 1><<<blocks, AD_THREADS, 0, st>>>(a);        \
+    else if (a.S_q == 2) attention_decode_kernel<DV, 2><<<blocks, AD_THREADS, 0, st>>>(a);   \
+    else attention_decode_kernel<DV, 4><<<blocks, AD_THREADS, 0, st>>>(a);                   \
+  } while (0)
+  if (D == 128) PK_AD_LAUNCH(128);
+  else PK_AD_LAUNCH(64);
+#undef PK_AD_LAUNCH
+  PK_LAUNCH_CHECK("attention_decode_kernel");
+  if (a.splits > 1) {
+    const int64_t items = (int64_t)rows * (D / 8);
+    const int grid = (int)std::min<int64_t>((items + 255) / 256, 8192);
+    if (D == 128) fa_combine_kernel<128><<<grid, 256, 0, st>>>(a);
+    else fa_combine_kernel<64><<<grid, 256, 0, st>>>(a);
+    PK_LAUNCH_CHECK("fa_combine_kernel");
+  }
+  return PK_OK;
+}
+
 // Configs of attention as descriptors: the flash kernel's two tile shapes
 // for D 64 / 128 ({queries, keys per step, D, 8 waves, 16-byte vectors,
 // D/16 MFMA k-steps per product, K/V ring slots}), the generic kernel
@@ -342,6 +397,12 @@ int fa_qg_of(const pk_config &c, int D) {
 int attention_run(const uint16_t *Q, const uint16_t *K, const uint16_t *V, uint16_t *O, int BH,
                   int S_q, int S_kv, int D, int kv_rows, float scale, int causal, int mode, hipStream_t st,
                   const AttModule *mod = nullptr) {
+  if (mode == 0 && scale > 0.f && decode_applicable(S_q, S_kv, causal != 0) &&
+      fa_applicable(S_kv, S_kv, D, kv_rows, Q, K, V, O, nullptr, nullptr, nullptr, nullptr, 1)) {
+    return attention_decode(FaArgs{Q, K, V, nullptr, nullptr, nullptr, nullptr, O, nullptr, nullptr, BH, S_q, S_kv,
+                                   S_kv, kv_rows, scale, causal, 1, 1},
+                            D, st);
+  }
   if (mode >= 0) {
     const int qg = mode ? mode : fa_default_qg(BH, S_q, causal != 0);
     if (scale > 0.f && fa_applicable(S_kv, S_kv, D, kv_rows, Q, K, V, O, nullptr, nullptr, nullptr, nullptr,
@@ -396,6 +457,12 @@ int fused_kv_append_attention(const uint16_t *Q, uint16_t *Kc, uint16_t *Vc, con
     auto fits = [&](int g) {
       return fa_applicable(S_kv, S_cache, D, cache_capacity, Q, Kc, Vc, O, Kn, Vn, Kc, Vc, fa_bkv(g));
     };
+    if (!mode && decode_applicable(S_q, S_kv, causal != 0) &&
+        fa_applicable(S_kv, S_cache, D, cache_capacity, Q, Kc, Vc, O, Kn, Vn, Kc, Vc, 1)) {
+      return attention_decode(FaArgs{Q, Kc, Vc, Kn, Vn, Kc, Vc, O, nullptr, nullptr, (int)BH, S_q, S_kv, S_cache,
+                                     cache_capacity, scale, causal, 1, 1},
+                              D, st);
+    }
     if (!mode && qg == 2 && !fits(2)) qg = 4;  // S_cache on a 64-key but not a 128-key step
     if (fits(qg)) {
       // the append happens inside the attention kernel

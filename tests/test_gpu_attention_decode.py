@@ -1,0 +1,56 @@
+"""Attention of 1 to 4 queries per head (attention_decode_kernel): batch and
+wave edges of the key range, key splits, causal limits, the fused append."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from polykernel_amd import metrics as mt
+from polykernel_amd import synth
+from tests.bounds import _att_bound_bad
+from tests.helpers import from_dev, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(oracle, got, q, k, v, causal):
+    want = oracle.attention_prefill(q, k, v, None, causal)
+    rep = mt.report(got, want)
+    assert rep.cosine >= 0.999 and rep.pcc >= 0.99, rep
+    assert _att_bound_bad(oracle, got, want, q, k, v, causal) == 0, rep
+
+
+# keys: one, below / at / above a batch (32 keys at D 128, 64 at 64), the 8
+# waves' batches, and enough for several key splits; heads that split and not
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,Sq,Skv", [(1, 1, 1, 1), (2, 3, 1, 31), (1, 2, 1, 64), (1, 2, 2, 65), (2, 2, 3, 255),
+                                        (1, 3, 4, 257), (1, 2, 1, 4099), (1, 2, 4, 2050), (9, 29, 1, 70)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_decode_attention(gpu, oracle, B, H, Sq, Skv, D, causal):
+    from polykernel_amd import kernels
+
+    print(f"decode attention B{B} H{H} Sq{Sq} Skv{Skv} D{D} causal={causal}", flush=True)
+    q = synth.normal_bf16((B, H, Sq, D), 180)
+    k = synth.normal_bf16((B, H, Skv, D), 181)
+    v = synth.normal_bf16((B, H, Skv, D), 182)
+    got = from_dev(kernels.attention_prefill(to_dev(q), to_dev(k), to_dev(v), None, causal))
+    _check(oracle, got, q, k, v, causal)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,Sq,Sc,spare", [(1, 2, 1, 0, 0), (2, 2, 1, 127, 5), (1, 3, 3, 128, 0), (2, 2, 4, 1021, 2),
+                                             (1, 2, 2, 2047, 0)])
+def test_decode_append_attention(gpu, oracle, B, H, Sq, Sc, spare, D):
+    """The appended rows land in the caches bit for bit, nothing else moves, and
+    the new rows are seen although the cache is written by the same launch."""
+    from polykernel_amd import kernels
+
+    print(f"decode append B{B} H{H} Sq{Sq} Sc{Sc} D{D}", flush=True)
+    q, kn, vn = (synth.normal_bf16((B, H, Sq, D), 183 + i) for i in range(3))
+    kc, vc = (synth.normal_bf16((B, H, Sc + Sq + spare, D), 186 + i) for i in range(2))
+    dk, dv = to_dev(kc), to_dev(vc)
+    got = from_dev(kernels.fused_kv_append_attention(to_dev(q), to_dev(kn), to_dev(vn), dk, dv, Sc))
+    for cache, new, dev in ((kc, kn, dk), (vc, vn, dv)):
+        cache[:, :, Sc:Sc + Sq] = new
+        assert np.array_equal(from_dev(dev), cache)
+    _check(oracle, got, q, kc[:, :, :Sc + Sq], vc[:, :, :Sc + Sq], True)
