@@ -252,9 +252,9 @@ PK_API int pk_op_configs(const char *op, long long M, long long N, long long K, 
  * split over waves and workgroups): for those it is the nearest tile. */
 PK_API int pk_op_default_config(const char *op, long long M, long long N, long long K, pk_config *out);
 
-/* The streaming kernel's configuration for this shape, which
- * launch_matmul_int8 uses up to 32 rows (more take the ring kernel, which is
- * no configuration).  Returns PK_ERR_UNSUPPORTED when the streaming kernel
+/* The column-split streaming kernel's configuration for this shape, which
+ * launch_matmul_int8 uses for weights above 100 MB up to 32 rows (more rows or
+ * smaller weights take kernels that are no configuration).  Returns PK_ERR_UNSUPPORTED when the streaming kernel
  * does not take the shape. */
 PK_API int pk_int8_default_config(int M, int N, int K, pk_config *out);
 

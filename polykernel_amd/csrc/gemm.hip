@@ -163,10 +163,12 @@ int gemm_launch_variant(const GemmArgs &g, int v, bool vec, hipStream_t st) {
 
 // ---- decode-sized calls (gemm_stream.hpp) -----------------------------------
 // The streaming kernel's variants, by slice width (16 * nt columns) and rows
-// (16 * mt): WK waves and STAGES ring stages, chosen so that two workgroups
-// fit a CU's LDS where the width allows it.  `rate` is the weight bytes per ns
-// one workgroup draws, fitted to [16, N, K] for N 512-16384, K 768-16384
-// (narrow slices read short runs: 32 bytes per weight row at nt 1).
+// (16 * mt), with the fewest waves and ring stages that keep the rate: two
+// waves stream faster than four or eight, since the rows in flight then span
+// fewer DRAM pages ([16, 16384, 4096] 24.1 us with 2 waves of 3 stages, 26.7
+// with 4, 26.8 with 8; 4 waves of 6 stages 27.4).  `rate` is the weight bytes
+// per ns one workgroup draws, fitted to [16-64, N, K] for N 512-28672, K
+// 512-16384 (narrow slices read short runs: 32 bytes per weight row at nt 1).
 struct StreamVariant {
   int nt, mt;
   double rate;
@@ -184,9 +186,9 @@ void stream_launch(dim3 grid, hipStream_t st, const GemmStreamArgs &a) {
     }                                                                                                 \
   }
 const StreamVariant kStream[] = {
-    PK_GS(4, 1, 4, 3, 28.0), PK_GS(8, 1, 4, 2, 40.0), PK_GS(2, 1, 8, 3, 15.5), PK_GS(1, 1, 8, 8, 8.3),
-    PK_GS(4, 2, 4, 3, 24.0), PK_GS(8, 2, 4, 3, 36.0), PK_GS(2, 2, 8, 3, 13.0), PK_GS(1, 2, 8, 4, 7.0),
-    PK_GS(4, 4, 4, 3, 19.0), PK_GS(8, 4, 2, 4, 30.0), PK_GS(2, 4, 8, 3, 10.0), PK_GS(1, 4, 8, 4, 6.0),
+    PK_GS(4, 1, 2, 3, 30.0), PK_GS(8, 1, 2, 2, 45.0), PK_GS(2, 1, 2, 4, 16.0), PK_GS(1, 1, 4, 4, 10.0),
+    PK_GS(4, 2, 2, 3, 27.0), PK_GS(8, 2, 2, 2, 40.0), PK_GS(2, 2, 2, 4, 14.5), PK_GS(1, 2, 4, 4, 9.0),
+    PK_GS(4, 4, 2, 3, 22.0), PK_GS(8, 4, 2, 3, 33.0), PK_GS(2, 4, 4, 3, 11.0), PK_GS(1, 4, 4, 4, 7.5),
 };
 #undef PK_GS
 constexpr int kStreamRows = 64;
@@ -202,13 +204,17 @@ bool stream_shape_ok(int M, int N, int K) {
 }
 
 // Slice width and K splits by a time model (us) fitted to the same sweep: 3
-// for the launch, the larger of the HBM time of all weights (5.7 TB/s; A's own
-// loads cost 0.35 of the weights' per byte) and of the busiest CU's units, and
-// for a split 2.5 for the reduction's launch plus its partials at 5 TB/s.
-// Rows of N * 2 bytes that do not start on 128-byte lines share lines between
-// slices: the wide slice then streams at 0.9, the others at 0.72 ([8, 50256,
-// 2048]: 44.9 us with 128 columns, 60.0 with 64).  Splits use at most
-// `scratch` bytes of partials.
+// for the launch, the larger of the memory time of all weights (6.4 TB/s; A's
+// own loads cost a part of the weights' per byte) and of the busiest CU's
+// units, and for a split 2.5 for the reduction's launch plus its partials at 5
+// TB/s.  Grids between one and two and a half workgroups per CU stream slower
+// ([16, 28672, 8192] 75.8 us with 224 units, 82.5 with 448, 80.5 with 672), and
+// so do split slices of 128-byte runs.  Rows of N * 2 bytes that do not start
+// on 128-byte lines share lines between slices: the wide slice then streams at
+// 0.9, the others at 0.72 ([8, 50256, 2048]: 44 us with 128 columns, 59 with
+// 64).  Four or more splits whose starts lie a multiple of 16 MB apart meet in
+// the same memory channels, so such a split is one step longer ([16, 4096,
+// 16384] in 8: 29.0 -> 27.1 us).  Splits use at most `scratch` bytes.
 bool stream_plan(int M, int N, int K, size_t scratch, StreamPlan &best) {
   if (!stream_shape_ok(M, N, K)) return false;
   const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
@@ -217,17 +223,20 @@ bool stream_plan(int M, int N, int K, size_t scratch, StreamPlan &best) {
   for (const StreamVariant &v : kStream) {
     if (v.mt != mt) continue;
     const int nb = 16 * v.nt, slices = (N + nb - 1) / nb;
-    const double a_share = 1.0 + 0.35 * (v.mt - 1) / v.nt;
+    const double a_share = 1.0 + (v.mt == 4 ? 0.45 : 0.35) * (v.mt - 1) / v.nt;
     const double line = N % 64 == 0 ? 1.0 : v.nt == 8 ? 0.9 : 0.72;
-    const double hbm = (double)N * K * 2 * a_share / (5.7e6 * line);
-    for (int s : {1, 2, 3, 4, 6, 8, 12, 14, 16}) {
-      const int steps = (ksteps + s - 1) / s;
+    for (int s : {1, 2, 3, 4, 5, 6, 8, 10, 12, 14, 16}) {
+      int steps = (ksteps + s - 1) / s;
       if (s > 1 && steps < 8) break;
+      if (s >= 4 && (size_t)steps * GS_KSTEP * N * 2 % (size_t(16) << 20) == 0) ++steps;
       const int splits = (ksteps + steps - 1) / steps;
       const size_t part = splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
       if (part > scratch) break;
-      const double rounds = std::ceil((double)slices * splits / 256);
-      double us = 3.0 + std::max(hbm, rounds * steps * GS_KSTEP * nb * 2 / (v.rate * 1e3 * line));
+      const int64_t units = (int64_t)slices * splits;
+      const double rounds = std::ceil(units / 256.0);
+      const double grid = units <= 256 ? 1.0 : units < 640 ? 1.2 : 1.04;
+      const double hbm = (double)N * K * 2 * a_share * grid * (v.nt == 4 && splits > 1 ? 1.1 : 1.0) / 6.4e6;
+      double us = 3.0 + std::max(hbm, rounds * steps * GS_KSTEP * nb * 2 / (v.rate * 1e3)) / line;
       if (splits > 1) us += 2.5 + 2.0 * part / 5e6;
       if (!best.v || us < best_us * (1 - 1e-9)) {
         best_us = us;

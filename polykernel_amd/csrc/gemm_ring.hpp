@@ -51,12 +51,10 @@ struct GemmRingArgs {
   const float *scale;  // (g.B and g.bias are then unused)
 };
 
-// Workgroup -> (split, tile row, tile column): each XCD (workgroup b runs on
-// XCD b % 8) takes a contiguous run of units, a split's tiles in groups of 8
-// tile rows, so that an XCD's L2 holds panels its tiles share.
+// Workgroup -> (split, tile row, tile column): each XCD takes a contiguous run
+// of units, a split's tiles in groups of 8 tile rows.
 __device__ __forceinline__ void ring_unit(int bid, int total, int tm, int tn, int &split, int &mt, int &nt) {
-  const int q = total >> 3, rem = total & 7, xcd = bid & 7;
-  const int b = xcd * q + min(xcd, rem) + (bid >> 3);
+  const int b = xcd_unit(bid, total);
   split = b / (tm * tn);
   const int r = b - split * tm * tn;
   const int group = r / (8 * tn), first = group * 8;

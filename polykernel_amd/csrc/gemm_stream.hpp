@@ -25,6 +25,11 @@
 // added in LDS in wave order; one K split applies the epilogue in place,
 // several store fp32 partials that gemm_reduce_body adds in split order.
 //
+// Measured: [16, 16384, 4096] 56 -> 24.1 us and [16, 4096, 16384] 205 -> 27.1 us
+// with its reduction (134 MB of weights each, 5.6 and 5.0 TB/s), [16, 28672,
+// 8192] 75.8 us (6.2 TB/s).  Without the MFMAs and without A's loads (timing
+// only) the first takes 24.6 and 22.3 us: the rest is the weight stream.
+//
 // Needs K % 8 == 0, N % 8 == 0 and 16-byte aligned A and B; K % 32 != 0 runs a
 // last step whose missing rows are zeroed in registers.
 #pragma once
@@ -121,10 +126,8 @@ __device__ __forceinline__ void gemm_stream_body(const GemmStreamArgs &a) {
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wk = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // workgroups of one XCD (b % 8) take consecutive units
-  const int units = a.slices * a.splits;
-  int u = blockIdx.x;
-  if (units % 8 == 0) u = (u & 7) * (units >> 3) + (u >> 3);
+  // consecutive slices share the lines of narrow runs
+  const int u = xcd_unit(blockIdx.x, a.slices * a.splits);
   const int slice = u / a.splits, split = u % a.splits;
   const int n0 = slice * WN;
   const int m0 = blockIdx.y * 16 * MT;

@@ -226,6 +226,80 @@ __global__ __launch_bounds__(WAVES * 64, 1) void int8_stream_kernel(I8sArgs g) {
   stream_body<NT, MT, WAVES, STAGES, EPI>(g);
 }
 
+// Four or more K splits whose starts lie a multiple of 16 MB apart meet in the
+// same memory channels; such a split is made one step longer ([16, 8192, 28672]
+// in 14: 45.0 us at 32 steps of 64 rows, 43.2 at 33).
+bool aliased_split(int splits, int steps, int N) {
+  return splits >= 4 && (size_t)steps * I8S_KSTEP * N % (size_t(16) << 20) == 0;
+}
+
+// ---- decode calls on smaller weights (kstream_body) ----------------------------
+template <int NT, int MT, int WK, int STAGES, int EPI>
+__global__ __launch_bounds__(WK * 64) void int8_kstream_kernel(I8sArgs a) {
+  kstream_body<NT, MT, WK, STAGES, EPI>(a);
+}
+// By slice width (16 * nt columns) and rows (16 * mt); `rate`: weight bytes per
+// ns of one workgroup, fitted to [1-32, N, K] for N 1040-16384, K 520-28672.
+struct KsVariant {
+  int nt, mt;
+  double rate;
+  void (*fn[3])(dim3, hipStream_t, const I8sArgs &);
+};
+template <int NT, int MT, int WK, int STAGES, int EPI>
+void kstream_launch(dim3 grid, hipStream_t st, const I8sArgs &a) {
+  int8_kstream_kernel<NT, MT, WK, STAGES, EPI><<<grid, WK * 64, 0, st>>>(a);
+}
+#define I8K_V(NT, MT, WK, S, RATE)                                                                    \
+  {                                                                                                   \
+    NT, MT, RATE, {                                                                                   \
+      kstream_launch<NT, MT, WK, S, I8_NONE>, kstream_launch<NT, MT, WK, S, I8_GELU>,                 \
+          kstream_launch<NT, MT, WK, S, I8_RESID>                                                     \
+    }                                                                                                 \
+  }
+const KsVariant kI8k[] = {
+    I8K_V(8, 1, 4, 2, 33.0), I8K_V(4, 1, 4, 2, 18.0), I8K_V(2, 1, 4, 3, 11.0), I8K_V(1, 1, 4, 4, 7.3),
+    I8K_V(8, 2, 4, 2, 29.0), I8K_V(4, 2, 4, 2, 17.0), I8K_V(2, 2, 4, 3, 9.5),  I8K_V(1, 2, 4, 4, 6.5),
+};
+#undef I8K_V
+struct KsPlan {
+  const KsVariant *v = nullptr;
+  int splits = 1, split_steps = 0, slices = 0;
+};
+// Up to 32 rows and weights of at most 100 MB, where the reduction of the
+// column-split stream's partials is a large part of the call ([16, 16384, 4096]
+// 20.5 -> 17.8 us, [16, 11008, 4096] 16.9 -> 14.0, [32, 4096, 14336] 23.4 ->
+// 19.5); above, its 512-byte runs win ([16, 28672, 8192] 43.5 against 46.4).
+// The time model is that of the bf16 streaming kernel with this kernel's
+// rates, and 5.8 TB/s of memory.
+bool kstream_plan(int M, int N, int K, size_t scratch, KsPlan &best) {
+  if (M > 32 || N % 16 != 0 || K % 8 != 0 || (size_t)K * N > (size_t)100000000) return false;
+  const int mt = M <= 16 ? 1 : 2;
+  const int ksteps = (K + I8S_KSTEP - 1) / I8S_KSTEP;
+  double best_us = 0;
+  for (const KsVariant &v : kI8k) {
+    if (v.mt != mt) continue;
+    const int nb = 16 * v.nt, slices = (N + nb - 1) / nb;
+    for (int s : {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16}) {
+      int steps = (ksteps + s - 1) / s;
+      if (s > 1 && steps < 6) break;
+      if (aliased_split(s, steps, N)) ++steps;
+      const int splits = (ksteps + steps - 1) / steps;
+      const size_t part = splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
+      if (part > scratch) break;
+      const int64_t units = (int64_t)slices * splits;
+      const double rounds = std::ceil(units / 256.0);
+      const double hbm = (double)N * K * (units <= 256 ? 1.0 : 1.1) * (mt == 2 ? 1.1 : 1.0) / 5.8e6;
+      double us = 3.0 + std::max(hbm, rounds * steps * I8S_KSTEP * nb / (v.rate * 1e3));
+      if (splits > 1) us += 2.5 + 2.0 * part / 5e6;
+      if (!best.v || us < best_us * (1 - 1e-9)) {
+        best_us = us;
+        best = KsPlan{&v, splits, steps, slices};
+      }
+    }
+  }
+  return best.v != nullptr;
+}
+
 // ---- prompt-sized calls (gemm_ring.hpp, weights widened in registers) ---------
 template <int FM, int WN, int STAGES, int EPI>
 __global__ __launch_bounds__(gk::GR_THREADS, 1) void int8_ring_kernel(gk::GemmRingArgs a) {
@@ -246,21 +320,14 @@ const RingLaunch kI8RingFn[][3] = {I8R_V(2, 2, 6), I8R_V(4, 2, 5), I8R_V(5, 2, 5
 // block of rows ([300, 12288, 4096] 87 us with five blocks of 64, 43.8 here) or
 // widen a weight for few MFMAs (M 64: [64, 12288, 4096] 29.0 and 22.0 us, M 33:
 // [33, 12288, 4096] 25.9 and 21); at M 32 it still wins or ties.  The model is
-// fitted to 32 shapes of 33-1000 rows: within 0.6 % of the best variant.  The
-// scratch is capped at the static buffer of launch_matmul_int8_noalloc, so
-// that entry points with and without a workspace of their own split alike.
+// fitted to 32 shapes of 33-1000 rows: within 0.6 % of the best variant.
 constexpr int kI8RingRows = 32;
 constexpr RingModel kI8RingModel{5.4, 1.1, 0.12, 6.4e6, 2.0, 4.4e6};
 constexpr size_t kInt8ScratchBytes = size_t(16) << 20;
 RingChoice i8_ring_plan(int M, int N, int K, size_t scratch) {
   if (M <= kI8RingRows) return RingChoice{};
-  return ring_choose(kI8Ring, (int)(sizeof kI8Ring / sizeof kI8Ring[0]), kI8RingModel, M, N, K, 1,
-                     std::min(scratch, kInt8ScratchBytes));
+  return ring_choose(kI8Ring, (int)(sizeof kI8Ring / sizeof kI8Ring[0]), kI8RingModel, M, N, K, 1, scratch);
 }
-size_t i8_ring_part(const RingChoice &p, int M, int N) {
-  return p.splits > 1 ? (size_t)p.splits * M * N * sizeof(float) : 0;
-}
-
 // Number of K splits: enough workgroups to cover the chip ~4x, each wave
 // keeping at least 8 steps.
 int choose_splits(int M, int N, int K) {
@@ -399,6 +466,7 @@ bool i8s_plan(int M, int N, int K, const pk_config *req, int cus, I8sPlan &best)
       } else {
         split_steps = (ksteps + s_req - 1) / s_req;
         if (s_req > 1 && split_steps < 4) break;
+        if (aliased_split(s_req, split_steps, N)) ++split_steps;
       }
       const int splits = (ksteps + split_steps - 1) / split_steps;
       const double units = (double)slices * splits * mblocks;
@@ -450,6 +518,10 @@ int int8_configs(int M, int N, int K, pk_config *out, int cap) {
       last = split_steps;
       if (n < cap && out) out[n] = i8s_config(v, split_steps);
       ++n;
+      if (aliased_split(s, split_steps, N)) {  // what i8s_plan takes instead
+        if (n < cap && out) out[n] = i8s_config(v, split_steps + 1);
+        ++n;
+      }
     }
   }
   return n;
@@ -520,28 +592,46 @@ int int8_run(int epi, const uint16_t *A, const int8_t *W, const float *scale, ui
   }
   I8sPlan plan;
   if (!cfg && aligned16(A) && aligned16(W) && aligned16(scale) && aligned16(C) && (epi != I8_RESID || aligned16(R))) {
-    // a caller's scratch is refused where the streaming or generic kernel's splits would not fit it
-    if (ws && i8_ring_plan(M, N, K, 0).tile >= 0) {
+    // a caller's scratch is refused where the column-split or generic kernel's splits would not fit it
+    if (ws) {
       if (int rc = check_workspace(i8s_plan(M, N, K, nullptr, device_cus(), plan) ? i8s_workspace(plan, M, N)
                                                                                   : generic_workspace(M, N, K, nullptr),
                                    ws_bytes))
         return rc;
     }
-    // caller scratch as it is, library scratch as far as it can be had
-    RingChoice p = i8_ring_plan(M, N, K, ws ? (aligned16(ws) ? ws_bytes : 0) : kInt8ScratchBytes);
+    // a caller's scratch as it is (launch_matmul_int8_noalloc's static buffer
+    // is the cap for all, so that calls with and without it split alike),
+    // library scratch as far as it can be had
+    KsPlan ks;
+    RingChoice ring;
+    auto choose = [&](size_t scratch) {
+      ks = KsPlan{};
+      scratch = std::min(scratch, kInt8ScratchBytes);
+      if (!kstream_plan(M, N, K, scratch, ks)) ring = i8_ring_plan(M, N, K, scratch);
+      const int splits = ks.v ? ks.splits : ring.tile >= 0 ? ring.splits : 1;
+      return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
+    };
     WorkspaceLease lease;
-    if (p.tile >= 0 && p.splits > 1 && !ws) {
-      int rc = library_workspace(0, i8_ring_part(p, M, N), st, lease);
+    const size_t part = choose(ws ? (aligned16(ws) ? ws_bytes : 0) : kInt8ScratchBytes);
+    float *partial = static_cast<float *>(ws);
+    if (part && !ws) {
+      int rc = library_workspace(0, part, st, lease);
       if (rc) return rc;
-      if (lease.bytes >= i8_ring_part(p, M, N)) ws = lease.ptr;
-      else p = i8_ring_plan(M, N, K, 0);
+      partial = static_cast<float *>(lease.ptr);
+      if (lease.bytes < part) choose(0);
     }
-    if (p.tile >= 0) {
-      const gk::GemmRingArgs a{{A, nullptr, C, nullptr, R, tab, M, N, K}, static_cast<float *>(ws), p.splits,
-                               p.split_tiles, W, scale};
-      kI8RingFn[p.tile][epi](dim3(p.units), st, a);
+    if (ks.v) {
+      const int units = ks.slices * ks.splits;
+      const I8sArgs a{A, W, scale, partial, C, R, tab, M, N, K, ks.splits, ks.split_steps, units};
+      ks.v->fn[epi](dim3(units, (M + 16 * ks.v->mt - 1) / (16 * ks.v->mt)), st, a);
+      PK_LAUNCH_CHECK("int8_kstream_kernel");
+      return ks.splits > 1 ? reduce_run(epi, Int8Args{A, W, scale, partial, C, R, tab, M, N, K, ks.splits, 0}, st) : PK_OK;
+    }
+    if (ring.tile >= 0) {
+      const gk::GemmRingArgs a{{A, nullptr, C, nullptr, R, tab, M, N, K}, partial, ring.splits, ring.split_tiles, W, scale};
+      kI8RingFn[ring.tile][epi](dim3(ring.units), st, a);
       PK_LAUNCH_CHECK("int8_ring_kernel");
-      return p.splits > 1 ? reduce_run(epi, Int8Args{A, W, scale, a.partial, C, R, tab, M, N, K, p.splits, 0}, st) : PK_OK;
+      return ring.splits > 1 ? reduce_run(epi, Int8Args{A, W, scale, partial, C, R, tab, M, N, K, ring.splits, 0}, st) : PK_OK;
     }
   }
   const bool fast = aligned16(A) && aligned16(W) && aligned16(scale) && aligned16(C) &&

@@ -384,5 +384,152 @@ __device__ __forceinline__ void stream_body(const I8sArgs &g) {
 
 }
 
+// ---------------------------------------------------------------------------
+// The same stream with K split over the waves (up to 32 rows; what
+// launch_matmul_int8 and the decode chain run unless a configuration asks for
+// stream_body).  A workgroup owns a slice of 16*NT columns and one K split; its
+// WK waves take the 64-row steps w, w + WK, ... of the split through private
+// rings, add their tiles in LDS and finish in place, so that a slice count
+// near the CU count needs no split partials and no second launch at all --
+// stream_body's waves split the slice by columns and leave 4-14 partials per
+// output to a reduction of 4-5 us.  Few waves and a short ring (2 waves of 2-3
+// stages) stream faster than many: the fewer rows of the matrix are in flight,
+// the more of them fall into open DRAM pages.  W and A stages, transpose reads
+// and widening as in stream_body; K % 8 == 0 (the last step's missing rows are
+// zeroed in A's fragments), N % 16 == 0, 16-byte aligned operands.
+// ---------------------------------------------------------------------------
+
+template <int NT, int MT, int WK, int STAGES, int EPI>
+__device__ __forceinline__ void kstream_body(const I8sArgs &g) {
+  static_assert(NT == 1 || NT == 2 || NT == 4 || NT == 8 || NT == 16, "column tiles");
+  constexpr int W_BYTES = 1024 * NT, STAGE = W_BYTES + 2048 * MT, RING = STAGES * STAGE;
+  constexpr int P = NT + 2 * MT;           // DMA instructions per step
+  constexpr int WN = 16 * NT, LD = WN + 4;
+  static_assert(16 * MT * LD * 4 <= RING, "the wave's partial tile reuses its ring");
+  __shared__ __attribute__((aligned(1024))) uint8_t ring[WK * RING];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wk = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // consecutive slices share the lines of narrow runs
+  const int u = xcd_unit(blockIdx.x, g.units);
+  const int slice = u / g.splits, split = u % g.splits;
+  const int n0 = slice * WN, m0 = blockIdx.y * 16 * MT;
+  const int ksteps = (g.K + I8S_KSTEP - 1) / I8S_KSTEP;
+  const int w0 = split * g.split_steps;
+  const int wsteps = min(ksteps, w0 + g.split_steps) - w0;
+  const int T = wsteps > wk ? (wsteps - wk + WK - 1) / WK : 0;
+
+  const pk_u32x4 w_rsrc = rsrc_words(g.W + n0, (uint32_t)((size_t)g.K * g.N - n0));
+  const pk_u32x4 a_rsrc = rsrc_words(g.A + (size_t)m0 * g.K, (uint32_t)((size_t)min(g.M - m0, 16 * MT) * g.K * 2));
+  uint32_t w_off[NT], a_off[2 * MT];
+#pragma unroll
+  for (int q = 0; q < NT; ++q) {
+    const int c = 64 * q + lane, row = c / NT, s = c % NT;
+    w_off[q] = (uint32_t)(row * g.N + min(16 * (s ^ i8s_xw<NT>(row)), g.N - 16 - n0));
+  }
+  const int a_k = 8 * ((lane & 7) ^ ((lane >> 3) & 7));  // k of the lane's A chunk (row = 8 q + lane / 8)
+#pragma unroll
+  for (int q = 0; q < 2 * MT; ++q) a_off[q] = (uint32_t)(min(8 * q + (lane >> 3), g.M - 1 - m0) * g.K + a_k) * 2u;
+
+  uint8_t *my = ring + wk * RING;
+  auto issue = [&](int st, int t) __attribute__((always_inline)) {
+    const int k0 = (w0 + wk + WK * t) * I8S_KSTEP;
+    uint8_t *base = my + st * STAGE;
+    if (k0 + I8S_KSTEP <= g.K) {
+#pragma unroll
+      for (int q = 0; q < NT; ++q) dma_lds16<true>(w_rsrc, base + 1024 * q, w_off[q], (uint32_t)k0 * g.N);
+#pragma unroll
+      for (int q = 0; q < 2 * MT; ++q) dma_lds16(a_rsrc, base + W_BYTES + 1024 * q, a_off[q], k0 * 2);
+    } else {  // rows past K repeat the last valid ones
+      const int last = g.K - 1 - k0;
+#pragma unroll
+      for (int q = 0; q < NT; ++q)
+        dma_lds16<true>(w_rsrc, base + 1024 * q, w_off[q] - (uint32_t)(max(0, (64 * q + lane) / NT - last) * g.N),
+                        (uint32_t)k0 * g.N);
+#pragma unroll
+      for (int q = 0; q < 2 * MT; ++q)
+        dma_lds16(a_rsrc, base + W_BYTES + 1024 * q, a_off[q] - (uint32_t)max(0, a_k - (last & ~7)) * 2u, k0 * 2);
+    }
+  };
+
+  const int grp = lane >> 4, gi = lane & 15;
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[mt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](int st, int k_left) __attribute__((always_inline)) {
+    const uint8_t *base = my + st * STAGE;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const bool none = 32 * kk + 8 * grp >= k_left;
+      bf16x8 af[MT];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const int row = 16 * mt + gi;
+        u32x4 v = *reinterpret_cast<const u32x4 *>(base + W_BYTES + row * 128 + 16 * ((4 * kk + grp) ^ (row & 7)));
+        if (none) v = u32x4{0, 0, 0, 0};
+        af[mt] = __builtin_bit_cast(bf16x8, v);
+      }
+      const int row = 32 * kk + 8 * grp + (gi >> 1);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const bf16x8 b = widen8(__builtin_amdgcn_ds_read_tr8_b64_v2i32(
+            (lds_v2i32 *)(base + row * WN + 16 * (j ^ i8s_xw<NT>(row)) + 8 * (gi & 1))));
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          acc[mt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, af[mt], acc[mt][j], 0, 0, 0);
+      }
+    }
+  };
+
+#pragma unroll
+  for (int p = 0; p < STAGES - 1; ++p)
+    if (p < T) issue(p, p);
+  int t = 0, st = 0;
+  for (; t + STAGES - 1 < T; ++t) {
+    lgkm_wait0();  // reads of the stage being refilled are done
+    issue(st == 0 ? STAGES - 1 : st - 1, t + STAGES - 1);
+    vm_wait<(STAGES - 1) * P>();
+    compute(st, I8S_KSTEP);
+    st = st == STAGES - 1 ? 0 : st + 1;
+  }
+  vm_wait<0>();
+  for (; t < T; ++t) {
+    compute(st, g.K - (w0 + wk + WK * t) * I8S_KSTEP);
+    st = st == STAGES - 1 ? 0 : st + 1;
+  }
+
+  // ---- add the WK tiles in wave order
+  lgkm_wait0();
+  float *tile = reinterpret_cast<float *>(my);
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+      *reinterpret_cast<f32x4 *>(tile + (16 * mt + gi) * LD + 16 * j + 4 * grp) = acc[mt][j];
+  __syncthreads();
+  constexpr int C8 = WN / 8;
+  for (int it = tid; it < 16 * MT * C8; it += WK * 64) {
+    const int r = it / C8, c = 8 * (it % C8);
+    const int m = m0 + r, n = n0 + c;
+    if (m >= g.M || n >= g.N) continue;
+    const float *p = reinterpret_cast<const float *>(ring) + r * LD + c;
+    f32x4 v0 = *reinterpret_cast<const f32x4 *>(p), v1 = *reinterpret_cast<const f32x4 *>(p + 4);
+#pragma unroll
+    for (int k = 1; k < WK; ++k) {
+      const float *q = p + k * (RING / 4);
+      v0 += *reinterpret_cast<const f32x4 *>(q);
+      v1 += *reinterpret_cast<const f32x4 *>(q + 4);
+    }
+    if (g.splits > 1) {
+      float *o = g.partial + ((size_t)split * g.M + m) * g.N + n;
+      *reinterpret_cast<f32x4 *>(o) = v0;
+      *reinterpret_cast<f32x4 *>(o + 4) = v1;
+    } else {
+      int8_epilogue8<EPI>(v0, v1, m, n, g.N, g.scale, g.R, g.gelu_tab, g.C);
+    }
+  }
+}
+
 }  // namespace i8s
 }  // namespace pk

@@ -331,6 +331,14 @@ __device__ __forceinline__ uint32_t gelu_pair_exact(uint32_t w, const uint16_t *
   return gelu_bits(w & 0xFFFFu, tab) | (gelu_bits(w >> 16, tab) << 16);
 }
 
+// Workgroup b of a one-dimensional grid runs on XCD b % 8: the unit that gives
+// each XCD a contiguous run of units, for any number of them, so that units
+// which share cache lines or panels share an L2.
+__device__ __forceinline__ int xcd_unit(int b, int units) {
+  const int xcd = b & 7;
+  return xcd * (units >> 3) + min(xcd, units & 7) + (b >> 3);
+}
+
 // ---- direct-to-LDS loads ----------------------------------------------------
 typedef __attribute__((address_space(3))) void lds_void;
 

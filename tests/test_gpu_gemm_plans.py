@@ -129,15 +129,19 @@ def test_rmsnorm_matmul_split(gpu, M, N, Kd):
         assert torch.equal(kernels.fused_rmsnorm_matmul(x, w, g, 1e-6).view(torch.int16), got.view(torch.int16))
 
 
-# the int8 ring kernel's five tiles (64 x 128 ... 160 x 256), K tails, K splits
+# the int8 K-split stream: slices of 16 to 128 columns (few, ragged, whole), rows
+# at the edges of its 16- and 32-row blocks, K tails of 8 to 56, K splits in
+# library scratch (long K) -- and above 32 rows the int8 ring kernel's five tiles (64 x 128 ... 160 x 256), K tails, K splits
 # (512 columns, long K), N with a ragged 16-column chunk
-@pytest.mark.parametrize("M,N,Kd", [(33, 16, 8), (65, 144, 72), (129, 272, 520), (48, 512, 4096), (300, 2064, 1032),
+@pytest.mark.parametrize("M,N,Kd", [(1, 16, 8), (16, 16, 72), (17, 144, 520), (5, 1040, 520), (32, 3968, 1472),
+                                    (3, 1472, 3968), (16, 2048, 8200), (32, 4096, 4160), (16, 16384, 136),
+                                    (9, 11008, 1024), (20, 16384, 512), (33, 16, 8), (65, 144, 72), (129, 272, 520), (48, 512, 4096), (300, 2064, 1032),
                                     (391, 6688, 64), (300, 12288, 64), (879, 6464, 72), (1060, 7184, 136),
                                     (600, 1040, 4104)])
-def test_int8_ring_integer_bit_exact(gpu, oracle, M, N, Kd):
+def test_int8_plans_integer_bit_exact(gpu, oracle, M, N, Kd):
     from polykernel_amd import _lib, kernels
 
-    print(f"int8 ring {M}x{N}x{Kd}", flush=True)
+    print(f"int8 {M}x{N}x{Kd}", flush=True)
     a, wq, s = _int8_exact_inputs(M, N, Kd, 160)
     r = rng_bf16((M, N), 163)
     da, dw, ds, dr = to_dev(a), to_dev(wq), to_dev(s), to_dev(r)
