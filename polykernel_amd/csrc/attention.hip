@@ -59,6 +59,18 @@ __global__ __launch_bounds__(FA_THREADS, 1) void attention_fa_kernel(FaArgs g) {
   fa_body<DP, QG, FUSED>(g);
 }
 
+// The 64 x 128 tile at D 64 with half the ring (two K and V slots, 70 KiB of
+// LDS): as it is, or in 128 registers so that two workgroups share a CU.  Same
+// bits as the full ring.
+constexpr int FA_RING_D64 = 64 * 1024;
+template <bool FUSED>
+__global__ __launch_bounds__(FA_THREADS, 1) void attention_fa_half_kernel(FaArgs g) {
+  fa_body<64, 2, FUSED, FA_RING_D64>(g);
+}
+__global__ __launch_bounds__(FA_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void attention_fa_pair_kernel(FaArgs g) {
+  fa_body<64, 2, false, FA_RING_D64>(g);
+}
+
 template <int DP>
 __global__ __launch_bounds__(256) void fa_combine_kernel(FaArgs g) {
   fa_combine_body<DP>(g);
@@ -69,7 +81,11 @@ __global__ __launch_bounds__(AD_THREADS) void attention_decode_kernel(FaArgs g) 
   att_decode_body<D, NQ>(g);
 }
 
-__global__ __launch_bounds__(256) void kv_append_kernel(pk_kv_append_args a) { kv_append_body(a); }
+// The appended rows of K and V in one launch (grid.y 2).
+__global__ __launch_bounds__(256) void kv_append_pair_kernel(pk_kv_append_args k, pk_kv_append_args v) {
+  if (blockIdx.y == 0) kv_append_body(k);
+  else kv_append_body(v);
+}
 
 // Launch an entry point of an emitted code object (hipModuleLaunchKernel),
 // with the same grid and arguments the linked kernel gets.
@@ -185,16 +201,25 @@ int attention_wide(AttArgs g, hipStream_t st, const AttModule *mod) {
   return PK_OK;
 }
 
-int kv_append_inplace_launch(uint16_t *cache, const uint16_t *neu, int64_t BH, int64_t Sc, int64_t Sn, int64_t D,
-                             int64_t cap, hipStream_t st, const AttModule *mod) {
+// The new rows of K and V into the caches: one launch, or an emitted object's
+// entry point twice.
+int kv_append_inplace_launch(uint16_t *Kc, const uint16_t *Kn, uint16_t *Vc, const uint16_t *Vn, int64_t BH, int64_t Sc,
+                             int64_t Sn, int64_t D, int64_t cap, hipStream_t st, const AttModule *mod) {
   if (BH * Sn * D == 0) return PK_OK;
-  const int vec = (D % 8 == 0) && aligned16(cache) && aligned16(neu);
-  const int64_t units = BH * Sn * (vec ? D / 8 : D);
-  const int grid = (int)std::min<int64_t>(std::max<int64_t>((units + 255) / 256, 1), 256 * 64);
-  pk_kv_append_args a{cache, neu, BH, Sc, Sn, D, cap, vec};
-  if (mod) return run_module(mod->kv_append, "pk_kv_append", grid, 256, a, st);
-  kv_append_kernel<<<grid, 256, 0, st>>>(a);
-  PK_LAUNCH_CHECK("kv_append_kernel");
+  auto args = [&](uint16_t *cache, const uint16_t *neu) {
+    return pk_kv_append_args{cache, neu, BH, Sc, Sn, D, cap, (D % 8 == 0) && aligned16(cache) && aligned16(neu)};
+  };
+  auto blocks = [&](const pk_kv_append_args &a) {
+    const int64_t units = BH * Sn * (a.vec ? D / 8 : D);
+    return (int)std::min<int64_t>(std::max<int64_t>((units + 255) / 256, 1), 256 * 64);
+  };
+  const pk_kv_append_args k = args(Kc, Kn), v = args(Vc, Vn);
+  if (mod) {
+    int rc = run_module(mod->kv_append, "pk_kv_append", blocks(k), 256, k, st);
+    return rc ? rc : run_module(mod->kv_append, "pk_kv_append", blocks(v), 256, v, st);
+  }
+  kv_append_pair_kernel<<<dim3(std::max(blocks(k), blocks(v)), 2), 256, 0, st>>>(k, v);
+  PK_LAUNCH_CHECK("kv_append_pair_kernel");
   return PK_OK;
 }
 
@@ -202,8 +227,8 @@ int kv_append_inplace_launch(uint16_t *cache, const uint16_t *neu, int64_t BH, i
 
 // The flash-style kernel when the shape suits it: D 64 or 128 and 16-byte
 // aligned tensors (callers also require scale > 0: the kernel tracks the
-// running max on unscaled scores).  With Kn/Vn (fused append) the new rows
-// must start on a key step of the tile shape (S_cache a multiple of bkv).
+// running max on unscaled scores).  With Kn/Vn (fused append) S_cache must be a
+// multiple of bkv.
 bool fa_applicable(int S_kv, int S_cache, int D, int kv_rows, const void *Q, const void *K, const void *V,
                    const void *O, const void *Kn, const void *Vn, const void *Kc, const void *Vc, int bkv) {
   if (D != 64 && D != 128) return false;
@@ -212,7 +237,7 @@ bool fa_applicable(int S_kv, int S_cache, int D, int kv_rows, const void *Q, con
   if ((size_t)kv_rows * D * 2 >= (size_t(1) << 31)) return false;
   if (Kn) {
     if (!aligned16(Kn) || !aligned16(Vn) || !aligned16(Kc) || !aligned16(Vc)) return false;
-    if (S_cache % bkv != 0) return false;  // one source per key step
+    if (S_cache % bkv != 0) return false;
     if ((size_t)(S_kv - S_cache) * D * 2 >= (size_t(1) << 31)) return false;
   }
   return true;
@@ -232,28 +257,73 @@ constexpr int fa_bkv(int qg) { return 32 * (FA_WAVES / qg); }
 // tiles balance it (measured at D 128: S_q 2048 91.7 against 102.5 us, 4096
 // 271 against 287 us, 2 x 2048 165 against 173 us; at 1024 queries 128 x 64
 // wins, 35.3 against 38.4 us, and without the mask it wins at every length).
-int fa_default_qg(int64_t BH, int S_q, bool causal) {
+//
+// At D 64 the 64 x 128 tile also runs with two workgroups per CU, whose
+// softmax and MFMA phases overlap (the kernel is VALU-bound there: 12 MFMAs
+// against ~120 VALU instructions per wave and step), so it wins from the second
+// round on (us, 128 x 64 / 64 x 128 / the pair, causal): 84 heads of 1224 72.2 /
+// 77.2 / 57.8, 32 of 4096 182 / 182 / 151, 40 of 1024 unmasked 42.5 / 38.6 /
+// 30.1, 32 of 1024 22.5 / 26.0 / 21.4; one round of 128 x 64 keeps short key
+// ranges (256 heads of 128 7.8 / 10.6 / 8.9, 64 of 512 15.4 / 19.2 / 15.5).
+int fa_default_qg(int64_t BH, int S_q, int S_kv, int D, bool causal) {
+  if (D == 64) {
+    const int64_t wide = BH * ((S_q + fa_bq(4) - 1) / fa_bq(4)), fine = BH * ((S_q + fa_bq(2) - 1) / fa_bq(2));
+    return wide <= 256 && fine > 256 && S_kv <= 512 ? 4 : 2;
+  }
   if (causal && S_q >= 2048) return 2;
   return BH * ((S_q + fa_bq(4) - 1) / fa_bq(4)) >= 256 ? 4 : 2;
 }
 
+// Whether the built-in choice runs two workgroups per CU (D 64, more than one
+// round).  The append stays out of that kernel: inside its 128 registers it
+// spilled (128 heads, 256 + 2048: 65.7 us against 46.8 fused in the 128 x 64 tile).
+bool fa_pairs(int64_t BH, int S_q, int D, int qg) {
+  return D == 64 && qg == 2 && BH * ((S_q + fa_bq(2) - 1) / fa_bq(2)) > 256;
+}
+
+// Key splits of the built-in choice: few tiles over many keys leave CUs idle, so
+// splits follow the time of the longest tile's steps (1.6 us each at D 128, 1.0
+// at 64) against the merge (4 us and its reads;
+// 8 heads of 500 queries and keys in 4 took 15.9 us against 12.7 unsplit), within one
+// round of 256 workgroups: 16 heads of 7 on 1000 cached keys 19.5 -> 14.6 us, 12
+// of 29 on 3200 26.1 -> 20.6.  A configuration keeps split_count's >= 8 steps.
+int fa_splits(int64_t tiles, int steps, int D) {
+  const double step_us = D == 128 ? 1.6 : 1.0;
+  int best = 1;
+  double best_us = 0.9 * steps * step_us;
+  for (int s = 2; s <= 16 && tiles * s <= 256 && s <= steps; s *= 2) {
+    const double us = (steps + s - 1) / s * step_us + 4.0 + 0.25 * s;
+    if (us < best_us) {
+      best_us = us;
+      best = s;
+    }
+  }
+  return best;
+}
+
 // Launch the flash-style kernel with QG query groups per workgroup, with
 // enough key splits to reach ~256 workgroups, each split keeping >= 8 steps.
-int attention_fa(FaArgs a, int D, int qg, hipStream_t st, const AttModule *mod) {
+// `built_in`: no configuration was asked for, so D 64 may take the half ring:
+// alone on a CU in one round ([32 heads, 333 + 1501] 21.3 -> 19.1 us, 16 of 1021
+// 14.1 -> 13.2; 32 of 512 on 4096 keys 36.0 -> 36.5), in pairs above.
+int attention_fa(FaArgs a, int D, int qg, bool built_in, hipStream_t st, const AttModule *mod) {
   const int BQ = fa_bq(qg), BKV = fa_bkv(qg);
   a.q_tiles = (a.S_q + BQ - 1) / BQ;
   const int ntiles = (a.S_kv + BKV - 1) / BKV;
-  a.splits = split_count((int64_t)a.BH * a.q_tiles, ntiles, 8, 8);
+  const size_t rows = (size_t)a.BH * a.S_q;
+  auto part_bytes = [&](int splits) { return splits > 1 ? (size_t)splits * rows * (D + 2) * sizeof(float) : 0; };
+  const int base = split_count((int64_t)a.BH * a.q_tiles, ntiles, 8, 8);
+  a.splits = built_in ? std::max(base, fa_splits((int64_t)a.BH * a.q_tiles, ntiles, D)) : base;
   if (int rc = grid_ok(a.BH, a.q_tiles, a.splits, "attention")) return rc;
   WorkspaceLease lease;  // held until the merge kernel is queued
   if (a.splits > 1) {
-    const size_t rows = (size_t)a.BH * a.S_q;
-    const size_t bytes_o = (size_t)a.splits * rows * D * sizeof(float);
-    const size_t bytes = bytes_o + (size_t)a.splits * rows * 2 * sizeof(float);
-    int rc = library_workspace(bytes, st, lease);
+    int rc = library_workspace(part_bytes(base), part_bytes(a.splits), st, lease);
     if (rc) return rc;
+    if (lease.bytes < part_bytes(a.splits)) a.splits = base;  // the workspace can't grow now
+  }
+  if (a.splits > 1) {
     a.part_o = static_cast<float *>(lease.ptr);
-    a.part_ml = reinterpret_cast<float *>(static_cast<char *>(lease.ptr) + bytes_o);
+    a.part_ml = a.part_o + (size_t)a.splits * rows * D;
   }
   const int blocks = a.BH * a.q_tiles * a.splits;
   const bool fused = a.Kn != nullptr;
@@ -272,7 +342,14 @@ int attention_fa(FaArgs a, int D, int qg, hipStream_t st, const AttModule *mod) 
     if (fused) attention_fa_kernel<DPV, QGV, true><<<blocks, FA_THREADS, 0, st>>>(a);       \
     else attention_fa_kernel<DPV, QGV, false><<<blocks, FA_THREADS, 0, st>>>(a);            \
   } while (0)
-  if (D == 128) {
+  if (built_in && D == 64 && qg == 2) {
+    if (!fa_pairs(a.BH, a.S_q, D, qg)) {
+      if (fused) attention_fa_half_kernel<true><<<blocks, FA_THREADS, 0, st>>>(a);
+      else attention_fa_half_kernel<false><<<blocks, FA_THREADS, 0, st>>>(a);
+    } else {
+      attention_fa_pair_kernel<<<blocks, FA_THREADS, 0, st>>>(a);
+    }
+  } else if (D == 128) {
     if (qg == 4) PK_FA_LAUNCH(128, 4);
     else PK_FA_LAUNCH(128, 2);
   } else {
@@ -376,7 +453,7 @@ int attention_configs(int S_q, int S_kv, int D, pk_config *out, int cap) {
 // causal mask (the op is the reference's causal KV-append prefill).
 bool attention_config(int S_q, int S_kv, int D, pk_config *out) {
   if (S_q <= 0 || S_kv <= 0 || D <= 0 || D > AW_DMAX) return false;
-  if (D == 64 || D == 128) *out = fa_config(fa_default_qg(32, S_q, true), D);
+  if (D == 64 || D == 128) *out = fa_config(fa_default_qg(32, S_q, S_kv, D, true), D);
   else generic_attention_config(D, out);
   return true;
 }
@@ -404,12 +481,12 @@ int attention_run(const uint16_t *Q, const uint16_t *K, const uint16_t *V, uint1
                             D, st);
   }
   if (mode >= 0) {
-    const int qg = mode ? mode : fa_default_qg(BH, S_q, causal != 0);
+    const int qg = mode ? mode : fa_default_qg(BH, S_q, S_kv, D, causal != 0);
     if (scale > 0.f && fa_applicable(S_kv, S_kv, D, kv_rows, Q, K, V, O, nullptr, nullptr, nullptr, nullptr,
                                      fa_bkv(qg))) {
       FaArgs a{Q, K, V, nullptr, nullptr, nullptr, nullptr, O, nullptr, nullptr, BH, S_q, S_kv, S_kv, kv_rows,
                scale, causal, 1, 1};
-      return attention_fa(a, D, qg, st, mod);
+      return attention_fa(a, D, qg, mode == 0, st, mod);
     }
     if (mode) {
       set_error("attention: the flash kernel (%d x %d tiles) needs D 64 or 128, 16-byte aligned tensors and "
@@ -453,22 +530,23 @@ int fused_kv_append_attention(const uint16_t *Q, uint16_t *Kc, uint16_t *Vc, con
                INT32_MAX);
   const int S_kv = S_cache + S_q;
   if (S_q > 0 && scale > 0.f && mode >= 0) {
-    int qg = mode ? mode : fa_default_qg(BH, S_q, causal != 0);
-    auto fits = [&](int g) {
-      return fa_applicable(S_kv, S_cache, D, cache_capacity, Q, Kc, Vc, O, Kn, Vn, Kc, Vc, fa_bkv(g));
+    int qg = mode ? mode : fa_default_qg(BH, S_q, S_kv, D, causal != 0);
+    // the append inside the attention kernel needs S_cache on a key step of the
+    // tile; the decode kernel takes any, the pair kernel none
+    auto fits = [&](int bkv) {
+      return fa_applicable(S_kv, S_cache, D, cache_capacity, Q, Kc, Vc, O, Kn, Vn, Kc, Vc, bkv);
     };
-    if (!mode && decode_applicable(S_q, S_kv, causal != 0) &&
-        fa_applicable(S_kv, S_cache, D, cache_capacity, Q, Kc, Vc, O, Kn, Vn, Kc, Vc, 1)) {
+    if (!mode && decode_applicable(S_q, S_kv, causal != 0) && fits(1)) {
       return attention_decode(FaArgs{Q, Kc, Vc, Kn, Vn, Kc, Vc, O, nullptr, nullptr, (int)BH, S_q, S_kv, S_cache,
                                      cache_capacity, scale, causal, 1, 1},
                               D, st);
     }
-    if (!mode && qg == 2 && !fits(2)) qg = 4;  // S_cache on a 64-key but not a 128-key step
-    if (fits(qg)) {
+    if (!mode && D == 128 && qg == 2 && !fits(fa_bkv(2))) qg = 4;  // S_cache on a 64-key but not a 128-key step
+    if (fits(fa_bkv(qg)) && !(!mode && fa_pairs(BH, S_q, D, qg))) {
       // the append happens inside the attention kernel
       FaArgs a{Q, Kc, Vc, Kn, Vn, Kc, Vc, O, nullptr, nullptr, (int)BH, S_q, S_kv, S_cache, cache_capacity,
                scale, causal, 1, 1};
-      return attention_fa(a, D, qg, st, mod);
+      return attention_fa(a, D, qg, mode == 0, st, mod);
     }
   }
   if (mode > 0) {
@@ -477,9 +555,7 @@ int fused_kv_append_attention(const uint16_t *Q, uint16_t *Kc, uint16_t *Vc, con
               fa_bq(mode), fa_bkv(mode), fa_bkv(mode));
     return PK_ERR_UNSUPPORTED;
   }
-  int rc = kv_append_inplace_launch(Kc, Kn, BH, S_cache, S_q, D, cache_capacity, st, mod);
-  if (rc) return rc;
-  rc = kv_append_inplace_launch(Vc, Vn, BH, S_cache, S_q, D, cache_capacity, st, mod);
+  int rc = kv_append_inplace_launch(Kc, Kn, Vc, Vn, BH, S_cache, S_q, D, cache_capacity, st, mod);
   if (rc) return rc;
   if (S_q == 0) return PK_OK;
   return attention_run(Q, Kc, Vc, O, (int)BH, S_q, S_kv, D, cache_capacity, scale, causal, mode, st, mod);

@@ -569,15 +569,15 @@ constexpr int FA_WAVES = 8;
 constexpr int FA_THREADS = FA_WAVES * 64;
 constexpr int FA_RING = 128 * 1024;  // bytes of LDS ring
 
-
-template <int DP, int QG, bool FUSED>
+// RING: bytes of LDS for the K and V tiles.
+template <int DP, int QG, bool FUSED, int RING = FA_RING>
 __device__ __forceinline__ void fa_body(FaArgs g) {
   constexpr int KH = FA_WAVES / QG;          // key blocks of 32 per step
   constexpr int BQ = 32 * QG;                // queries per workgroup
   constexpr int BKV = 32 * KH;               // keys per step
   constexpr int CH = DP / 8;                 // 16-byte chunks per row
   constexpr int TB = BKV * DP * 2;           // bytes of one K (or V) tile
-  constexpr int SL = FA_RING / (2 * TB);     // slots of the K ring and of the V ring
+  constexpr int SL = RING / (2 * TB);     // slots of the K ring and of the V ring
   constexpr int NK = TB / 1024;              // DMA instructions per tile
   constexpr int NPW = NK / (FA_WAVES / 2);   // per wave per step
   constexpr int RPI = 1024 / (2 * DP);       // rows per DMA instruction
@@ -586,7 +586,7 @@ __device__ __forceinline__ void fa_body(FaArgs g) {
   constexpr int PS = DP + 4;                 // merge-buffer row stride (floats), 16 B padding
   constexpr int MERGE = FA_WAVES * 32 * PS * 4;
   // the ring, reused as the merge buffer after the last step
-  __shared__ __attribute__((aligned(1024))) uint8_t ring[MERGE > FA_RING ? MERGE : FA_RING];
+  __shared__ __attribute__((aligned(1024))) uint8_t ring[MERGE > RING ? MERGE : RING];
   __shared__ float ml_s[FA_WAVES][32][2];
 
   const int tid = threadIdx.x, lane = tid & 63;

@@ -1,5 +1,6 @@
 """Attention of 1 to 4 queries per head (attention_decode_kernel): batch and
-wave edges of the key range, key splits, causal limits, the fused append."""
+wave edges of the key range, key splits, causal limits, the fused append; and
+the flash kernel's built-in choices at head dim 64 and at any cache length."""
 from __future__ import annotations
 
 import numpy as np
@@ -54,3 +55,34 @@ def test_decode_append_attention(gpu, oracle, B, H, Sq, Sc, spare, D):
         cache[:, :, Sc:Sc + Sq] = new
         assert np.array_equal(from_dev(dev), cache)
     _check(oracle, got, q, kc[:, :, :Sc + Sq], vc[:, :, :Sc + Sq], True)
+
+
+# more than 4 queries: the step that holds row S_cache reads cached and new
+# rows -- first, last or only step, one row from either edge, in the middle of
+# a long unmasked run, with key splits (few heads) and with D 64 in one round
+# (half ring) and several (pairs)
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,Sq,Sc", [(1, 2, 5, 1), (1, 2, 70, 127), (1, 2, 70, 129), (2, 3, 33, 1000), (1, 4, 600, 65),
+                                       (1, 2, 333, 1501), (2, 16, 600, 961), (3, 40, 130, 201)])
+def test_flash_append_any_cache_length(gpu, oracle, B, H, Sq, Sc, D):
+    from polykernel_amd import kernels
+
+    print(f"flash append B{B} H{H} Sq{Sq} Sc{Sc} D{D}", flush=True)
+    q, kn, vn = (synth.normal_bf16((B, H, Sq, D), 190 + i) for i in range(3))
+    kc, vc = (synth.normal_bf16((B, H, Sc + Sq + 3, D), 193 + i) for i in range(2))
+    dk, dv = to_dev(kc), to_dev(vc)
+    got = from_dev(kernels.fused_kv_append_attention(to_dev(q), to_dev(kn), to_dev(vn), dk, dv, Sc))
+    for cache, new, dev in ((kc, kn, dk), (vc, vn, dv)):
+        cache[:, :, Sc:Sc + Sq] = new
+        assert np.array_equal(from_dev(dev), cache)
+    _check(oracle, got, q, kc[:, :, :Sc + Sq], vc[:, :, :Sc + Sq], True)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("BH,Sq,Skv", [(4, 65, 300), (5, 600, 2500), (300, 70, 200), (130, 200, 700)])
+def test_flash_d64_rings(gpu, oracle, BH, Sq, Skv, causal):
+    from polykernel_amd import kernels
+
+    q, k, v = (synth.normal_bf16((1, BH, n, 64), 196 + i) for i, n in enumerate((Sq, Skv, Skv)))
+    got = from_dev(kernels.attention_prefill(to_dev(q), to_dev(k), to_dev(v), None, causal))
+    _check(oracle, got, q, k, v, causal)
