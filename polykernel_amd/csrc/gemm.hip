@@ -317,11 +317,14 @@ struct GemmPlan {
   }
 };
 GemmPlan gemm_plan(int M, int N, int K, bool dma, size_t scratch) {
-  GemmPlan p;
-  if (M <= kStreamRows && stream_plan(M, N, K, scratch, p.stream)) return p;
-  p.ring = ring_plan(M, N, K, scratch);
-  if (dma && dma_us(M, N, K) <= p.ring.us) p.ring = RingChoice{};
-  return p;
+  static thread_local PlanMemo<GemmPlan> memo;
+  return memo.get(M, N, K, scratch, dma, [&] {
+    GemmPlan p;
+    if (M <= kStreamRows && stream_plan(M, N, K, scratch, p.stream)) return p;
+    p.ring = ring_plan(M, N, K, scratch);
+    if (dma && dma_us(M, N, K) <= p.ring.us) p.ring = RingChoice{};
+    return p;
+  });
 }
 
 // Bytes of split partials the built-in choice wants for aligned operands (0:

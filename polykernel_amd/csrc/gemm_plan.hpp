@@ -59,4 +59,30 @@ inline RingChoice ring_choose(const RingTile *tiles, int ntiles, const RingModel
   return best;
 }
 
+// A thread's last plans, by shape and scratch (a plan depends on nothing else):
+// a program's layers come back to the same few shapes, and a plan costs 0.5-1.2
+// us of a call whose kernels may take 5.
+template <typename Plan, int SLOTS = 16>
+class PlanMemo {
+ public:
+  template <typename F>
+  const Plan &get(int M, int N, int K, size_t scratch, int kind, F &&make) {
+    const uint32_t h = (uint32_t)M * 0x9E3779B1u ^ (uint32_t)N * 0x85EBCA6Bu ^ (uint32_t)K * 0xC2B2AE35u ^
+                       (uint32_t)(scratch >> 8) * 0x27D4EB2Fu ^ (uint32_t)kind;
+    Slot &s = slots_[(h ^ h >> 15) % SLOTS];
+    if (!s.set || s.M != M || s.N != N || s.K != K || s.scratch != scratch || s.kind != kind)
+      s = Slot{true, M, N, K, kind, scratch, make()};
+    return s.plan;
+  }
+
+ private:
+  struct Slot {
+    bool set = false;
+    int M, N, K, kind;
+    size_t scratch;
+    Plan plan;
+  };
+  Slot slots_[SLOTS];
+};
+
 }  // namespace pk

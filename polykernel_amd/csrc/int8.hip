@@ -328,6 +328,21 @@ RingChoice i8_ring_plan(int M, int N, int K, size_t scratch) {
   if (M <= kI8RingRows) return RingChoice{};
   return ring_choose(kI8Ring, (int)(sizeof kI8Ring / sizeof kI8Ring[0]), kI8RingModel, M, N, K, 1, scratch);
 }
+// The built-in choice ahead of the column-split and generic kernels; neither
+// set: those.
+struct Int8Plan {
+  KsPlan ks;
+  RingChoice ring;
+};
+Int8Plan int8_plan(int M, int N, int K, size_t scratch) {
+  static thread_local PlanMemo<Int8Plan> memo;
+  return memo.get(M, N, K, scratch, 0, [&] {
+    Int8Plan p;
+    if (!kstream_plan(M, N, K, scratch, p.ks)) p.ring = i8_ring_plan(M, N, K, scratch);
+    return p;
+  });
+}
+
 // Number of K splits: enough workgroups to cover the chip ~4x, each wave
 // keeping at least 8 steps.
 int choose_splits(int M, int N, int K) {
@@ -428,8 +443,7 @@ double i8s_run_efficiency(int run, int waves) {
 // 192; [4096, 16384] 22.4 at 256, 19.5 at 208; [16384, 4096] 22.7 at 256,
 // 19.9 at 160), while 220-224 units stream at full rate.  Fields of `req`
 // that are nonzero are honoured; returns false when nothing matches.
-bool i8s_plan(int M, int N, int K, const pk_config *req, int cus, I8sPlan &best) {
-  if (!i8s_shape_ok(M, N, K)) return false;
+bool i8s_search(int M, int N, int K, const pk_config *req, int cus, I8sPlan &best) {
   const int ksteps = K / I8S_KSTEP;
   // rows per block: 16 up to M 16, 32 up to M 64 (two blocks at M 64: the
   // 64-row variant holds only two ring stages; measured M 64 [8192, 28672]
@@ -486,6 +500,18 @@ bool i8s_plan(int M, int N, int K, const pk_config *req, int cus, I8sPlan &best)
     }
   }
   return found;
+}
+
+bool i8s_plan(int M, int N, int K, const pk_config *req, int cus, I8sPlan &best) {
+  if (!i8s_shape_ok(M, N, K)) return false;
+  if (req) return i8s_search(M, N, K, req, cus, best);
+  static thread_local PlanMemo<I8sPlan> memo;  // v null: no variant takes the shape
+  best = memo.get(M, N, K, 0, cus, [&] {
+    I8sPlan p;
+    if (!i8s_search(M, N, K, nullptr, cus, p)) p = I8sPlan{};
+    return p;
+  });
+  return best.v != nullptr;
 }
 
 size_t i8s_workspace(const I8sPlan &p, int M, int N) {
@@ -602,13 +628,10 @@ int int8_run(int epi, const uint16_t *A, const int8_t *W, const float *scale, ui
     // a caller's scratch as it is (launch_matmul_int8_noalloc's static buffer
     // is the cap for all, so that calls with and without it split alike),
     // library scratch as far as it can be had
-    KsPlan ks;
-    RingChoice ring;
+    Int8Plan p;
     auto choose = [&](size_t scratch) {
-      ks = KsPlan{};
-      scratch = std::min(scratch, kInt8ScratchBytes);
-      if (!kstream_plan(M, N, K, scratch, ks)) ring = i8_ring_plan(M, N, K, scratch);
-      const int splits = ks.v ? ks.splits : ring.tile >= 0 ? ring.splits : 1;
+      p = int8_plan(M, N, K, std::min(scratch, kInt8ScratchBytes));
+      const int splits = p.ks.v ? p.ks.splits : p.ring.tile >= 0 ? p.ring.splits : 1;
       return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
     };
     WorkspaceLease lease;
@@ -620,6 +643,8 @@ int int8_run(int epi, const uint16_t *A, const int8_t *W, const float *scale, ui
       partial = static_cast<float *>(lease.ptr);
       if (lease.bytes < part) choose(0);
     }
+    const KsPlan &ks = p.ks;
+    const RingChoice &ring = p.ring;
     if (ks.v) {
       const int units = ks.slices * ks.splits;
       const I8sArgs a{A, W, scale, partial, C, R, tab, M, N, K, ks.splits, ks.split_steps, units};

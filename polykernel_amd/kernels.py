@@ -20,8 +20,16 @@ from ._lib import check
 bf16 = torch.bfloat16
 
 
+# torch's own handle of the current stream: torch.cuda.current_stream() builds a
+# Stream object around it, 2.8 us of the 9.3 us that a small call took.
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
+_current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    if _current_raw_stream is None or _current_device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _current_raw_stream(_current_device())
 
 
 def _dev(t: torch.Tensor, dtype: torch.dtype, name: str) -> int:
