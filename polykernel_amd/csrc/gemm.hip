@@ -483,6 +483,30 @@ bool rmsnorm_matmul_config(int M, int N, int K, pk_config *out) {
   return gemm_default(M, N, K, out);
 }
 
+// The library workspace of a row normalisation followed by the GEMM: the rows,
+// and behind them the GEMM's split partials where the workspace can hold them
+// (*part: their bytes, 0 if not).
+int normed_rows_workspace(int M, int N, int K, void *st, WorkspaceLease &lease, void **scratch, size_t *part) {
+  const size_t row_bytes = ((size_t)M * K * 2 + 255) & ~size_t(255);
+  *part = gemm_scratch_bytes(M, N, K);
+  int rc = library_workspace((size_t)M * K * 2, *part ? row_bytes + *part : (size_t)M * K * 2, st, lease);
+  if (rc) return rc;
+  *scratch = static_cast<char *>(lease.ptr) + row_bytes;
+  if (lease.bytes < row_bytes + *part) *part = 0;
+  return PK_OK;
+}
+
+int gemm_planned(const uint16_t *A, const uint16_t *B, uint16_t *C, int M, int N, int K, void *scratch,
+                 size_t scratch_bytes, void *st, bool *ran) {
+  const GemmArgs g{A, B, C, nullptr, nullptr, nullptr, M, N, K};
+  *ran = false;
+  if (!gemm_vec_ok(g)) return PK_OK;
+  const GemmPlan p = gemm_plan(M, N, K, gemm_dma_fits(g), std::min(scratch_bytes, kGemmScratchMax));
+  if (!p.stream.v && p.ring.tile < 0) return PK_OK;
+  *ran = true;
+  return gemm_run(EPI_NONE, A, B, C, nullptr, nullptr, M, N, K, (hipStream_t)st, -1, scratch, scratch_bytes);
+}
+
 int fused_rmsnorm_matmul(const uint16_t *x, const uint16_t *gamma, const uint16_t *W, uint16_t *out,
                          int M, int N, int K, float eps, hipStream_t st, const char *name) {
   PK_CHECK_ARG(x && W && out, "%s: null tensor pointer", name);
@@ -499,18 +523,16 @@ int fused_rmsnorm_matmul(const uint16_t *x, const uint16_t *gamma, const uint16_
     PK_LAUNCH_CHECK(name);
     return PK_OK;
   }
-  // Otherwise: normalise once into library workspace, then the plain GEMM, its
-  // split partials behind the rows where the workspace can hold them too.
+  // Otherwise: normalise once into library workspace, then the plain GEMM.
   WorkspaceLease lease;  // held until the GEMM that reads the panel is queued
-  const size_t row_bytes = ((size_t)M * K * 2 + 255) & ~size_t(255);
-  const size_t part = gemm_scratch_bytes(M, N, K);
-  int rc = library_workspace((size_t)M * K * 2, part ? row_bytes + part : (size_t)M * K * 2, st, lease);
+  void *scratch = nullptr;
+  size_t part = 0;
+  int rc = normed_rows_workspace(M, N, K, st, lease, &scratch, &part);
   if (rc) return rc;
   uint16_t *a = static_cast<uint16_t *>(lease.ptr);
   rc = rmsnorm_launch(x, gamma, a, M, K, eps, st);
   if (rc) return rc;
-  return gemm_run(EPI_NONE, a, W, out, nullptr, nullptr, M, N, K, st, -1, static_cast<char *>(lease.ptr) + row_bytes,
-                  lease.bytes >= row_bytes + part ? part : 0);
+  return gemm_run(EPI_NONE, a, W, out, nullptr, nullptr, M, N, K, st, -1, scratch, part);
 }
 
 }  // namespace pk

@@ -375,7 +375,9 @@ LaunchFn CodeObjectPanelLauncher(std::shared_ptr<ModuleTable> table) {
     ModuleTable::Loaded *mod = table->Get(*bin, {"pk_row", "pk_row_any", "pk_gemm"}, error);
     if (!mod) return false;
     WorkspaceLease lease;  // the normalised rows, held until the GEMM is queued
-    if (library_workspace((size_t)p->M * p->K * 2, p->stream, lease) != PK_OK) {
+    void *scratch = nullptr;
+    size_t part = 0;
+    if (normed_rows_workspace(p->M, p->N, p->K, p->stream, lease, &scratch, &part) != PK_OK) {
       error = std::string("library workspace: ") + pk_last_error();
       return false;
     }
@@ -385,6 +387,14 @@ LaunchFn CodeObjectPanelLauncher(std::shared_ptr<ModuleTable> table) {
     if (!RowLaunch(mod, row, pk_row_args{p->x, nullptr, p->gamma, xn, p->M, p->K, 1.0f / (float)p->K, p->eps},
                    p->stream, error))
       return false;
+    // the entry point's choice for few rows or tiles is no configuration: its
+    // kernel then forms the product, so that a served call gives its bits
+    bool ran = false;
+    if (gemm_planned(xn, p->W, p->out, p->M, p->N, p->K, scratch, part, p->stream, &ran) != PK_OK) {
+      error = std::string("RMSNorm -> MatMul: ") + pk_last_error();
+      return false;
+    }
+    if (ran) return true;
     pk_gemm_args g{xn, p->W, p->out, nullptr, nullptr, nullptr, p->M, p->N, p->K};
     unsigned tiles = 0;
     if (!TileGrid(p->M, p->N, p->K, c.block_m, c.block_n, tiles, error)) return false;

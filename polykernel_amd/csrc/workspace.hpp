@@ -38,6 +38,14 @@ int library_workspace(size_t bytes, void *stream, WorkspaceLease &lease);
 // short (lease.bytes tells), and is refused only where `need` would be.
 int library_workspace(size_t need, size_t want, void *stream, WorkspaceLease &lease);
 
+// RMSNorm -> MatMul outside the panel kernel, for its launchers: the workspace
+// lease (lease.ptr: the normalised rows; *scratch: *part bytes for split
+// partials), and the product of aligned rows where the entry point's choice
+// is a kernel that no configuration names (*ran; otherwise nothing is launched).
+int normed_rows_workspace(int M, int N, int K, void *stream, WorkspaceLease &lease, void **scratch, size_t *part);
+int gemm_planned(const unsigned short *A, const unsigned short *B, unsigned short *C, int M, int N, int K, void *scratch,
+                 size_t scratch_bytes, void *stream, bool *ran);
+
 // Frees the calling device's slot of `stream` after hipStreamSynchronize on
 // it; the next call on that stream allocates again.  PK_OK when there is no
 // slot.
