@@ -42,6 +42,11 @@ __global__ __launch_bounds__(NW > 4 ? NW * 64 : kBlock) void rmsnorm_vec_kernel(
   rmsnorm_vec_body<NW, VPT, RESID>(a);
 }
 
+template <int VPT, bool RESID>
+__global__ __launch_bounds__(VPT * 64) void rmsnorm_shared_kernel(RowArgs a) {
+  rmsnorm_shared_body<VPT, RESID>(a);
+}
+
 template <bool RESID>
 __global__ __launch_bounds__(kBlock) void rmsnorm_generic_kernel(RowArgs a) {
   rmsnorm_generic_body<RESID>(a);
@@ -245,6 +250,25 @@ bool softmax_ragged_run(const RowArgs &a, hipStream_t st) {
   return true;
 }
 
+// The workgroup-per-row kernel for few rows, whose time is that of a single
+// row's chain: up to 512 rows, 1024 with a residual.  us in a replayed graph,
+// one wave per row against a workgroup: RMSNorm [16, 4096] 5.17, 3.49;
+// [512, 4096] 5.89, 4.63; [1024, 4096] 7.39, 7.76; [16, 1024] 2.83, 2.45.
+// Residual + RMSNorm [16, 4096] 7.53, 3.56; [1024, 4096] 11.25, 8.62;
+// [1024, 1024] 3.80, 3.20; [4096, 3072] 19.0, 20.2.  Rows of at most 64
+// vectors have nothing to share, longer ones than 512 their own workgroup.
+// False: another kernel's rows.
+template <bool RESID>
+bool rmsnorm_shared_run(const RowArgs &a, const pk_config &c, hipStream_t st) {
+  if (c.block_m != 4 || a.rows > (RESID ? 1024 : 512)) return false;
+  const unsigned rows = (unsigned)a.rows;
+  switch (c.unroll) {
+    case 2: rmsnorm_shared_kernel<2, RESID><<<rows, 128, 0, st>>>(a); return true;
+    case 4: rmsnorm_shared_kernel<4, RESID><<<rows, 256, 0, st>>>(a); return true;
+    case 8: rmsnorm_shared_kernel<8, RESID><<<rows, 512, 0, st>>>(a); return true;
+  }
+  return false;
+}
 // cfg null: the built-in choice (the first candidate, or the generic kernel
 // when the operands are not 16-byte aligned); otherwise a listed config, which
 // must be the generic one when they are not.
@@ -270,6 +294,10 @@ int rmsnorm_dispatch(const uint16_t *x, const uint16_t *r, const uint16_t *w, ui
   } else {
     row_configs(false, rows, cols, &c, 1);
     if (!aligned) c = pk_config{1, cols, 0, 4, 1, 1, 1};
+    if (aligned && rmsnorm_shared_run<RESID>(a, c, st)) {
+      PK_LAUNCH_CHECK(name);
+      return PK_OK;
+    }
   }
   int rc = rmsnorm_run<RESID>(a, c, st);
   if (rc) return rc;

@@ -182,6 +182,64 @@ __device__ __forceinline__ void rmsnorm_vec_body(const RowArgs &a) {
   }
 }
 
+// Few rows of at most VPT * 64 vectors: a workgroup of VPT waves per row.  A
+// few rows leave the chip idle, and one wave of rmsnorm_vec_body<1, VPT> is a
+// serial chain: 8 VPT divisions per lane, gamma fetched only after the sum.
+// Here wave i loads vector i of each lane's column set (and its gamma), adds
+// the residual and leaves the bf16 words in LDS; every wave then forms the
+// whole sum from LDS in the one-wave kernel's order, so that the bits are that
+// kernel's, and divides and stores its own vector.
+template <int VPT, bool RESID>
+__device__ __forceinline__ void rmsnorm_shared_body(const RowArgs &a) {
+#pragma clang fp contract(off)
+  __shared__ U4 words[VPT * 64];
+  const uint16_t *__restrict__ x = static_cast<const uint16_t *>(a.in);
+  const uint16_t *__restrict__ w = a.gamma;
+  const int lane = threadIdx.x & 63, mine = threadIdx.x, nvec = a.cols >> 3;
+  const size_t at = (size_t)blockIdx.x * a.cols + (size_t)mine * 8;
+  U4 xw{0, 0, 0, 0}, gw{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};  // bf16 1.0
+  float v[8];
+  if (mine < nvec) {
+    xw = ld16(x + at);
+    U4 rw;
+    if constexpr (RESID) rw = ld16(a.aux + at);
+    if (w) gw = ld16(w + (size_t)mine * 8);
+    if constexpr (RESID) {
+      float rv[8];
+      unpack8(xw, v);
+      unpack8(rw, rv);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = v[e] + rv[e];
+      xw = pack8(v);
+    }
+  }
+  words[mine] = xw;
+  __syncthreads();
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    if (lane + i * 64 < nvec) {
+      float t[8];
+      unpack8(words[lane + i * 64], t);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss += t[e] * t[e];
+    }
+  }
+  ss = wave_sum(ss);
+  const float rms = sqrtf(ss * a.inv_cols + a.eps);
+  if (mine >= nvec) return;
+  float o[8], g[8];
+  unpack8(xw, v);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = v[e] / rms;
+  if (w) {
+    unpack8(gw, g);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] *= g[e];
+  }
+  st16(a.out + at, pack8(o));
+}
+
 // Generic path (any cols / alignment): one block per row, two passes over the
 // row (the second from cache).  Column indices are unsigned so that stepping
 // past a cols near INT32_MAX cannot wrap.
