@@ -24,6 +24,7 @@
 
 #include "gemm_kernels.hpp"
 #include "gemm_plan.hpp"
+#include "gemm_odd.hpp"
 #include "gemm_ring.hpp"
 
 namespace pk {
@@ -49,6 +50,10 @@ __global__ __launch_bounds__(WK * 64) void gemm_stream_kernel(GemmStreamArgs a) 
   gemm_stream_body<NT, MT, WK, STAGES, EPI>(a);
 }
 
+template <int NT, int MT, int WK, int DEPTH>
+__global__ __launch_bounds__(WK * 64, 1) void gemm_odd_kernel(GemmArgs g) {
+  gemm_odd_body<NT, MT, WK, DEPTH>(g);
+}
 template <int FM, int WN, int STAGES, int EPI>
 __global__ __launch_bounds__(GR_THREADS, 1) void gemm_ring_kernel(GemmRingArgs a) {
   gemm_ring_body<FM, WN, STAGES, EPI>(a);
@@ -267,6 +272,27 @@ int stream_run(int epi, const GemmArgs &g, const StreamPlan &p, void *scratch, h
   return p.splits > 1 ? reduce_run(epi, g, a.partial, p.splits, st) : PK_OK;
 }
 
+// ---- few rows and weights without 16-byte rows (gemm_odd.hpp) ---------------
+// At most kStreamRows rows of A in whole 16-byte chunks; B and C at any element.
+// Against the 64 x 64 tiles with element loads (us, rotating weights): [1, 50257,
+// 2048] 251 / 45.5, [64, 50257, 4096] 580 / 115, [16, 12001, 4096] 261 / 27.6, [8,
+// 5003, 2048] 99 / 9.1, [64, 2101, 512] 26.1 / 12.4.  Wide slices share fewer
+// lines at their edges and are taken where they still fill the chip.
+bool odd_ok(const GemmArgs &g) {
+  return g.M <= kStreamRows && g.K % 8 == 0 && g.N >= 8 && aligned16(g.A) && (size_t)g.K * g.N * 2 < (size_t(1) << 31);
+}
+template <int MT>
+int odd_run(const GemmArgs &g, hipStream_t st) {
+  if (g.N >= 128 * 160) gemm_odd_kernel<8, MT, 4, 3><<<(g.N + 127) / 128, 256, 0, st>>>(g);
+  else if (g.N >= 64 * 128) gemm_odd_kernel<4, MT, 8, 4><<<(g.N + 63) / 64, 512, 0, st>>>(g);
+  else gemm_odd_kernel<2, MT, 8, 5><<<(g.N + 31) / 32, 512, 0, st>>>(g);
+  PK_LAUNCH_CHECK("gemm_odd_kernel");
+  return PK_OK;
+}
+int odd_run(const GemmArgs &g, hipStream_t st) {
+  return g.M <= 16 ? odd_run<1>(g, st) : g.M <= 32 ? odd_run<2>(g, st) : odd_run<4>(g, st);
+}
+
 // ---- prompt-sized calls (gemm_ring.hpp) -------------------------------------
 using RingLaunch = void (*)(dim3, hipStream_t, const GemmRingArgs &);
 template <int FM, int WN, int STAGES, int EPI>
@@ -440,6 +466,7 @@ int gemm_run(int epi, const uint16_t *A, const uint16_t *B, uint16_t *C, const u
     if (p.stream.v) return stream_run(epi, g, p.stream, scratch, st);
     if (p.ring.tile >= 0) return ring_run(epi, g, p.ring, scratch, st);
   }
+  if (tile < 0 && epi == EPI_NONE && !gemm_vec_ok(g) && odd_ok(g)) return odd_run(g, st);
   if (tile < 0) tile = gemm_dma_fits(g) ? 0 : pick_tile(M, N, false);
   switch (epi) {
     case EPI_NONE: return gemm_dispatch<EPI_NONE>(g, tile, st);
@@ -500,9 +527,12 @@ int gemm_planned(const uint16_t *A, const uint16_t *B, uint16_t *C, int M, int N
                  size_t scratch_bytes, void *st, bool *ran) {
   const GemmArgs g{A, B, C, nullptr, nullptr, nullptr, M, N, K};
   *ran = false;
-  if (!gemm_vec_ok(g)) return PK_OK;
-  const GemmPlan p = gemm_plan(M, N, K, gemm_dma_fits(g), std::min(scratch_bytes, kGemmScratchMax));
-  if (!p.stream.v && p.ring.tile < 0) return PK_OK;
+  if (gemm_vec_ok(g)) {
+    const GemmPlan p = gemm_plan(M, N, K, gemm_dma_fits(g), std::min(scratch_bytes, kGemmScratchMax));
+    if (!p.stream.v && p.ring.tile < 0) return PK_OK;
+  } else if (!odd_ok(g)) {
+    return PK_OK;
+  }
   *ran = true;
   return gemm_run(EPI_NONE, A, B, C, nullptr, nullptr, M, N, K, (hipStream_t)st, -1, scratch, scratch_bytes);
 }

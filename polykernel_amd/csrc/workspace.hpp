@@ -40,7 +40,7 @@ int library_workspace(size_t need, size_t want, void *stream, WorkspaceLease &le
 
 // RMSNorm -> MatMul outside the panel kernel, for its launchers: the workspace
 // lease (lease.ptr: the normalised rows; *scratch: *part bytes for split
-// partials), and the product of aligned rows where the entry point's choice
+// partials), and the product where the entry point's choice
 // is a kernel that no configuration names (*ran; otherwise nothing is launched).
 int normed_rows_workspace(int M, int N, int K, void *stream, WorkspaceLease &lease, void **scratch, size_t *part);
 int gemm_planned(const unsigned short *A, const unsigned short *B, unsigned short *C, int M, int N, int K, void *scratch,
