@@ -274,6 +274,24 @@ PK_API int pk_gemm_config_ex(int epi, const uint16_t *A, const uint16_t *B, uint
                              const uint16_t *bias, const uint16_t *R, int M, int N, int K,
                              const pk_config *cfg, void *stream);
 
+/* The kernel an entry point's built-in choice runs: PK_PLAN_TILE (a
+ * configuration or the generic kernel) or one of the kernels that are no
+ * configuration, its rows and columns per workgroup, the splits of K (or of the
+ * keys) and the k-steps of each. */
+enum { PK_PLAN_TILE = 0, PK_PLAN_STREAM = 1, PK_PLAN_RING = 2, PK_PLAN_ODD = 3 };
+typedef struct pk_plan {
+  int kernel, block_m, block_n, splits, split_steps;
+} pk_plan;
+
+/* Test hooks: the plan of a GEMM with 16-byte aligned operands, epilogue `epi`
+ * (as pk_gemm_ex) and `scratch_bytes` of room for split partials (no device is
+ * needed), and one GEMM by a given stream or ring plan, whose partials go to
+ * `workspace`.  A plan no variant matches returns PK_ERR_UNSUPPORTED. */
+PK_API int pk_gemm_plan(int epi, int M, int N, int K, size_t scratch_bytes, pk_plan *out);
+PK_API int pk_gemm_plan_ex(int epi, const uint16_t *A, const uint16_t *B, uint16_t *C,
+                           const uint16_t *bias, const uint16_t *R, int M, int N, int K,
+                           const pk_plan *plan, void *workspace, size_t workspace_bytes, void *stream);
+
 /* launch_fused_kv_append_attention with an explicit configuration (one of
  * pk_op_configs("fused_kv_append_attention", S_q, S_cache + S_q, D); NULL =
  * built-in choice).  A flash configuration the operands do not allow

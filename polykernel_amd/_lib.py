@@ -44,6 +44,15 @@ class Config(C.Structure):
         return {f: getattr(self, f) for f, _ in self._fields_}
 
 
+class Plan(C.Structure):
+    """struct pk_plan (include/polykernel_amd.h): the kernel of a built-in choice."""
+
+    _fields_ = [("kernel", C.c_int), ("block_m", C.c_int), ("block_n", C.c_int), ("splits", C.c_int),
+                ("split_steps", C.c_int)]
+
+
+PLAN_TILE, PLAN_STREAM, PLAN_RING, PLAN_ODD = range(4)
+
 P = C.c_void_p
 I = C.c_int
 F = C.c_float
@@ -90,6 +99,8 @@ SIGNATURES = {
     "pk_int8_default_config": (I, [I, I, I, C.POINTER(Config)]),
     "pk_matmul_int8_ex": (I, [I, P, P, P, P, P, I, I, I, C.POINTER(Config), P, SZ, P]),
     "pk_gemm_config_ex": (I, [I, P, P, P, P, P, I, I, I, C.POINTER(Config), P]),
+    "pk_gemm_plan": (I, [I, I, I, I, SZ, C.POINTER(Plan)]),
+    "pk_gemm_plan_ex": (I, [I, P, P, P, P, P, I, I, I, C.POINTER(Plan), P, SZ, P]),
     "pk_op_configs": (I, [C.c_char_p, LL, LL, LL, C.POINTER(Config), I]),
     "pk_op_default_config": (I, [C.c_char_p, LL, LL, LL, C.POINTER(Config)]),
     "pk_naive_matmul": (I, [I, P, P, P, P, P, I, I, I, P]),

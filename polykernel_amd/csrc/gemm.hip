@@ -203,9 +203,11 @@ struct StreamPlan {
   int splits = 1, split_steps = 0, slices = 0;
 };
 
-// Whether the streaming kernel takes the shape (operands 16-byte aligned).
+// Whether the streaming kernel takes the shape (operands 16-byte aligned): its
+// buffer descriptors and lane offsets hold both operands in 32 bits.
 bool stream_shape_ok(int M, int N, int K) {
-  return M <= kStreamRows && N % 8 == 0 && K % 8 == 0 && (size_t)K * N * 2 < (size_t(1) << 31);
+  return M <= kStreamRows && N % 8 == 0 && K % 8 == 0 && (size_t)K * N * 2 < (size_t(1) << 31) &&
+         (size_t)M * K * 2 < (size_t(1) << 31);
 }
 
 // Slice width and K splits by a time model (us) fitted to the same sweep: 3
@@ -667,6 +669,68 @@ int pk_gemm_ex(int epi, const uint16_t *A, const uint16_t *B, uint16_t *C, const
   PK_CHECK_ARG(M > 0 && N > 0 && K > 0, "pk_gemm_ex: invalid shape");
   PK_CHECK_ARG(epi >= 0 && epi <= 3 && tile >= -1 && tile <= 3, "pk_gemm_ex: bad epi/tile");
   return gemm_run(epi, A, B, C, bias, R, M, N, K, (hipStream_t)stream, tile);
+}
+
+int pk_gemm_plan(int epi, int M, int N, int K, size_t scratch_bytes, pk_plan *out) {
+  PK_CHECK_ARG(out && M > 0 && N > 0 && K > 0 && epi >= 0 && epi <= 3, "pk_gemm_plan: invalid argument");
+  if (int rc = tile_grid_ok(M, N, K, 64, 64, "pk_gemm_plan")) return rc;
+  *out = pk_plan{};
+  out->splits = 1;
+  if (K % 8 == 0 && N % 8 == 0) {
+    const GemmPlan p = gemm_plan(M, N, K, gemm_dma_shape_ok(N, K), std::min(scratch_bytes, kGemmScratchMax));
+    if (p.stream.v) {
+      *out = pk_plan{PK_PLAN_STREAM, 16 * p.stream.v->mt, 16 * p.stream.v->nt, p.stream.splits, p.stream.split_steps};
+      return PK_OK;
+    }
+    if (p.ring.tile >= 0) {
+      const RingTile &t = kRing[p.ring.tile];
+      *out = pk_plan{PK_PLAN_RING, 32 * t.fm, 64 * t.wn, p.ring.splits, p.ring.split_tiles};
+      return PK_OK;
+    }
+  } else if (epi == EPI_NONE && odd_ok(GemmArgs{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K})) {
+    out->kernel = PK_PLAN_ODD;
+    return PK_OK;
+  }
+  const int tile = K % 8 == 0 && N % 8 == 0 && gemm_dma_shape_ok(N, K) ? 0 : pick_tile(M, N, false);
+  out->block_m = out->block_n = tile == 0 ? 256 : tile == 1 ? 128 : 64;
+  return PK_OK;
+}
+
+int pk_gemm_plan_ex(int epi, const uint16_t *A, const uint16_t *B, uint16_t *C, const uint16_t *bias,
+                    const uint16_t *R, int M, int N, int K, const pk_plan *plan, void *workspace,
+                    size_t workspace_bytes, void *stream) {
+  PK_CHECK_ARG(A && B && C && plan, "pk_gemm_plan_ex: null pointer");
+  PK_CHECK_ARG(M > 0 && N > 0 && K > 0 && epi >= 0 && epi <= 3, "pk_gemm_plan_ex: invalid shape or epilogue");
+  PK_CHECK_ARG(plan->splits >= 1, "pk_gemm_plan_ex: splits %d", plan->splits);
+  if (int rc = tile_grid_ok(M, N, K, 64, 64, "pk_gemm_plan_ex")) return rc;
+  GemmArgs g{A, B, C, bias, R, nullptr, M, N, K};
+  if (epi == EPI_BIAS_GELU)
+    if (int rc = gelu_table(&g.gelu_tab)) return rc;
+  // the splits of the plan as the planners form them: whole k-steps, none empty
+  const bool stream_kernel = plan->kernel == PK_PLAN_STREAM;
+  const int ksteps = (K + (stream_kernel ? GS_KSTEP : GR_BK) - 1) / (stream_kernel ? GS_KSTEP : GR_BK);
+  const int steps = (ksteps + plan->splits - 1) / plan->splits, splits = (ksteps + steps - 1) / steps;
+  const size_t part = splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
+  if (part && (workspace_bytes < part || !aligned16(workspace))) {
+    set_error("pk_gemm_plan_ex: %zu aligned bytes of workspace required, got %zu", part, workspace_bytes);
+    return PK_ERR_WORKSPACE;
+  }
+  if (stream_kernel && gemm_vec_ok(g) && stream_shape_ok(M, N, K)) {
+    for (const StreamVariant &v : kStream)
+      if (16 * v.mt == plan->block_m && 16 * v.nt == plan->block_n)
+        return stream_run(epi, g, StreamPlan{&v, splits, steps, (N + 16 * v.nt - 1) / (16 * v.nt)}, workspace,
+                          (hipStream_t)stream);
+  } else if (plan->kernel == PK_PLAN_RING && gemm_vec_ok(g) && ring_shape_ok(N, K, 2)) {
+    for (int i = 0; i < (int)(sizeof kRing / sizeof kRing[0]); ++i) {
+      const int64_t units = (((int64_t)M + 32 * kRing[i].fm - 1) / (32 * kRing[i].fm)) *
+                            (((int64_t)N + 64 * kRing[i].wn - 1) / (64 * kRing[i].wn)) * splits;
+      if (32 * kRing[i].fm == plan->block_m && 64 * kRing[i].wn == plan->block_n && units <= INT32_MAX / 2)
+        return ring_run(epi, g, RingChoice{i, splits, steps, (int)units, 0}, workspace, (hipStream_t)stream);
+    }
+  }
+  set_error("pk_gemm_plan_ex: kernel %d with %d x %d blocks does not take M=%d N=%d K=%d with these operands",
+            plan->kernel, plan->block_m, plan->block_n, M, N, K);
+  return PK_ERR_UNSUPPORTED;
 }
 
 }  // extern "C"

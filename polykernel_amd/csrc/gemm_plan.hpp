@@ -30,13 +30,17 @@ struct RingChoice {
   double us = 0;
 };
 
+// Whether the ring kernel takes the shape (16-byte aligned operands).
+inline bool ring_shape_ok(int N, int K, int weight_bytes) {
+  return N % (16 / weight_bytes) == 0 && K % 8 == 0 && (size_t)K * N * weight_bytes < (size_t(1) << 31) &&
+         (size_t)160 * K * 2 < (size_t(1) << 31);
+}
+
 // Splits use at most `scratch` bytes of fp32 partials.
 inline RingChoice ring_choose(const RingTile *tiles, int ntiles, const RingModel &c, int M, int N, int K,
                               int weight_bytes, size_t scratch) {
   RingChoice best;
-  if (N % (16 / weight_bytes) != 0 || K % 8 != 0 || (size_t)K * N * weight_bytes >= (size_t(1) << 31) ||
-      (size_t)160 * K * 2 >= (size_t(1) << 31))
-    return best;
+  if (!ring_shape_ok(N, K, weight_bytes)) return best;
   const int ktiles = (K + 63) / 64;
   const double bytes = (double)N * K * weight_bytes + 2.0 * ((double)M * K + (double)M * N);
   for (int i = 0; i < ntiles; ++i) {

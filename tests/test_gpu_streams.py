@@ -8,7 +8,7 @@
 * The DMA GEMM addresses A through a buffer descriptor whose 32-bit record
   count covers only the tile's own 256 rows, so A operands of 4 GiB and more
   are read in full (integer inputs: bit-exact against the oracle on rows
-  around the 2^32-byte boundary).
+  around the 2^32-byte boundary); few rows that reach it keep the tile kernel.
 """
 from __future__ import annotations
 
@@ -138,6 +138,32 @@ def test_dma_gemm_a_operand_beyond_4gib(gpu, oracle):
     bad = np.flatnonzero((got != want).any(axis=1))
     assert bad.size == 0, f"rows {rows[bad][:10]} differ"
     del A, C
+    torch.cuda.empty_cache()
+
+
+def test_few_rows_of_a_beyond_4gib(gpu):
+    """32 rows of 2^26 elements: A is exactly 2^32 bytes, which the streaming
+    kernel's 32-bit descriptor would hold as 0.  Integer inputs whose sums fit
+    fp32 exactly, so the float64 product is the oracle."""
+    import torch
+
+    from polykernel_amd import kernels
+
+    M, Kd, N = 32, 1 << 26, 8
+    _say(f"matmul {M}x{N}x{Kd}")
+    gen = torch.Generator(device="cuda").manual_seed(17)
+    A = torch.empty((M, Kd), dtype=torch.bfloat16, device="cuda")
+    B = torch.randint(-1, 2, (Kd, N), device="cuda", generator=gen, dtype=torch.int8).to(torch.bfloat16)
+    want = torch.zeros(M, N, dtype=torch.float64, device="cuda")
+    for k0 in range(0, Kd, 1 << 22):
+        k1 = k0 + (1 << 22)
+        A[:, k0:k1] = torch.randint(-1, 2, (M, 1 << 22), device="cuda", generator=gen, dtype=torch.int8)
+        want += A[:, k0:k1].double() @ B[k0:k1].double()
+    got = kernels.matmul(A, B)
+    torch.cuda.synchronize()
+    assert want.abs().max() < 1 << 24 and want.abs().max() > 0
+    assert torch.equal(got, want.float().to(torch.bfloat16))
+    del A, B
     torch.cuda.empty_cache()
 
 
