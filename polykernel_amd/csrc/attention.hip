@@ -372,6 +372,12 @@ int attention_fa(FaArgs a, int D, int qg, bool built_in, hipStream_t st, const A
 // takes (any S_cache, since rows are read one by one) when every query sees a
 // key.  Key splits while the (b, h) alone leave CUs idle, each keeping a batch
 // per wave.
+// Key splits of the flash kernel's 64 x 128 tile for the same call (128 x 64
+// where only that tile could append).
+int decode_base_splits(const FaArgs &a) {
+  const int bkv = a.Kn && a.S_cache % 128 != 0 && a.S_cache % 64 == 0 ? 64 : 128;
+  return split_count(a.BH, (a.S_kv + bkv - 1) / bkv, 8, 8);
+}
 bool decode_applicable(int S_q, int S_kv, bool causal) {
   return S_q > 0 && S_q <= AD_MAX_Q && S_kv > 0 && (!causal || S_kv >= S_q);
 }
@@ -381,18 +387,17 @@ int attention_decode(FaArgs a, int D, hipStream_t st) {
   a.splits = 1;
   while (a.BH * a.splits < 256 && a.S_kv / (a.splits * 2) >= AD_WAVES * batch && a.splits < 64) a.splits *= 2;
   const size_t rows = (size_t)a.BH * a.S_q;
-  const size_t bytes_o = (size_t)a.splits * rows * D * sizeof(float);
+  const size_t split_bytes = rows * (D + 2) * sizeof(float);
   WorkspaceLease lease;  // held until the merge kernel is queued
   if (a.splits > 1) {
-    const size_t bytes = bytes_o + (size_t)a.splits * rows * 2 * sizeof(float);
-    int rc = library_workspace(0, bytes, st, lease);
+    // a call the flash kernel splits too is refused without workspace for its
+    // splits, as it is there; the others run with the splits that fit
+    const int base = decode_base_splits(a);
+    int rc = library_workspace(base > 1 ? std::min(base, a.splits) * split_bytes : 0, a.splits * split_bytes, st, lease);
     if (rc) return rc;
-    if (lease.bytes >= bytes) {
-      a.part_o = static_cast<float *>(lease.ptr);
-      a.part_ml = reinterpret_cast<float *>(static_cast<char *>(lease.ptr) + bytes_o);
-    } else {
-      a.splits = 1;
-    }
+    while (a.splits > 1 && lease.bytes < a.splits * split_bytes) a.splits /= 2;
+    a.part_o = static_cast<float *>(lease.ptr);
+    a.part_ml = a.part_o + (size_t)a.splits * rows * D;
   }
   if (int rc = grid_ok(a.BH, 1, a.splits, "attention")) return rc;
   const int blocks = a.BH * a.splits;

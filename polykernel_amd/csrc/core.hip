@@ -144,14 +144,6 @@ int gelu_table(const uint16_t **table) {
 }
 
 namespace {
-// Whether memory can't be allocated now because `st` is being captured (or its
-// state can't be told, as on the null stream beside a capturing one).
-bool capturing(void *st) {
-  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(static_cast<hipStream_t>(st), &s) == hipSuccess) return s != hipStreamCaptureStatusNone;
-  (void)hipGetLastError();
-  return true;
-}
 size_t ws_round(size_t bytes) {
   size_t n = size_t(1) << 20;
   while (n < bytes) n <<= 1;
@@ -191,9 +183,19 @@ int library_workspace(size_t need, size_t want, void *st, WorkspaceLease &lease)
     slot->bytes = ws_round(bytes);
     return e;
   };
-  // beyond `need` only where it can be had: not during a capture, not when memory is short
-  if (want > need && slot->bytes < want && !capturing(st) && grow(want) != hipSuccess) (void)hipGetLastError();
-  if (slot->bytes < need) PK_HIP(grow(need));
+  if (slot->bytes < need) {
+    if (want > need && grow(want) != hipSuccess) (void)hipGetLastError();
+    if (slot->bytes < need) PK_HIP(grow(need));
+  } else if (slot->bytes < want) {
+    // A call that could do without: allocated in the relaxed capture mode, so
+    // that a capture on this or another stream goes on (the stricter modes
+    // invalidate it, and the same call in a captured graph would keep fewer
+    // splits on every replay).
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool set = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    if (!set || grow(want) != hipSuccess) (void)hipGetLastError();
+    if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
   lease.bytes = slot->bytes;
   lease.ptr = slot->ptr;
   lease.keep = slot;

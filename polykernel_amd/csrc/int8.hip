@@ -618,13 +618,12 @@ int int8_run(int epi, const uint16_t *A, const int8_t *W, const float *scale, ui
   }
   I8sPlan plan;
   if (!cfg && aligned16(A) && aligned16(W) && aligned16(scale) && aligned16(C) && (epi != I8_RESID || aligned16(R))) {
-    // a caller's scratch is refused where the column-split or generic kernel's splits would not fit it
-    if (ws) {
-      if (int rc = check_workspace(i8s_plan(M, N, K, nullptr, device_cus(), plan) ? i8s_workspace(plan, M, N)
-                                                                                  : generic_workspace(M, N, K, nullptr),
-                                   ws_bytes))
-        return rc;
-    }
+    // scratch is refused where the column-split or generic kernel's splits would not fit it
+    auto base = [&] {
+      return i8s_plan(M, N, K, nullptr, device_cus(), plan) ? i8s_workspace(plan, M, N) : generic_workspace(M, N, K, nullptr);
+    };
+    if (ws)
+      if (int rc = check_workspace(base(), ws_bytes)) return rc;
     // a caller's scratch as it is (launch_matmul_int8_noalloc's static buffer
     // is the cap for all, so that calls with and without it split alike),
     // library scratch as far as it can be had
@@ -638,10 +637,10 @@ int int8_run(int epi, const uint16_t *A, const int8_t *W, const float *scale, ui
     const size_t part = choose(ws ? (aligned16(ws) ? ws_bytes : 0) : kInt8ScratchBytes);
     float *partial = static_cast<float *>(ws);
     if (part && !ws) {
-      int rc = library_workspace(0, part, st, lease);
+      int rc = library_workspace(std::min(base(), part), part, st, lease);
       if (rc) return rc;
       partial = static_cast<float *>(lease.ptr);
-      if (lease.bytes < part) choose(0);
+      if (lease.bytes < part) choose(lease.bytes);
     }
     const KsPlan &ks = p.ks;
     const RingChoice &ring = p.ring;

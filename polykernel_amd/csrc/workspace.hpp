@@ -34,8 +34,9 @@ struct WorkspaceLease {
 // stream).  Returns a PK_* status.
 int library_workspace(size_t bytes, void *stream, WorkspaceLease &lease);
 // The same for a caller that works with `need` bytes and better with `want`:
-// the buffer grows to `want` unless the stream is being captured or memory is
-// short (lease.bytes tells), and is refused only where `need` would be.
+// the buffer grows to `want` unless memory is short (lease.bytes tells), also
+// while a stream is captured, and is refused only where `need` would be (a
+// buffer short of `need` on a captured stream, for one).
 int library_workspace(size_t need, size_t want, void *stream, WorkspaceLease &lease);
 
 // RMSNorm -> MatMul outside the panel kernel, for its launchers: the workspace

@@ -324,3 +324,132 @@ def test_mlp_block_and_decode_chain_in_replayed_graphs(gpu):
             assert torch.equal(o.view(torch.int16), eager.view(torch.int16)), (name, rep)
             assert launch(eager, st()) == 0  # eager work between replays
             torch.cuda.synchronize()
+
+
+class _Capture:
+    """A capture in the strictest mode (global) on one stream, ended by end():
+    True if it went through."""
+
+    def __init__(self, stream):
+        import ctypes
+
+        self.hip, self.st, self.C = ctypes.CDLL("libamdhip64.so"), ctypes.c_void_p(stream.cuda_stream), ctypes
+        assert self.hip.hipStreamBeginCapture(self.st, 0) == 0
+
+    def end(self):
+        graph = self.C.c_void_p()
+        rc = self.hip.hipStreamEndCapture(self.st, self.C.byref(graph))
+        self.hip.hipGetLastError()
+        if graph.value:
+            self.hip.hipGraphDestroy(graph)
+        return rc == 0
+
+
+def _decode_case(Skv, seed=90, H=8, D=128):
+    return [to_dev(rng_bf16((1, H, n, D), seed + i)) for i, n in enumerate((1, Skv, Skv))]
+
+
+def test_optional_workspace_leaves_captures_alone(gpu):
+    """A call whose split partials are optional, first made on a stream while
+    another stream is being captured: the capture goes on, and the call gives
+    the bits of a later one."""
+    import torch
+
+    from polykernel_amd import kernels
+
+    lib = _lib_loaded()
+    q, k, v = _decode_case(1024)  # 8 heads: split over workgroups; the flash kernel would not
+    want = kernels.attention_prefill(q, k, v)
+    out = torch.empty_like(want)
+    torch.cuda.synchronize()
+    captured, eager = torch.cuda.Stream(), torch.cuda.Stream()
+    x = to_dev(rng_bf16((8, 512), 95))
+    y = torch.empty_like(x)
+    cap = _Capture(captured)
+    rc = [lib.launch_rmsnorm(x.data_ptr(), None, y.data_ptr(), 8, 512, 1e-6, captured.cuda_stream)]
+    rc.append(lib.launch_attention_prefill(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), 1, 8, 1, 1024, 128,
+                                           1 / np.sqrt(128), 1, eager.cuda_stream))
+    rc.append(lib.launch_rmsnorm(x.data_ptr(), None, y.data_ptr(), 8, 512, 1e-6, captured.cuda_stream))
+    ended = cap.end()
+    eager.synchronize()
+    assert rc == [0, 0, 0] and ended
+    assert torch.equal(out, want)
+
+
+def test_required_workspace_refused_under_capture(gpu):
+    """A call that has always needed split partials is refused, not run without
+    them, where a captured stream has no workspace yet.  (Each capture is of a
+    thread and a stream of its own: the refusal leaves it invalid.)"""
+    import ctypes
+
+    import torch
+
+    from polykernel_amd import _lib, kernels
+
+    lib = _lib_loaded()
+    hip = ctypes.CDLL("libamdhip64.so")
+    q, k, v = _decode_case(4096)  # the flash kernel splits these keys too
+    a, wq, s = _int8_case(96)
+    want = (kernels.attention_prefill(q, k, v), kernels.matmul_int8(a, wq, s))
+    outs = [torch.full_like(w, 7.0) for w in want]
+    torch.cuda.synchronize()
+    calls = (lambda sp: lib.launch_attention_prefill(q.data_ptr(), k.data_ptr(), v.data_ptr(), outs[0].data_ptr(), 1, 8,
+                                                     1, 4096, 128, 1 / np.sqrt(128), 1, sp),
+             lambda sp: lib.launch_matmul_int8(a.data_ptr(), wq.data_ptr(), s.data_ptr(), outs[1].data_ptr(), 16, 4096,
+                                               8192, sp))
+    rcs = []
+
+    def refused(call):
+        st = ctypes.c_void_p()
+        if hip.hipStreamCreate(ctypes.byref(st)) or hip.hipStreamBeginCapture(st, 1):  # 1: this thread only
+            return
+        rcs.append(call(st))
+        graph = ctypes.c_void_p()
+        hip.hipStreamEndCapture(st, ctypes.byref(graph))
+        hip.hipGetLastError()
+
+    for call in calls:
+        t = threading.Thread(target=refused, args=(call,))
+        t.start(), t.join(60)
+    assert rcs == [_lib.PK_ERR_HIP] * 2, rcs
+    assert all(bool((o == 7.0).all()) for o in outs)
+    st = torch.cuda.Stream()
+    for call, out, w in zip(calls, outs, want):
+        assert call(st.cuda_stream) == 0
+        st.synchronize()
+        assert torch.equal(out, w)
+
+
+def test_graph_captured_with_rows_only_gives_the_eager_bits(gpu):
+    """RMSNorm -> MatMul captured on a stream whose workspace holds the
+    normalised rows but no split partials yet: every replay gives the bits of
+    an eager call."""
+    import torch
+
+    from polykernel_amd import kernels, synth
+
+    M, N, Kd = 64, 768, 3072
+    x = to_dev(synth.normal_bf16((M, Kd), 97))
+    g = to_dev(synth.normal_bf16((Kd,), 98, 0.1, 1.0))
+    w = to_dev(synth.normal_bf16((Kd, N), 99, 1 / np.sqrt(Kd)))
+    want = kernels.fused_rmsnorm_matmul(x, w, g, 1e-6)
+    wide = to_dev(synth.normal_bf16((Kd, 40960), 100, 1 / np.sqrt(Kd)))  # fills the chip: no K split
+    st = torch.cuda.Stream()
+    with torch.cuda.stream(st):
+        kernels.fused_rmsnorm_matmul(x, wide, g, 1e-6)
+        torch.cuda.synchronize()
+        gr = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(gr, stream=st):
+            out = kernels.fused_rmsnorm_matmul(x, w, g, 1e-6)
+    for _ in range(3):
+        out.fill_(0)
+        gr.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert torch.equal(kernels.fused_rmsnorm_matmul(x, w, g, 1e-6), want)
+
+
+def _lib_loaded():
+    from polykernel_amd import _lib
+
+    return _lib.load()
