@@ -292,6 +292,12 @@ PK_API int pk_gemm_plan_ex(int epi, const uint16_t *A, const uint16_t *B, uint16
                            const uint16_t *bias, const uint16_t *R, int M, int N, int K,
                            const pk_plan *plan, void *workspace, size_t workspace_bytes, void *stream);
 
+/* The same for the int8 product (epilogues as pk_matmul_int8_ex). */
+PK_API int pk_int8_plan(int M, int N, int K, size_t scratch_bytes, pk_plan *out);
+PK_API int pk_int8_plan_ex(int epi, const uint16_t *A, const int8_t *Wq, const float *scale,
+                           uint16_t *C, const uint16_t *R, int M, int N, int K, const pk_plan *plan,
+                           void *workspace, size_t workspace_bytes, void *stream);
+
 /* launch_fused_kv_append_attention with an explicit configuration (one of
  * pk_op_configs("fused_kv_append_attention", S_q, S_cache + S_q, D); NULL =
  * built-in choice).  A flash configuration the operands do not allow

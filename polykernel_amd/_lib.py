@@ -101,6 +101,8 @@ SIGNATURES = {
     "pk_gemm_config_ex": (I, [I, P, P, P, P, P, I, I, I, C.POINTER(Config), P]),
     "pk_gemm_plan": (I, [I, I, I, I, SZ, C.POINTER(Plan)]),
     "pk_gemm_plan_ex": (I, [I, P, P, P, P, P, I, I, I, C.POINTER(Plan), P, SZ, P]),
+    "pk_int8_plan": (I, [I, I, I, SZ, C.POINTER(Plan)]),
+    "pk_int8_plan_ex": (I, [I, P, P, P, P, P, I, I, I, C.POINTER(Plan), P, SZ, P]),
     "pk_op_configs": (I, [C.c_char_p, LL, LL, LL, C.POINTER(Config), I]),
     "pk_op_default_config": (I, [C.c_char_p, LL, LL, LL, C.POINTER(Config)]),
     "pk_naive_matmul": (I, [I, P, P, P, P, P, I, I, I, P]),

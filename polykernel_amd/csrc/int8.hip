@@ -608,6 +608,25 @@ static int reduce_run(int epi, const Int8Args &g, hipStream_t st) {
   return PK_OK;
 }
 
+// One product by a K-split stream or ring plan (16-byte aligned operands).
+static int int8_plan_run(int epi, const uint16_t *A, const int8_t *W, const float *scale, uint16_t *C, const uint16_t *R,
+                         const uint16_t *tab, int M, int N, int K, const Int8Plan &p, float *partial, hipStream_t st) {
+  const KsPlan &ks = p.ks;
+  const RingChoice &ring = p.ring;
+  const int splits = ks.v ? ks.splits : ring.splits;
+  if (ks.v) {
+    const int units = ks.slices * ks.splits;
+    const I8sArgs a{A, W, scale, partial, C, R, tab, M, N, K, ks.splits, ks.split_steps, units};
+    ks.v->fn[epi](dim3(units, (M + 16 * ks.v->mt - 1) / (16 * ks.v->mt)), st, a);
+    PK_LAUNCH_CHECK("int8_kstream_kernel");
+  } else {
+    const gk::GemmRingArgs a{{A, nullptr, C, nullptr, R, tab, M, N, K}, partial, ring.splits, ring.split_tiles, W, scale};
+    kI8RingFn[ring.tile][epi](dim3(ring.units), st, a);
+    PK_LAUNCH_CHECK("int8_ring_kernel");
+  }
+  return splits > 1 ? reduce_run(epi, Int8Args{A, W, scale, partial, C, R, tab, M, N, K, splits, 0}, st) : PK_OK;
+}
+
 int int8_run(int epi, const uint16_t *A, const int8_t *W, const float *scale, uint16_t *C,
              const uint16_t *R, int M, int N, int K, const pk_config *cfg, void *ws,
              size_t ws_bytes, hipStream_t st) {
@@ -642,21 +661,7 @@ int int8_run(int epi, const uint16_t *A, const int8_t *W, const float *scale, ui
       partial = static_cast<float *>(lease.ptr);
       if (lease.bytes < part) choose(lease.bytes);
     }
-    const KsPlan &ks = p.ks;
-    const RingChoice &ring = p.ring;
-    if (ks.v) {
-      const int units = ks.slices * ks.splits;
-      const I8sArgs a{A, W, scale, partial, C, R, tab, M, N, K, ks.splits, ks.split_steps, units};
-      ks.v->fn[epi](dim3(units, (M + 16 * ks.v->mt - 1) / (16 * ks.v->mt)), st, a);
-      PK_LAUNCH_CHECK("int8_kstream_kernel");
-      return ks.splits > 1 ? reduce_run(epi, Int8Args{A, W, scale, partial, C, R, tab, M, N, K, ks.splits, 0}, st) : PK_OK;
-    }
-    if (ring.tile >= 0) {
-      const gk::GemmRingArgs a{{A, nullptr, C, nullptr, R, tab, M, N, K}, partial, ring.splits, ring.split_tiles, W, scale};
-      kI8RingFn[ring.tile][epi](dim3(ring.units), st, a);
-      PK_LAUNCH_CHECK("int8_ring_kernel");
-      return ring.splits > 1 ? reduce_run(epi, Int8Args{A, W, scale, partial, C, R, tab, M, N, K, ring.splits, 0}, st) : PK_OK;
-    }
+    if (p.ks.v || p.ring.tile >= 0) return int8_plan_run(epi, A, W, scale, C, R, tab, M, N, K, p, partial, st);
   }
   const bool fast = aligned16(A) && aligned16(W) && aligned16(scale) && aligned16(C) &&
                     (epi != I8_RESID || aligned16(R)) && i8s_plan(M, N, K, cfg, device_cus(), plan);
@@ -791,6 +796,54 @@ int pk_matmul_int8_ex(int epi, const uint16_t *A, const int8_t *Wq, const float 
   PK_CHECK_ARG(M >= 0 && N >= 0 && K > 0, "pk_matmul_int8_ex: invalid shape M=%d N=%d K=%d", M, N, K);
   if (M == 0 || N == 0) return PK_OK;
   return int8_run(epi, A, Wq, scale, C, R, M, N, K, cfg, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+int pk_int8_plan(int M, int N, int K, size_t scratch_bytes, pk_plan *out) {
+  PK_CHECK_ARG(out && M > 0 && N > 0 && K > 0, "pk_int8_plan: invalid argument");
+  const Int8Plan p = int8_plan(M, N, K, std::min(scratch_bytes, kInt8ScratchBytes));
+  *out = pk_plan{PK_PLAN_TILE, 0, 0, 1, 0};
+  if (p.ks.v) *out = pk_plan{PK_PLAN_STREAM, 16 * p.ks.v->mt, 16 * p.ks.v->nt, p.ks.splits, p.ks.split_steps};
+  else if (p.ring.tile >= 0)
+    *out = pk_plan{PK_PLAN_RING, 32 * kI8Ring[p.ring.tile].fm, 64 * kI8Ring[p.ring.tile].wn, p.ring.splits, p.ring.split_tiles};
+  return PK_OK;
+}
+
+int pk_int8_plan_ex(int epi, const uint16_t *A, const int8_t *Wq, const float *scale, uint16_t *C, const uint16_t *R,
+                    int M, int N, int K, const pk_plan *plan, void *workspace, size_t workspace_bytes, void *stream) {
+  PK_CHECK_ARG(epi >= I8_NONE && epi <= I8_RESID, "pk_int8_plan_ex: epilogue %d not in 0..2", epi);
+  PK_CHECK_ARG(A && Wq && scale && C && plan && (epi != I8_RESID || R), "pk_int8_plan_ex: null pointer");
+  PK_CHECK_ARG(M > 0 && N > 0 && K > 0 && plan->splits >= 1, "pk_int8_plan_ex: invalid shape or plan");
+  const uint16_t *tab = nullptr;
+  if (epi == I8_GELU)
+    if (int rc = gelu_table(&tab)) return rc;
+  const int ksteps = (K + 63) / 64;  // of both kernels
+  const int steps = (ksteps + plan->splits - 1) / plan->splits, splits = (ksteps + steps - 1) / steps;
+  const size_t part = splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
+  if (part && (workspace_bytes < part || !aligned16(workspace))) {
+    set_error("pk_int8_plan_ex: %zu aligned bytes of workspace required, got %zu", part, workspace_bytes);
+    return PK_ERR_WORKSPACE;
+  }
+  Int8Plan p;
+  if (aligned16(A) && aligned16(Wq) && aligned16(scale) && aligned16(C) && (epi != I8_RESID || aligned16(R)) &&
+      ring_shape_ok(N, K, 1)) {
+    if (plan->kernel == PK_PLAN_STREAM) {
+      for (const KsVariant &v : kI8k)
+        if (16 * v.mt == plan->block_m && 16 * v.nt == plan->block_n)
+          p.ks = KsPlan{&v, splits, steps, (N + 16 * v.nt - 1) / (16 * v.nt)};
+    } else if (plan->kernel == PK_PLAN_RING) {
+      for (int i = 0; i < (int)(sizeof kI8Ring / sizeof kI8Ring[0]); ++i) {
+        const int64_t units = (((int64_t)M + 32 * kI8Ring[i].fm - 1) / (32 * kI8Ring[i].fm)) *
+                              (((int64_t)N + 64 * kI8Ring[i].wn - 1) / (64 * kI8Ring[i].wn)) * splits;
+        if (32 * kI8Ring[i].fm == plan->block_m && 64 * kI8Ring[i].wn == plan->block_n && units <= INT32_MAX / 2)
+          p.ring = RingChoice{i, splits, steps, (int)units, 0};
+      }
+    }
+  }
+  if (p.ks.v || p.ring.tile >= 0)
+    return int8_plan_run(epi, A, Wq, scale, C, R, tab, M, N, K, p, static_cast<float *>(workspace), (hipStream_t)stream);
+  set_error("pk_int8_plan_ex: kernel %d with %d x %d blocks does not take M=%d N=%d K=%d with these operands",
+            plan->kernel, plan->block_m, plan->block_n, M, N, K);
+  return PK_ERR_UNSUPPORTED;
 }
 
 size_t pk_decode_mlp_int8_workspace_size(int M, int d, int F) {
