@@ -279,14 +279,18 @@ int stream_run(int epi, const GemmArgs &g, const StreamPlan &p, void *scratch, h
 // Against the 64 x 64 tiles with element loads (us, rotating weights): [1, 50257,
 // 2048] 251 / 45.5, [64, 50257, 4096] 580 / 115, [16, 12001, 4096] 261 / 27.6, [8,
 // 5003, 2048] 99 / 9.1, [64, 2101, 512] 26.1 / 12.4.  Wide slices share fewer
-// lines at their edges and are taken where they still fill the chip.
+// lines at their edges and are taken where they still fill the chip and K has
+// more than a k-step or two ([22, 20770, 8] 4.9 us on tiles, 6.6 wide, 5 narrow);
+// above 32 rows such a K leaves mostly the stores of single outputs, at which the
+// tiles are faster ([51, 25172, 8] 5.9 / 9.7, [43, 59653, 16] 11.9 / 16.8).
 bool odd_ok(const GemmArgs &g) {
-  return g.M <= kStreamRows && g.K % 8 == 0 && g.N >= 8 && aligned16(g.A) && (size_t)g.K * g.N * 2 < (size_t(1) << 31);
+  return g.M <= kStreamRows && g.K % 8 == 0 && g.N >= 8 && aligned16(g.A) && (size_t)g.K * g.N * 2 < (size_t(1) << 31) &&
+         (g.M <= 32 || g.N <= 64 * 128 || g.K >= 64);
 }
 template <int MT>
 int odd_run(const GemmArgs &g, hipStream_t st) {
-  if (g.N >= 128 * 160) gemm_odd_kernel<8, MT, 4, 3><<<(g.N + 127) / 128, 256, 0, st>>>(g);
-  else if (g.N >= 64 * 128) gemm_odd_kernel<4, MT, 8, 4><<<(g.N + 63) / 64, 512, 0, st>>>(g);
+  if (g.N >= 128 * 160 && g.K >= 64) gemm_odd_kernel<8, MT, 4, 3><<<(g.N + 127) / 128, 256, 0, st>>>(g);
+  else if (g.N >= 64 * 128 && g.K >= 64) gemm_odd_kernel<4, MT, 8, 4><<<(g.N + 63) / 64, 512, 0, st>>>(g);
   else gemm_odd_kernel<2, MT, 8, 5><<<(g.N + 31) / 32, 512, 0, st>>>(g);
   PK_LAUNCH_CHECK("gemm_odd_kernel");
   return PK_OK;
@@ -310,6 +314,7 @@ const RingTile kRing[] = {{2, 2, 0.27}, {3, 2, 0.375}, {4, 2, 0.44}, {3, 4, 0.67
 const RingLaunch kRingFn[][4] = {PK_GR(2, 2, 4), PK_GR(3, 2, 4), PK_GR(4, 2, 4),
                                  PK_GR(3, 4, 3), PK_GR(4, 4, 3), PK_GR(5, 4, 3)};
 #undef PK_GR
+constexpr int kRingWide = 3;  // 96 x 256
 
 // Fitted to 60 shapes of 65-3850 rows, N 512-16384 and K 512-16384: its choice
 // is within 0.7 % of the best variant in the geometric mean, 10 % at worst.
@@ -332,38 +337,6 @@ int ring_run(int epi, const GemmArgs &g, const RingChoice &p, void *scratch, hip
   return p.splits > 1 ? reduce_run(epi, g, a.partial, p.splits, st) : PK_OK;
 }
 
-// The kernel of the built-in choice for vector-aligned operands and at most
-// `scratch` bytes of partials: the streaming kernel up to kStreamRows rows,
-// above it the ring kernel or, where its model is no slower, the 256 x 256 one
-// (`dma`: it takes these operands).  Neither plan set: the tiles of pick_tile.
-struct GemmPlan {
-  StreamPlan stream;
-  RingChoice ring;
-  size_t part(int M, int N) const {
-    const int s = stream.v ? stream.splits : ring.tile >= 0 ? ring.splits : 1;
-    return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
-  }
-};
-GemmPlan gemm_plan(int M, int N, int K, bool dma, size_t scratch) {
-  static thread_local PlanMemo<GemmPlan> memo;
-  return memo.get(M, N, K, scratch, dma, [&] {
-    GemmPlan p;
-    if (M <= kStreamRows && stream_plan(M, N, K, scratch, p.stream)) return p;
-    p.ring = ring_plan(M, N, K, scratch);
-    if (dma && dma_us(M, N, K) <= p.ring.us) p.ring = RingChoice{};
-    return p;
-  });
-}
-
-// Bytes of split partials the built-in choice wants for aligned operands (0:
-// none); a caller with less scratch gets the best choice within it.
-constexpr size_t kGemmScratchMax = size_t(64) << 20;
-size_t gemm_scratch_bytes(int M, int N, int K) {
-  constexpr int most = INT32_MAX - 1023;  // as tile_grid_ok
-  if (M <= 0 || N <= 0 || K <= 0 || M > most || N > most || K > most) return 0;
-  return gemm_plan(M, N, K, gemm_dma_shape_ok(N, K), kGemmScratchMax).part(M, N);
-}
-
 // Largest tile that still gives at least ~one workgroup per CU.
 // With the direct-to-LDS kernel (`dma`), 256x256 from 72 tiles up: even one
 // round that leaves most CUs idle beats the 128x128 kernel's rounds (K 4096:
@@ -379,6 +352,99 @@ int pick_tile(int M, int N, bool dma) {
   if (t256 >= (dma ? 72 : 200)) return 0;
   if (t128 >= 200) return 1;
   return 2;
+}
+
+// Whether the ring plan is faster than the tile of pick_tile (`tile`; `dma`: tile
+// 0 is the direct-to-LDS kernel).  All figures without and with K split alike, us
+// in a replayed graph, tile / ring.
+//
+// Against the 256 x 256 direct-to-LDS kernel: the two time models, and for GELU
+// what the epilogues take in each round -- 1.5 us per 10 000 outputs of the ring's
+// tile, which finishes them 32 rows at a time, 3 us and 1 per further round of the
+// other ([4000, 2304, 256] 20.3 / 22.7, [10000, 4096, 512] 76.6 / 98.8 with GELU,
+// 16.4 / 14.6 and 65.6 / 71.5 without; with these terms the choice is within
+// 0.2 % of the better one over 366 shapes, 4.4 % without).
+// Against the register-staged 64 x 64 kernel: it starts at 2.9 us (4.7 with GELU)
+// and takes 0.42 per 64-deep k-step, one tile of the ring 4.4 (6.1) and 0.24: a
+// deep ring to fill, waves' tiles to add.  So the ring needs some k: [300, 1024,
+// K 128] 4.0 / 5.0, 256 4.8 / 5.5, 384 6.5 / 6.3, 512 7.0 / 6.8; with an epilogue
+// that reads more, on a filled chip, less ([700, 4096, 128] + bias and residual
+// 9.9 / 8.9), and where the columns fill a fraction of its tile, whose lanes then
+// finish rows alone, more ([1555, 16, 512] + GELU 7.7 / 9.7).
+// Against the register-staged 128 and 256 tiles it wins unless K is tiny and the
+// epilogue empty ([4000, 1024, 64] 4.2 / 4.5, [4000, 16384, 8] 45.9 / 55).
+bool ring_pays(int epi, int M, int N, int K, int tile, bool dma, const RingChoice &p) {
+  if (tile == 0 && dma) {
+    double ring = p.us, direct = dma_us(M, N, K);
+    if (epi == EPI_BIAS_GELU) {
+      const RingTile &t = kRing[p.tile];
+      ring += std::ceil(p.units / 256.0) * 1.5e-4 * (32 * t.fm) * (64 * t.wn);
+      direct += 2.0 + std::ceil((((int64_t)M + 255) / 256) * (((int64_t)N + 255) / 256) / 256.0);
+    }
+    return ring < direct;
+  }
+  if (tile == 2) {
+    const int64_t units = (((int64_t)M + 63) / 64) * (((int64_t)N + 63) / 64);
+    if (epi == EPI_NONE) return K >= (units <= 32 ? 448 : 352);
+    if (epi == EPI_BIAS_GELU)
+      return K >= (N <= 32 ? (units <= 32 ? 704 : 448) : units <= 64 ? 352 : units <= 256 ? 256 : 136);
+    return K >= (N <= 32 ? (units <= 32 ? 512 : 384) : units <= 32 ? 320 : units <= 256 ? 224 : 136);
+  }
+  if (epi != EPI_NONE || K > 64) return true;
+  return tile == 1 ? (((int64_t)M + 127) / 128) * (((int64_t)N + 127) / 128) > 496 : (int64_t)M * N < 24000000;
+}
+
+// Up to kStreamRows rows: whether the streaming kernel is faster than the 64 x 64
+// tile, where pick_tile has that one.  It is, but for 33-64 rows on a second round
+// of 64-column slices over a short K, whose wide slices leave half the waves
+// ([64, 16448, 64] + bias and residual 6.0 / 7.2 us tile / stream, [64, 20000, 16] 3.9 / 4.5).
+bool stream_pays(int epi, int M, int N, int K, int tile) {
+  return M <= 32 || N <= 16384 || tile != 2 || K > (epi == EPI_NONE ? 256 : 512);
+}
+// 33-64 rows and more than 256 slices of 128 columns, a vocabulary head say: a
+// second round of slices that no CU shares evenly streams at 3.5-4.2 TB/s, one
+// round of the ring's 96 x 256 tiles at 4.6-4.9 ([64, 42496, 4544] 117 -> 78.7 us, 97
+// on 256 x 256 tiles; [40, 50256, 2560] 56.9 -> 48.0).
+bool ring_streams(int M, int N, int K) {
+  return M > 32 && N > 32768 && N <= 65536 && K >= 2048 && ring_shape_ok(N, K, 2);
+}
+
+// The kernel of the built-in choice for vector-aligned operands and at most
+// `scratch` bytes of partials: the streaming kernel up to kStreamRows rows,
+// above it the ring kernel where it pays, else `tile` (`dma`: the 256 x 256
+// direct-to-LDS kernel takes these operands).
+struct GemmPlan {
+  StreamPlan stream;
+  RingChoice ring;
+  int tile = 0;
+  size_t part(int M, int N) const {
+    const int s = stream.v ? stream.splits : ring.tile >= 0 ? ring.splits : 1;
+    return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
+  }
+};
+GemmPlan gemm_plan(int epi, int M, int N, int K, bool dma, size_t scratch) {
+  static thread_local PlanMemo<GemmPlan> memo;
+  return memo.get(M, N, K, scratch, epi << 1 | dma, [&] {
+    GemmPlan p;
+    p.tile = pick_tile(M, N, dma);
+    if (M <= kStreamRows && ring_streams(M, N, K)) {
+      p.ring = RingChoice{kRingWide, 1, (K + GR_BK - 1) / GR_BK, (N + 255) / 256, 0};
+      return p;
+    }
+    if (M <= kStreamRows && stream_pays(epi, M, N, K, p.tile) && stream_plan(M, N, K, scratch, p.stream)) return p;
+    p.ring = ring_plan(M, N, K, scratch);
+    if (p.ring.tile >= 0 && !ring_pays(epi, M, N, K, p.tile, dma, p.ring)) p.ring = RingChoice{};
+    return p;
+  });
+}
+
+// Bytes of split partials the built-in choice wants for aligned operands (0:
+// none); a caller with less scratch gets the best choice within it.
+constexpr size_t kGemmScratchMax = size_t(64) << 20;
+size_t gemm_scratch_bytes(int epi, int M, int N, int K) {
+  constexpr int most = INT32_MAX - 1023;  // as tile_grid_ok
+  if (M <= 0 || N <= 0 || K <= 0 || M > most || N > most || K > most) return 0;
+  return gemm_plan(epi, M, N, K, gemm_dma_shape_ok(N, K), kGemmScratchMax).part(M, N);
 }
 
 }  // namespace
@@ -464,12 +530,14 @@ int gemm_run(int epi, const uint16_t *A, const uint16_t *B, uint16_t *C, const u
     if (rc) return rc;
   }
   if (tile < 0 && gemm_vec_ok(g)) {
-    const GemmPlan p = gemm_plan(M, N, K, gemm_dma_fits(g), aligned16(scratch) ? std::min(scratch_bytes, kGemmScratchMax) : 0);
+    const GemmPlan p =
+        gemm_plan(epi, M, N, K, gemm_dma_fits(g), aligned16(scratch) ? std::min(scratch_bytes, kGemmScratchMax) : 0);
     if (p.stream.v) return stream_run(epi, g, p.stream, scratch, st);
     if (p.ring.tile >= 0) return ring_run(epi, g, p.ring, scratch, st);
+    tile = p.tile;
   }
-  if (tile < 0 && epi == EPI_NONE && !gemm_vec_ok(g) && odd_ok(g)) return odd_run(g, st);
-  if (tile < 0) tile = gemm_dma_fits(g) ? 0 : pick_tile(M, N, false);
+  if (tile < 0 && epi == EPI_NONE && odd_ok(g)) return odd_run(g, st);
+  if (tile < 0) tile = pick_tile(M, N, false);
   switch (epi) {
     case EPI_NONE: return gemm_dispatch<EPI_NONE>(g, tile, st);
     case EPI_BIAS_GELU: return gemm_dispatch<EPI_BIAS_GELU>(g, tile, st);
@@ -517,7 +585,7 @@ bool rmsnorm_matmul_config(int M, int N, int K, pk_config *out) {
 // (*part: their bytes, 0 if not).
 int normed_rows_workspace(int M, int N, int K, void *st, WorkspaceLease &lease, void **scratch, size_t *part) {
   const size_t row_bytes = ((size_t)M * K * 2 + 255) & ~size_t(255);
-  *part = gemm_scratch_bytes(M, N, K);
+  *part = gemm_scratch_bytes(EPI_NONE, M, N, K);
   int rc = library_workspace((size_t)M * K * 2, *part ? row_bytes + *part : (size_t)M * K * 2, st, lease);
   if (rc) return rc;
   *scratch = static_cast<char *>(lease.ptr) + row_bytes;
@@ -530,7 +598,7 @@ int gemm_planned(const uint16_t *A, const uint16_t *B, uint16_t *C, int M, int N
   const GemmArgs g{A, B, C, nullptr, nullptr, nullptr, M, N, K};
   *ran = false;
   if (gemm_vec_ok(g)) {
-    const GemmPlan p = gemm_plan(M, N, K, gemm_dma_fits(g), std::min(scratch_bytes, kGemmScratchMax));
+    const GemmPlan p = gemm_plan(EPI_NONE, M, N, K, gemm_dma_fits(g), std::min(scratch_bytes, kGemmScratchMax));
     if (!p.stream.v && p.ring.tile < 0) return PK_OK;
   } else if (!odd_ok(g)) {
     return PK_OK;
@@ -621,7 +689,7 @@ static size_t mlp_rows_bytes(int M, int d, int F) {
 
 size_t pk_mlp_block_workspace_size(int M, int d, int F) {
   if (M <= 0 || d <= 0 || F <= 0) return 0;  // no launch takes a workspace
-  return mlp_rows_bytes(M, d, F) + std::max(gemm_scratch_bytes(M, F, d), gemm_scratch_bytes(M, d, F));
+  return mlp_rows_bytes(M, d, F) + std::max(gemm_scratch_bytes(EPI_BIAS_GELU, M, F, d), gemm_scratch_bytes(EPI_BIAS_RESID, M, d, F));
 }
 
 int launch_mlp_block(const uint16_t *x, const uint16_t *gamma, const uint16_t *W1,
@@ -677,7 +745,8 @@ int pk_gemm_plan(int epi, int M, int N, int K, size_t scratch_bytes, pk_plan *ou
   *out = pk_plan{};
   out->splits = 1;
   if (K % 8 == 0 && N % 8 == 0) {
-    const GemmPlan p = gemm_plan(M, N, K, gemm_dma_shape_ok(N, K), std::min(scratch_bytes, kGemmScratchMax));
+    const GemmPlan p = gemm_plan(epi, M, N, K, gemm_dma_shape_ok(N, K), std::min(scratch_bytes, kGemmScratchMax));
+    out->block_m = out->block_n = p.tile == 0 ? 256 : p.tile == 1 ? 128 : 64;
     if (p.stream.v) {
       *out = pk_plan{PK_PLAN_STREAM, 16 * p.stream.v->mt, 16 * p.stream.v->nt, p.stream.splits, p.stream.split_steps};
       return PK_OK;
@@ -687,12 +756,12 @@ int pk_gemm_plan(int epi, int M, int N, int K, size_t scratch_bytes, pk_plan *ou
       *out = pk_plan{PK_PLAN_RING, 32 * t.fm, 64 * t.wn, p.ring.splits, p.ring.split_tiles};
       return PK_OK;
     }
-  } else if (epi == EPI_NONE && odd_ok(GemmArgs{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K})) {
-    out->kernel = PK_PLAN_ODD;
     return PK_OK;
   }
-  const int tile = K % 8 == 0 && N % 8 == 0 && gemm_dma_shape_ok(N, K) ? 0 : pick_tile(M, N, false);
+  const int tile = pick_tile(M, N, false);
   out->block_m = out->block_n = tile == 0 ? 256 : tile == 1 ? 128 : 64;
+  if (epi == EPI_NONE && odd_ok(GemmArgs{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K}))
+    *out = pk_plan{PK_PLAN_ODD, 0, 0, 1, 0};
   return PK_OK;
 }
 

@@ -1,6 +1,7 @@
-"""GEMMs of decode and prompt size (the weight-streaming and the ring kernel):
-every slice width, tile, row block and epilogue at ragged edges, with and
-without K splits."""
+"""GEMMs of decode and prompt size through the entry points' own choice of
+kernel, at ragged edges, with every epilogue, with and without K splits.  (Each
+variant of the streaming and ring kernels by name, over several rounds of its
+ring: test_gpu_plan_variants.py.)"""
 from __future__ import annotations
 
 import ctypes
@@ -25,9 +26,9 @@ def test_small_m_gemm_integer_bit_exact(gpu, oracle, M, N, Kd):
     _check_integer(oracle, M, N, Kd)
 
 
-# the ring kernel's six tiles (64 x 128 ... 160 x 256), one row over a tile,
-# K below, at and above a k-tile of 64 with tails of 8 to 56, one and several
-# rounds of a ring slot
+# above 64 rows: one row over a tile of 64 to 160 rows, K below, at and above a
+# k-tile of 64 with tails of 8 to 56 (the tile kernels for a short K, the ring
+# kernel for a long one)
 @pytest.mark.parametrize("M,N,Kd", [(65, 8, 8), (97, 136, 72), (129, 264, 520), (272, 6592, 40), (391, 6680, 64),
                                     (514, 6744, 120), (879, 6456, 72), (1060, 7184, 200), (161, 2056, 1336)])
 def test_ring_gemm_integer_bit_exact(gpu, oracle, M, N, Kd):
@@ -131,8 +132,8 @@ def test_rmsnorm_matmul_split(gpu, M, N, Kd):
 
 # the int8 K-split stream: slices of 16 to 128 columns (few, ragged, whole), rows
 # at the edges of its 16- and 32-row blocks, K tails of 8 to 56, K splits in
-# library scratch (long K) -- and above 32 rows the int8 ring kernel's five tiles (64 x 128 ... 160 x 256), K tails, K splits
-# (512 columns, long K), N with a ragged 16-column chunk
+# library scratch (long K) -- and above 32 rows K tails, K splits (512 columns,
+# long K), N with a ragged 16-column chunk
 @pytest.mark.parametrize("M,N,Kd", [(1, 16, 8), (16, 16, 72), (17, 144, 520), (5, 1040, 520), (32, 3968, 1472),
                                     (3, 1472, 3968), (16, 2048, 8200), (32, 4096, 4160), (16, 16384, 136),
                                     (9, 11008, 1024), (20, 16384, 512), (33, 16, 8), (65, 144, 72), (129, 272, 520), (48, 512, 4096), (300, 2064, 1032),

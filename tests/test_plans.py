@@ -22,3 +22,36 @@ def test_stream_kernel_holds_a_in_32_bits(M, Kd, N, stream):
     offsets: A of 2^31 bytes or more keeps the tile kernel."""
     for scratch in (0, 64 << 20):
         assert gemm_plan(M, N, Kd, scratch=scratch).kernel == (_lib.PLAN_STREAM if stream else _lib.PLAN_TILE)
+
+
+# us of tile / ring kernel in a replayed graph, rounded; both sides of every line of the rule
+@pytest.mark.parametrize("epi,M,N,Kd,ring", [
+    (0, 300, 1024, 128, False), (0, 300, 1024, 768, True),        # 4.0 / 5.0, 10.3 / 8.2
+    (0, 85, 16, 256, False), (0, 85, 16, 1024, True),             # 4.4 / 5.4, 9.3 / 8.3
+    (1, 700, 512, 64, False), (1, 700, 512, 768, True),           # 5.3 / 6.4, 11.9 / 9.9
+    (1, 1555, 16, 512, False), (1, 1555, 16, 1024, True),         # 7.7 / 9.7, 13.1 / 11.9
+    (2, 304, 1024, 64, False), (2, 700, 4096, 256, True),         # 4.4 / 5.2, 11.0 / 9.9
+    (3, 402, 24, 64, False),                                      # 4.0 / 5.1
+    (0, 4000, 1024, 64, False), (1, 4000, 1024, 64, True),        # 4.2 / 4.5, 14.1 / 11.1 (128 x 128)
+    (0, 4000, 16384, 8, False), (2, 4000, 4096, 8, True),         # 45.9 / 55, (register-staged 256 x 256)
+    (1, 4000, 2304, 256, False), (0, 4000, 2304, 256, True),      # 20.3 / 22.7, 16.4 / 14.6 (direct 256 x 256)
+    (1, 10000, 4096, 512, False), (1, 1500, 4096, 512, True),     # 76.6 / 98.8, 22.9 / 19.0
+    (0, 777, 12288, 4096, True), (1, 501, 8192, 2048, True), (2, 501, 2048, 8192, True), (0, 4096, 16384, 4096, False)])
+def test_gemm_takes_the_faster_kernel(epi, M, N, Kd, ring):
+    assert gemm_plan(M, N, Kd, epi).kernel == (_lib.PLAN_RING if ring else _lib.PLAN_TILE)
+
+
+@pytest.mark.parametrize("epi,M,N,Kd,plan", [
+    (2, 64, 16448, 64, (_lib.PLAN_TILE, 64, 64)), (0, 64, 20000, 16, (_lib.PLAN_TILE, 64, 64)),
+    (0, 32, 20000, 16, (_lib.PLAN_STREAM, 32, 128)), (0, 64, 20000, 1024, (_lib.PLAN_STREAM, 64, 128)),
+    (0, 64, 42496, 4544, (_lib.PLAN_RING, 96, 256)), (0, 40, 50256, 2560, (_lib.PLAN_RING, 96, 256)),
+    (0, 32, 50256, 2560, (_lib.PLAN_STREAM, 32, 128)), (0, 64, 16384, 4096, (_lib.PLAN_STREAM, 64, 64))])
+def test_few_rows_take_the_faster_kernel(epi, M, N, Kd, plan):
+    p = gemm_plan(M, N, Kd, epi, scratch=0)
+    assert (p.kernel, p.block_m, p.block_n) == plan
+
+
+@pytest.mark.parametrize("M,N,Kd,odd", [(1, 50257, 8, True), (32, 50257, 8, True), (33, 50257, 56, False),
+                                        (33, 50257, 64, True), (64, 8191, 8, True), (65, 50257, 64, False)])
+def test_odd_rows_take_the_faster_kernel(M, N, Kd, odd):
+    assert gemm_plan(M, N, Kd).kernel == (_lib.PLAN_ODD if odd else _lib.PLAN_TILE)
