@@ -270,10 +270,24 @@ struct KsPlan {
 // 20.5 -> 17.8 us, [16, 11008, 4096] 16.9 -> 14.0, [32, 4096, 14336] 23.4 ->
 // 19.5); above, its 512-byte runs win ([16, 28672, 8192] 43.5 against 46.4).
 // The time model is that of the bf16 streaming kernel with this kernel's
-// rates, and 5.8 TB/s of memory.
+// rates, and 5.8 TB/s of memory.  Rows of a multiple of 1024 bytes put a slice's
+// rows into the same few channels: on such weights above 32 MB a workgroup of 16
+// rows draws 28 bytes per ns, and 464-512 workgroups, two to a CU, stream as fast
+// as one full round, faster than a round that cannot be filled ([1, 5120, 16384] in
+// 12 21.9 us, in 5 26.5, column-split 21.7; [1, 3072, 22784] in 10 18.2, in 8 20.9,
+// 21.5; [1, 12288, 7296] in 5 21.4, in 2 23.5, 22.3).
+// Not taken, us column-split or generic / here: rows of a k-step or two over many
+// columns ([3, 24640, 32] 2.8 / 3.5, [29, 36064, 64] 5.8 / 7.2; whole 64-k steps only
+// past 256 slices), and few columns over a long K that is no multiple of 64, which
+// the generic kernel splits more finely ([26, 144, 28280] 14.6 / 17.4).
+bool kstream_pays(int N, int K) {
+  if (K % I8S_KSTEP == 0) return K > I8S_KSTEP || N <= 32768;
+  return (K > 104 || N < 4096) && !(N > 64 && N <= 192 && K > 8192);
+}
 bool kstream_plan(int M, int N, int K, size_t scratch, KsPlan &best) {
-  if (M > 32 || N % 16 != 0 || K % 8 != 0 || (size_t)K * N > (size_t)100000000) return false;
+  if (M > 32 || N % 16 != 0 || K % 8 != 0 || (size_t)K * N > (size_t)100000000 || !kstream_pays(N, K)) return false;
   const int mt = M <= 16 ? 1 : 2;
+  const bool lines = mt == 1 && N % 1024 == 0 && (size_t)K * N > (size_t)32000000;
   const int ksteps = (K + I8S_KSTEP - 1) / I8S_KSTEP;
   double best_us = 0;
   for (const KsVariant &v : kI8k) {
@@ -288,8 +302,12 @@ bool kstream_plan(int M, int N, int K, size_t scratch, KsPlan &best) {
       if (part > scratch) break;
       const int64_t units = (int64_t)slices * splits;
       const double rounds = std::ceil(units / 256.0);
-      const double hbm = (double)N * K * (units <= 256 ? 1.0 : 1.1) * (mt == 2 ? 1.1 : 1.0) / 5.8e6;
-      double us = 3.0 + std::max(hbm, rounds * steps * I8S_KSTEP * nb / (v.rate * 1e3));
+      const bool full = lines && units >= 464 && units <= 512;
+      const int round = slices <= 256 ? 256 / slices * slices : 0;  // the fullest single one
+      const double fill = units <= 256 ? 1.0 : !full ? 1.1 : round < (N <= 8192 ? 245 : 210) ? 0.96 : 1.0;
+      const double rate = lines && v.nt == 8 ? 28.0 : v.rate;
+      const double hbm = (double)N * K * fill * (mt == 2 ? 1.1 : 1.0) / 5.8e6;
+      double us = 3.0 + std::max(hbm, rounds * steps * I8S_KSTEP * nb / (rate * 1e3));
       if (splits > 1) us += 2.5 + 2.0 * part / 5e6;
       if (!best.v || us < best_us * (1 - 1e-9)) {
         best_us = us;
@@ -324,9 +342,26 @@ const RingLaunch kI8RingFn[][3] = {I8R_V(2, 2, 6), I8R_V(4, 2, 5), I8R_V(5, 2, 5
 constexpr int kI8RingRows = 32;
 constexpr RingModel kI8RingModel{5.4, 1.1, 0.12, 6.4e6, 2.0, 4.4e6};
 constexpr size_t kInt8ScratchBytes = size_t(16) << 20;
+// Whether the plan beats the column-split stream (K % 64 == 0) or the generic
+// kernel, us of those / here.  Its fixed cost is 4.9 against 2.9 and 2.7, so it
+// needs weights to read: `work` bytes, once for each 64 rows, as the stream does
+// ([53, 1024, 56] 3.0 / 4.9, [44, 512, 368] 4.1 / 6.8, [39, 8192, 64] 3.5 / 5.0;
+// [224, 2800, 184] generic 5.3 / 6.1).  Up to 128 columns the stream has no wide
+// slice ([108, 128, 512] 17.1 / 7.6).  Few tiles over a long K are split in 8 at
+// most, the others in 16 and more ([35, 688, 27968] 23 / 30, [66, 48, 27144]
+// generic 13 / 29, [150, 192, 16384] 17 / 21).
+bool i8_ring_pays(int M, int N, int K, const RingChoice &p) {
+  const double work = (double)((M + 63) / 64) * N * K;
+  if (K % I8S_KSTEP != 0)
+    return p.units > 128 ? p.units > 180 || work > 1.4e6 : (double)M * N * K > 2e8 && (int64_t)M * N > 50000;
+  if (p.splits >= 8 && p.units <= 72 && K > (p.units <= 40 ? 4096 : 8192)) return false;
+  return N <= 128 || !((work <= 1.3e6 && K <= 256) || (work <= 3e6 && K <= 128));
+}
 RingChoice i8_ring_plan(int M, int N, int K, size_t scratch) {
   if (M <= kI8RingRows) return RingChoice{};
-  return ring_choose(kI8Ring, (int)(sizeof kI8Ring / sizeof kI8Ring[0]), kI8RingModel, M, N, K, 1, scratch);
+  const RingChoice p =
+      ring_choose(kI8Ring, (int)(sizeof kI8Ring / sizeof kI8Ring[0]), kI8RingModel, M, N, K, 1, scratch);
+  return p.tile >= 0 && i8_ring_pays(M, N, K, p) ? p : RingChoice{};
 }
 // The built-in choice ahead of the column-split and generic kernels; neither
 // set: those.

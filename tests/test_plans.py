@@ -14,6 +14,12 @@ def gemm_plan(M, N, Kd, epi=0, scratch=64 << 20):
     return p
 
 
+def int8_plan(M, N, Kd, scratch=16 << 20):
+    p = _lib.Plan()
+    _lib.check(_lib.load().pk_int8_plan(M, N, Kd, scratch, C.byref(p)), "pk_int8_plan")
+    return p
+
+
 @pytest.mark.parametrize("M,Kd,N,stream", [(32, 1 << 26, 8, False), (64, 1 << 25, 8, False), (17, 126400000, 8, False),
                                            (64, 33554440, 16, False), (16, 1 << 26, 8, False), (15, 1 << 26, 8, True),
                                            (64, (1 << 24) - 8, 8, True), (1, 126400000, 8, True)])
@@ -55,3 +61,26 @@ def test_few_rows_take_the_faster_kernel(epi, M, N, Kd, plan):
                                         (33, 50257, 64, True), (64, 8191, 8, True), (65, 50257, 64, False)])
 def test_odd_rows_take_the_faster_kernel(M, N, Kd, odd):
     assert gemm_plan(M, N, Kd).kernel == (_lib.PLAN_ODD if odd else _lib.PLAN_TILE)
+
+
+T, S, R = _lib.PLAN_TILE, _lib.PLAN_STREAM, _lib.PLAN_RING
+
+
+# us of the column-split stream or generic kernel / of the K-split stream or ring
+@pytest.mark.parametrize("M,N,Kd,kernel", [
+    (53, 1024, 56, T), (44, 512, 368, T), (39, 8192, 64, T), (224, 2800, 184, T),  # 3.0 / 4.9, 4.1 / 6.8, 3.5 / 5.0, 5.3 / 6.1
+    (35, 688, 27968, T), (66, 48, 27144, T),                                       # 23 / 30, 13 / 29
+    (108, 128, 512, R), (300, 12288, 4096, R), (64, 12288, 4096, R), (33, 12288, 4096, R), (400, 4096, 1032, R),
+    (3, 24640, 32, T), (29, 36064, 64, T), (26, 144, 28280, T),                    # 2.8 / 3.5, 5.8 / 7.2, 14.6 / 17.4
+    (3, 4000, 104, S), (32, 30000, 64, S), (16, 16384, 4096, S), (32, 4096, 14336, S), (16, 28672, 8192, T)])
+def test_int8_takes_the_faster_kernel(M, N, Kd, kernel):
+    assert int8_plan(M, N, Kd).kernel == kernel
+
+
+# weights above 32 MB whose rows are a multiple of 1024 bytes: full rounds of workgroups
+@pytest.mark.parametrize("M,N,Kd", [(1, 5120, 16384), (1, 3072, 22784), (16, 8192, 8192), (8, 4096, 18944), (1, 20480, 4352),
+                                    (16, 6144, 14592), (1, 12288, 7296)])
+def test_int8_stream_fills_its_rounds(M, N, Kd):
+    p = int8_plan(M, N, Kd)
+    units = -(-N // p.block_n) * p.splits
+    assert p.kernel == S and (216 <= units <= 256 or 464 <= units <= 512), units
