@@ -278,7 +278,7 @@ PK_API int pk_gemm_config_ex(int epi, const uint16_t *A, const uint16_t *B, uint
  * configuration or the generic kernel) or one of the kernels that are no
  * configuration, its rows and columns per workgroup, the splits of K (or of the
  * keys) and the k-steps of each. */
-enum { PK_PLAN_TILE = 0, PK_PLAN_STREAM = 1, PK_PLAN_RING = 2, PK_PLAN_ODD = 3 };
+enum { PK_PLAN_TILE = 0, PK_PLAN_STREAM = 1, PK_PLAN_RING = 2, PK_PLAN_ODD = 3, PK_PLAN_RAGGED = 4 };
 typedef struct pk_plan {
   int kernel, block_m, block_n, splits, split_steps;
 } pk_plan;
@@ -297,6 +297,10 @@ PK_API int pk_int8_plan(int M, int N, int K, size_t scratch_bytes, pk_plan *out)
 PK_API int pk_int8_plan_ex(int epi, const uint16_t *A, const int8_t *Wq, const float *scale,
                            uint16_t *C, const uint16_t *R, int M, int N, int K, const pk_plan *plan,
                            void *workspace, size_t workspace_bytes, void *stream);
+
+/* The same for softmax, plain and masked (PK_PLAN_RAGGED: rows of a length that
+ * is no multiple of 8, read in whole chunks). */
+PK_API int pk_softmax_plan(int rows, int cols, pk_plan *out);
 
 /* launch_fused_kv_append_attention with an explicit configuration (one of
  * pk_op_configs("fused_kv_append_attention", S_q, S_cache + S_q, D); NULL =

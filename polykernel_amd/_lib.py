@@ -51,7 +51,7 @@ class Plan(C.Structure):
                 ("split_steps", C.c_int)]
 
 
-PLAN_TILE, PLAN_STREAM, PLAN_RING, PLAN_ODD = range(4)
+PLAN_TILE, PLAN_STREAM, PLAN_RING, PLAN_ODD, PLAN_RAGGED = range(5)
 
 P = C.c_void_p
 I = C.c_int
@@ -103,6 +103,7 @@ SIGNATURES = {
     "pk_gemm_plan_ex": (I, [I, P, P, P, P, P, I, I, I, C.POINTER(Plan), P, SZ, P]),
     "pk_int8_plan": (I, [I, I, I, SZ, C.POINTER(Plan)]),
     "pk_int8_plan_ex": (I, [I, P, P, P, P, P, I, I, I, C.POINTER(Plan), P, SZ, P]),
+    "pk_softmax_plan": (I, [I, I, C.POINTER(Plan)]),
     "pk_op_configs": (I, [C.c_char_p, LL, LL, LL, C.POINTER(Config), I]),
     "pk_op_default_config": (I, [C.c_char_p, LL, LL, LL, C.POINTER(Config)]),
     "pk_naive_matmul": (I, [I, P, P, P, P, P, I, I, I, P]),

@@ -234,8 +234,23 @@ int softmax_run(const RowArgs &a, const pk_config &c, hipStream_t st) {
 // just over 1024 would idle half of four).  [16336, 1021] masked 63.2 -> 26.9 us
 // (5.0 TB/s).  False: longer rows stay with the generic kernel (8 vectors per
 // lane of 16 waves would spill).
+//
+// Few short rows stay with the generic kernel too, whose 256 threads hold one
+// element of a row each, or a few, where a wave here has a chain of eight and
+// more: us in a replayed graph with a mask, generic / ragged, [64, 33] 2.6 / 3.8,
+// [1000, 33] 3.0 / 3.7, [2000, 65] 3.9 / 3.9; [512, 300] 3.5 / 3.7; [256, 700] 4.0 /
+// 4.4, [512, 1021] 5.8 / 5.6; [256, 1021] 4.7 / 5.2, [256, 1300] 6.0 / 5.4; [64, 2047] 6.2 / 3.9.
+bool softmax_few_rows(int rows, int cols) {
+  return rows <= (cols <= 256    ? 1536
+                  : cols <= 505  ? 640
+                  : cols <= 700  ? 512
+                  : cols <= 1009 ? 320
+                  : cols <= 1280 ? 256
+                                 : 0);
+}
 template <int MODE>
 bool softmax_ragged_run(const RowArgs &a, hipStream_t st) {
+  if (softmax_few_rows(a.rows, a.cols)) return false;
   const unsigned rows = (unsigned)a.rows, grid4 = rows / 4 + (rows % 4 != 0);
   const int64_t nvec = ((int64_t)a.cols + 14) / 8;
   if (nvec <= 64) softmax_ragged_kernel<1, 1, MODE><<<grid4, kBlock, 0, st>>>(a);
@@ -547,6 +562,12 @@ int launch_quantize_int8_per_channel(const uint16_t *W, int8_t *Wq, float *scale
   quant_scale_kernel<<<(N + kBlock - 1) / kBlock, kBlock, 0, st>>>(amax_bits, scale, N);
   quant_apply_kernel<<<grid_for((int64_t)K * N), kBlock, 0, st>>>(W, scale, Wq, K, N);
   PK_LAUNCH_CHECK("launch_quantize_int8_per_channel");
+  return PK_OK;
+}
+
+int pk_softmax_plan(int rows, int cols, pk_plan *out) {
+  PK_CHECK_ARG(out && rows > 0 && cols > 0, "pk_softmax_plan: invalid argument");
+  *out = pk_plan{cols % 8 != 0 && cols <= 32754 && !softmax_few_rows(rows, cols) ? PK_PLAN_RAGGED : PK_PLAN_TILE, 0, 0, 1, 0};
   return PK_OK;
 }
 

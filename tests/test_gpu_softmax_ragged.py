@@ -12,9 +12,11 @@ pytestmark = pytest.mark.gpu
 
 
 # one element up to the longest row, lengths just below and above a change of
-# waves or vectors per lane (498 ... 32754 columns), and row counts
-# that leave the last chunk of the tensor short or whole
-@pytest.mark.parametrize("rows,cols", [(1, 1), (5, 3), (8, 9), (3, 497), (6, 499), (7, 1009), (5, 1011), (4, 1521),
+# waves or vectors per lane (498 ... 32754 columns), and row counts that leave
+# the last chunk of the tensor short or whole; up to 1280 columns with few rows
+# (the generic kernel) and with more (the ragged one)
+@pytest.mark.parametrize("rows,cols", [(1537, 1), (1539, 3), (1544, 9), (2001, 255), (643, 497), (645, 499), (517, 699),
+                                       (323, 1009), (325, 1011), (257, 1279), (1, 1), (5, 3), (8, 9), (3, 497), (6, 499), (7, 1009), (5, 1011), (4, 1521),
                                        (5, 1523), (9, 2033), (5, 2035), (3, 4081), (3, 4083), (5, 8177), (3, 8179),
                                        (3, 16369), (3, 16371), (3, 32753), (2, 32755), (97, 1021)])
 def test_softmax_ragged_rows(gpu, oracle, rows, cols):
@@ -32,12 +34,13 @@ def test_softmax_ragged_rows(gpu, oracle, rows, cols):
         assert rep.max_ulp <= 1 and (1 - rep.bit_exact) * want.size <= max(2, 0.02 * want.size), rep
 
 
-def test_softmax_ragged_neighbour_rows_do_not_mix(gpu, oracle):
+@pytest.mark.parametrize("rows", [9, 263])  # the generic kernel, the ragged one
+def test_softmax_ragged_neighbour_rows_do_not_mix(gpu, oracle, rows):
     """A row of infinities or NaN between ordinary rows, and a fully masked row:
     only that row's outputs are affected, although its neighbours read its elements."""
     from polykernel_amd import kernels
 
-    rows, cols = 9, 1021
+    cols = 1021
     lg = synth.normal_f32((rows, cols), 173, 2.0)
     mask = synth.mask_bf16((rows, cols), 174, 0.3)
     mask[:, 0] = 0

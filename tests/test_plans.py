@@ -84,3 +84,14 @@ def test_int8_stream_fills_its_rounds(M, N, Kd):
     p = int8_plan(M, N, Kd)
     units = -(-N // p.block_n) * p.splits
     assert p.kernel == S and (216 <= units <= 256 or 464 <= units <= 512), units
+
+
+# us of the generic / the ragged kernel: 2.6 / 3.8, 3.0 / 3.7, 3.5 / 3.7, 4.0 / 4.4, 4.7 / 5.2, then the other way
+@pytest.mark.parametrize("rows,cols,ragged", [
+    (64, 33, False), (1000, 33, False), (512, 300, False), (256, 700, False), (256, 1021, False), (4000, 33, True),
+    (1000, 300, True), (512, 1021, True), (64, 2047, True), (1, 32753, True), (16336, 1021, True), (16336, 1024, False),
+    (1, 32755, False)])
+def test_softmax_takes_the_faster_kernel(rows, cols, ragged):
+    p = _lib.Plan()
+    _lib.check(_lib.load().pk_softmax_plan(rows, cols, C.byref(p)), "pk_softmax_plan")
+    assert (p.kernel == _lib.PLAN_RAGGED) == ragged
