@@ -278,7 +278,8 @@ PK_API int pk_gemm_config_ex(int epi, const uint16_t *A, const uint16_t *B, uint
  * configuration or the generic kernel) or one of the kernels that are no
  * configuration, its rows and columns per workgroup, the splits of K (or of the
  * keys) and the k-steps of each. */
-enum { PK_PLAN_TILE = 0, PK_PLAN_STREAM = 1, PK_PLAN_RING = 2, PK_PLAN_ODD = 3, PK_PLAN_RAGGED = 4 };
+enum { PK_PLAN_TILE = 0, PK_PLAN_STREAM = 1, PK_PLAN_RING = 2, PK_PLAN_ODD = 3, PK_PLAN_RAGGED = 4,
+       PK_PLAN_DECODE = 5, PK_PLAN_FLASH = 6, PK_PLAN_FLASH_HALF = 7, PK_PLAN_FLASH_PAIR = 8 };
 typedef struct pk_plan {
   int kernel, block_m, block_n, splits, split_steps;
 } pk_plan;
@@ -301,6 +302,11 @@ PK_API int pk_int8_plan_ex(int epi, const uint16_t *A, const int8_t *Wq, const f
 /* The same for softmax, plain and masked (PK_PLAN_RAGGED: rows of a length that
  * is no multiple of 8, read in whole chunks). */
 PK_API int pk_softmax_plan(int rows, int cols, pk_plan *out);
+
+/* The same for attention of BH heads on S_cache keys, or, with `append`, on S_q
+ * more behind them (aligned operands, scale > 0); `*fused` (may be NULL): the
+ * kernel appends.  After an append of its own a call takes the plan without one. */
+PK_API int pk_attention_plan(int BH, int S_q, int S_cache, int D, int append, int causal, pk_plan *out, int *fused);
 
 /* launch_fused_kv_append_attention with an explicit configuration (one of
  * pk_op_configs("fused_kv_append_attention", S_q, S_cache + S_q, D); NULL =

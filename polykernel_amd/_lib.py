@@ -52,6 +52,7 @@ class Plan(C.Structure):
 
 
 PLAN_TILE, PLAN_STREAM, PLAN_RING, PLAN_ODD, PLAN_RAGGED = range(5)
+PLAN_DECODE, PLAN_FLASH, PLAN_FLASH_HALF, PLAN_FLASH_PAIR = range(5, 9)
 
 P = C.c_void_p
 I = C.c_int
@@ -104,6 +105,7 @@ SIGNATURES = {
     "pk_int8_plan": (I, [I, I, I, SZ, C.POINTER(Plan)]),
     "pk_int8_plan_ex": (I, [I, P, P, P, P, P, I, I, I, C.POINTER(Plan), P, SZ, P]),
     "pk_softmax_plan": (I, [I, I, C.POINTER(Plan)]),
+    "pk_attention_plan": (I, [I, I, I, I, I, I, C.POINTER(Plan), C.POINTER(C.c_int)]),
     "pk_op_configs": (I, [C.c_char_p, LL, LL, LL, C.POINTER(Config), I]),
     "pk_op_default_config": (I, [C.c_char_p, LL, LL, LL, C.POINTER(Config)]),
     "pk_naive_matmul": (I, [I, P, P, P, P, P, I, I, I, P]),

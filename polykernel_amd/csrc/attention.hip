@@ -26,6 +26,7 @@
 // and att_combine_kernel merges the fp32 partials in split order.  Head dims
 // 64 and 128 take attention_fa_kernel (below), and up to 4 queries of them
 // attention_decode_kernel.
+#include <algorithm>
 #include <cstring>
 
 #include "attention_decode.hpp"
@@ -370,22 +371,35 @@ int attention_fa(FaArgs a, int D, int qg, bool built_in, hipStream_t st, const A
 
 // 1 to 4 queries per head: the streaming kernel, for operands the flash kernel
 // takes (any S_cache, since rows are read one by one) when every query sees a
-// key.  Key splits while the (b, h) alone leave CUs idle, each keeping a batch
-// per wave.
+// key.  Three or four queries on up to 128 keys of D 64 without an append are the
+// flash kernel's (one step and no merge of 32 lane groups: 96 heads of 4 on 4 keys
+// 5.0 us against 5.9).
+//
+// Key splits in one round of 256 workgroups (a CU holds one: a second round of a
+// few took 160 heads of 4096 keys at D 64 from 31 to 38 us, 100 heads in 4 instead
+// of 2 from 26 to 32 with four queries), each of about a batch per wave and more, and
+// no more than the merge's reads are worth (8 heads of 16384 keys 16.4 us in 10
+// to 16, 21.7 in 32).
+int decode_splits(int BH, int S_q, int S_kv, int D) {
+  const int batch = AD_U * 512 / D;  // keys of a wave's batch
+  const int batches = (S_kv + batch - 1) / batch;
+  const int most = batches >= 256 ? 16 : S_q <= 2 ? 8 : 12;
+  const int least = D == 64 ? 10 : 8;  // batches of a split
+  return std::max(1, std::min({256 / BH, most, (batches + least / 2) / least}));
+}
 // Key splits of the flash kernel's 64 x 128 tile for the same call (128 x 64
 // where only that tile could append).
 int decode_base_splits(const FaArgs &a) {
   const int bkv = a.Kn && a.S_cache % 128 != 0 && a.S_cache % 64 == 0 ? 64 : 128;
   return split_count(a.BH, (a.S_kv + bkv - 1) / bkv, 8, 8);
 }
-bool decode_applicable(int S_q, int S_kv, bool causal) {
+bool decode_applicable(int S_q, int S_kv, int D, bool append, bool causal) {
+  if (!append && S_q > 2 && D == 64 && S_kv <= 128) return false;
   return S_q > 0 && S_q <= AD_MAX_Q && S_kv > 0 && (!causal || S_kv >= S_q);
 }
 int attention_decode(FaArgs a, int D, hipStream_t st) {
   a.q_tiles = 1;
-  const int batch = AD_U * 512 / D;  // keys of a wave's batch
-  a.splits = 1;
-  while (a.BH * a.splits < 256 && a.S_kv / (a.splits * 2) >= AD_WAVES * batch && a.splits < 64) a.splits *= 2;
+  a.splits = decode_splits(a.BH, a.S_q, a.S_kv, D);
   const size_t rows = (size_t)a.BH * a.S_q;
   const size_t split_bytes = rows * (D + 2) * sizeof(float);
   WorkspaceLease lease;  // held until the merge kernel is queued
@@ -395,7 +409,7 @@ int attention_decode(FaArgs a, int D, hipStream_t st) {
     const int base = decode_base_splits(a);
     int rc = library_workspace(base > 1 ? std::min(base, a.splits) * split_bytes : 0, a.splits * split_bytes, st, lease);
     if (rc) return rc;
-    while (a.splits > 1 && lease.bytes < a.splits * split_bytes) a.splits /= 2;
+    a.splits = std::max(1, std::min(a.splits, (int)std::min<size_t>(lease.bytes / split_bytes, 256)));
     a.part_o = static_cast<float *>(lease.ptr);
     a.part_ml = a.part_o + (size_t)a.splits * rows * D;
   }
@@ -479,7 +493,7 @@ int fa_qg_of(const pk_config &c, int D) {
 int attention_run(const uint16_t *Q, const uint16_t *K, const uint16_t *V, uint16_t *O, int BH,
                   int S_q, int S_kv, int D, int kv_rows, float scale, int causal, int mode, hipStream_t st,
                   const AttModule *mod = nullptr) {
-  if (mode == 0 && scale > 0.f && decode_applicable(S_q, S_kv, causal != 0) &&
+  if (mode == 0 && scale > 0.f && decode_applicable(S_q, S_kv, D, false, causal != 0) &&
       fa_applicable(S_kv, S_kv, D, kv_rows, Q, K, V, O, nullptr, nullptr, nullptr, nullptr, 1)) {
     return attention_decode(FaArgs{Q, K, V, nullptr, nullptr, nullptr, nullptr, O, nullptr, nullptr, BH, S_q, S_kv,
                                    S_kv, kv_rows, scale, causal, 1, 1},
@@ -541,7 +555,7 @@ int fused_kv_append_attention(const uint16_t *Q, uint16_t *Kc, uint16_t *Vc, con
     auto fits = [&](int bkv) {
       return fa_applicable(S_kv, S_cache, D, cache_capacity, Q, Kc, Vc, O, Kn, Vn, Kc, Vc, bkv);
     };
-    if (!mode && decode_applicable(S_q, S_kv, causal != 0) && fits(1)) {
+    if (!mode && decode_applicable(S_q, S_kv, D, true, causal != 0) && fits(1)) {
       return attention_decode(FaArgs{Q, Kc, Vc, Kn, Vn, Kc, Vc, O, nullptr, nullptr, (int)BH, S_q, S_kv, S_cache,
                                      cache_capacity, scale, causal, 1, 1},
                               D, st);
@@ -571,6 +585,28 @@ int fused_kv_append_attention(const uint16_t *Q, uint16_t *Kc, uint16_t *Vc, con
 using namespace pk;
 
 extern "C" {
+
+int pk_attention_plan(int BH, int S_q, int S_cache, int D, int append, int causal, pk_plan *out, int *fused) {
+  PK_CHECK_ARG(out && BH > 0 && S_q > 0 && S_q <= INT32_MAX - 1023 && S_cache >= 0 && (append || S_cache > 0) && D > 0 &&
+                   S_cache <= INT32_MAX - 1023 - (append ? S_q : 0),
+               "pk_attention_plan: invalid argument");
+  const int S_kv = S_cache + (append ? S_q : 0);
+  const bool flash = D == 64 || D == 128;
+  int inside = 0;
+  if (flash && decode_applicable(S_q, S_kv, D, append != 0, causal != 0)) {
+    const int s = decode_splits(BH, S_q, S_kv, D);
+    *out = pk_plan{PK_PLAN_DECODE, S_q, AD_U * 512 / D, s, 0};
+    inside = append != 0;
+  } else if (flash) {
+    const int qg = fa_default_qg(BH, S_q, S_kv, D, causal != 0);
+    *out = pk_plan{PK_PLAN_FLASH, fa_bq(qg), fa_bkv(qg), 1, (S_kv + fa_bkv(qg) - 1) / fa_bkv(qg)};
+    inside = append && S_cache % fa_bkv(qg) == 0 && !fa_pairs(BH, S_q, D, qg);
+  } else {
+    *out = pk_plan{PK_PLAN_TILE, 0, 0, 1, 0};
+  }
+  if (fused) *fused = inside;
+  return PK_OK;
+}
 
 int launch_attention_prefill(const uint16_t *Q, const uint16_t *K, const uint16_t *V, uint16_t *O,
                              int B, int H, int S_q, int S_kv, int D, float scale, int causal,

@@ -40,6 +40,52 @@ __device__ __forceinline__ float row_lane_sum(float v) {
   return v;
 }
 
+// The merge over a wave's groups (lanes l, l ^ LPR, l ^ 2 LPR, ... up to l ^ 32)
+// by the two lane swaps and, for 8 lanes per row, a rotation by 8 in each 16.
+// With shuffles (LDS permutes) of every value it was most of a short call of
+// four queries: 1 head of 8 keys at D 64 8.2 us.
+__device__ __forceinline__ void xor16_pair(float a, float b, float &lo, float &hi) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  lo = __uint_as_float(r[0]);
+  hi = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float row_ror8(float v) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x128, 0xF, 0xF, true));
+}
+// f over the groups, in every lane.
+template <int LPR, typename F>
+__device__ __forceinline__ float group_combine(float v, F &&f) {
+  static_assert(LPR == 8 || LPR == 16, "lanes per row");
+  float lo, hi;
+  xor32_pair(v, lo, hi);
+  v = f(lo, hi);
+  xor16_pair(v, v, lo, hi);
+  v = f(lo, hi);
+  if constexpr (LPR == 8) v = f(v, row_ror8(v));
+  return v;
+}
+// Sums of v[0..7] over the groups: a swap of two values adds both at once, each
+// in one half of the lanes, so the lanes of 16-lane row r (0-3) end up with the
+// sums of v[4 (r / 2) + 2 (r % 2)] and the value after it.
+template <int LPR>
+__device__ __forceinline__ void group_sum8(const float (&v)[8], float &s0, float &s1) {
+  float h[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[e]), __float_as_uint(v[e + 4]), false, false);
+    h[e] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+  float lo, hi;
+  xor16_pair(h[0], h[2], lo, hi);
+  s0 = lo + hi;
+  xor16_pair(h[1], h[3], lo, hi);
+  s1 = lo + hi;
+  if constexpr (LPR == 8) {
+    s0 += row_ror8(s0);
+    s1 += row_ror8(s1);
+  }
+}
+
 template <int D, int NQ>
 __device__ __forceinline__ void att_decode_body(FaArgs g) {
   constexpr int LPR = D / 8;             // lanes per row
@@ -176,26 +222,29 @@ __device__ __forceinline__ void att_decode_body(FaArgs g) {
     if (nb < b_end) load(vr, Vp, Vnp, nb);
   }
 
-  // ---- merge the states of the wave's groups (lanes l, l ^ LPR, ...), then
-  // of the waves in LDS, in wave order
+  // ---- merge the states of the wave's groups, then of the waves in LDS, in wave
+  // order; a wave without a batch has nothing to merge
   auto weight = [&](float m, float M) __attribute__((always_inline)) {
     return m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - M) * c2);
   };
+  const bool any = split * per + wid < b_end;
 #pragma unroll
   for (int i = 0; i < NQ; ++i) {
-    float M = m_run[i];
+    float M = -INFINITY, l = 0.f, s0 = 0.f, s1 = 0.f;
+    if (any) {
+      M = group_combine<LPR>(m_run[i], [](float a, float b) __attribute__((always_inline)) { return fmaxf(a, b); });
+      const float w = weight(m_run[i], M);
+      l = group_combine<LPR>(l_run[i] * w, [](float a, float b) __attribute__((always_inline)) { return a + b; });
+      float v[8];
 #pragma unroll
-    for (int o = LPR; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
-    const float w = weight(m_run[i], M);
-    float l = l_run[i] * w;
-#pragma unroll
-    for (int o = LPR; o < 64; o <<= 1) l += __shfl_xor(l, o, 64);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float v = acc[i][e] * w;
-#pragma unroll
-      for (int o = LPR; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);
-      if (grp == 0) so[wid][i][d0 + e] = v;
+      for (int e = 0; e < 8; ++e) v[e] = acc[i][e] * w;
+      group_sum8<LPR>(v, s0, s1);
+    }
+    const int r = lane >> 4;
+    if (LPR == 16 || !(lane & 8)) {
+      float *o = &so[wid][i][d0 + 4 * (r >> 1) + 2 * (r & 1)];
+      o[0] = s0;
+      o[1] = s1;
     }
     if (lane == 0) {
       sml[wid][i][0] = M;

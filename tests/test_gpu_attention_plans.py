@@ -58,9 +58,9 @@ def test_decode_append_attention(gpu, oracle, B, H, Sq, Sc, spare, D):
 
 
 # more than 4 queries: the step that holds row S_cache reads cached and new
-# rows -- first, last or only step, one row from either edge, in the middle of
-# a long unmasked run, with key splits (few heads) and with D 64 in one round
-# (half ring) and several (pairs)
+# more than 4 queries behind a cache of any length: the append is a launch of its
+# own unless the cache ends on a key step of the tile; with key splits (few heads)
+# and with D 64 in one round (half ring) and several (pairs)
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("B,H,Sq,Sc", [(1, 2, 5, 1), (1, 2, 70, 127), (1, 2, 70, 129), (2, 3, 33, 1000), (1, 4, 600, 65),
                                        (1, 2, 333, 1501), (2, 16, 600, 961), (3, 40, 130, 201)])

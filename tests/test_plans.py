@@ -95,3 +95,31 @@ def test_softmax_takes_the_faster_kernel(rows, cols, ragged):
     p = _lib.Plan()
     _lib.check(_lib.load().pk_softmax_plan(rows, cols, C.byref(p)), "pk_softmax_plan")
     assert (p.kernel == _lib.PLAN_RAGGED) == ragged
+
+
+def attention_plan(BH, S_q, S_cache, D, append=True, causal=True):
+    p, fused = _lib.Plan(), C.c_int()
+    _lib.check(_lib.load().pk_attention_plan(BH, S_q, S_cache, D, int(append), int(causal), C.byref(p),
+                                             C.byref(fused)), "pk_attention_plan")
+    return p, bool(fused.value)
+
+
+# us with as many splits as before / now
+@pytest.mark.parametrize("BH,S_q,S_cache,D,append,splits", [
+    (160, 1, 4096, 64, False, 1),    # 38 in two rounds / 31
+    (100, 4, 4096, 64, False, 2),    # 32 in 4 / 26
+    (8, 1, 16384, 128, False, 16), (1, 1, 1 << 20, 128, False, 16),
+    (32, 1, 256, 128, True, 1), (32, 4, 2048, 128, True, 8), (1, 2, 8, 128, True, 1), (300, 1, 1 << 16, 64, True, 1)])
+def test_decode_splits(BH, S_q, S_cache, D, append, splits):
+    p, fused = attention_plan(BH, S_q, S_cache, D, append)
+    assert (p.kernel, p.splits, fused) == (_lib.PLAN_DECODE, splits, append)
+    assert p.splits == 1 or p.splits * BH <= 256
+
+
+@pytest.mark.parametrize("S_q,S_cache,D,append,decode", [
+    (4, 128, 64, False, False), (3, 4, 64, False, False), (4, 129, 64, False, True), (2, 4, 64, False, True),
+    (4, 128, 128, False, True), (4, 124, 64, True, True), (5, 4096, 64, False, False), (4, 0, 64, True, True)])
+def test_few_queries_on_short_keys(S_q, S_cache, D, append, decode):
+    """Three and four queries on up to 128 keys of D 64: flash 5.0 us, decode 5.9 (96 heads, 4 keys)."""
+    assert (attention_plan(96, S_q, S_cache, D, append)[0].kernel == _lib.PLAN_DECODE) == decode
+
