@@ -275,25 +275,31 @@ int fa_default_qg(int64_t BH, int S_q, int S_kv, int D, bool causal) {
   return BH * ((S_q + fa_bq(4) - 1) / fa_bq(4)) >= 256 ? 4 : 2;
 }
 
-// Whether the built-in choice runs two workgroups per CU (D 64, more than one
-// round).  The append stays out of that kernel: inside its 128 registers it
-// spilled (128 heads, 256 + 2048: 65.7 us against 46.8 fused in the 128 x 64 tile).
-bool fa_pairs(int64_t BH, int S_q, int D, int qg) {
-  return D == 64 && qg == 2 && BH * ((S_q + fa_bq(2) - 1) / fa_bq(2)) > 256;
-}
+// The flash kernel's K/V ring at D 64: the whole LDS, half of it (one workgroup
+// per CU all the same, fewer steps in flight), half of it in 128 registers (two).
+enum class FaRing { kFull, kHalf, kPair };
+struct FaChoice {
+  int qg = 2, splits = 1;
+  FaRing ring = FaRing::kFull;
+  bool fused = false;  // the append happens inside the kernel
+};
 
-// Key splits of the built-in choice: few tiles over many keys leave CUs idle, so
-// splits follow the time of the longest tile's steps (1.6 us each at D 128, 1.0
-// at 64) against the merge (4 us and its reads;
-// 8 heads of 500 queries and keys in 4 took 15.9 us against 12.7 unsplit), within one
-// round of 256 workgroups: 16 heads of 7 on 1000 cached keys 19.5 -> 14.6 us, 12
-// of 29 on 3200 26.1 -> 20.6.  A configuration keeps split_count's >= 8 steps.
-int fa_splits(int64_t tiles, int steps, int D) {
-  const double step_us = D == 128 ? 1.6 : 1.0;
+// Key splits of the built-in choice: few tiles over many keys leave CUs idle.  The
+// longest workgroup's steps (a 64 x 128 step takes 0.85 us at D 64 and 1.3 at 128,
+// and 0.4 more when all 256 CUs read) against the merge, whose part grows with
+// the rows it reads back, within one round of 256 workgroups.  16 heads of 7 on
+// 1000 cached keys at D 128 19.5 -> 14.6 us, 12 of 29 on 3200 26.1 -> 20.6; D 64, 7
+// heads of 1995 22.1 unsplit, 32.0 in 2; 108 of 99 on 2816 27.8 and 39.8.  More than
+// 8 keep 8 steps each, since the merge reads them one after the other (4 heads of 16
+// on 8192 keys 18.3 us in 8, 19.8 in 16).  A configuration keeps split_count's.
+int fa_splits(int64_t tiles, int steps, int64_t rows, int D) {
+  const double step_us = D == 128 ? 1.3 : 0.85, fill_us = D == 128 ? 0.37 : 0.39;
+  const double row_us = D == 128 ? 0.25e-3 : 0.07e-3;
   int best = 1;
-  double best_us = 0.9 * steps * step_us;
-  for (int s = 2; s <= 16 && tiles * s <= 256 && s <= steps; s *= 2) {
-    const double us = (steps + s - 1) / s * step_us + 4.0 + 0.25 * s;
+  double best_us = steps * (step_us + fill_us * tiles / 256);
+  for (int s : {2, 3, 4, 6, 8, 12, 16}) {
+    if (tiles * s > 256 || (s > 8 ? 8 : 2) * s > steps) break;
+    const double us = (steps + s - 1) / s * (step_us + fill_us * tiles * s / 256) + 2.7 + s * (0.1 + row_us * rows);
     if (us < best_us) {
       best_us = us;
       best = s;
@@ -302,25 +308,66 @@ int fa_splits(int64_t tiles, int steps, int D) {
   return best;
 }
 
-// Launch the flash-style kernel with QG query groups per workgroup, with
-// enough key splits to reach ~256 workgroups, each split keeping >= 8 steps.
-// `built_in`: no configuration was asked for, so D 64 may take the half ring:
-// alone on a CU in one round ([32 heads, 333 + 1501] 21.3 -> 19.1 us, 16 of 1021
-// 14.1 -> 13.2; 32 of 512 on 4096 keys 36.0 -> 36.5), in pairs above.
-int attention_fa(FaArgs a, int D, int qg, bool built_in, hipStream_t st, const AttModule *mod) {
+// The built-in choice of the flash kernel's variant: S_cache >= 0 appends S_kv -
+// S_cache rows behind S_cache cached ones, -1 is attention alone.
+//
+// The tile starts from fa_default_qg.  At D 128 an append behind a multiple of 64 but
+// not of 128 rows takes the 128 x 64 tile, which can append there.  At D 64 that
+// pays up to 128 keys (64 + 5 to 64 + 38: 6.3 to 8.1 us against 7.4 to 9.2 with the append
+// launched first; 128 to 256 keys 1.06 times as long), and more than one round of
+// 64-query tiles whose prompts fill 65 to 128 rows keeps it while there is little to
+// read (449 heads of 68 on 73 keys 13.2 us against 16.0 in pairs; behind a cache, where
+// the append would be a launch of its own, up to 256 keys: 466 of 74 + 128 22.6 against
+// 26.1), and one round of it up to 704 instead of 512 keys (64 heads of 500 + 64 19.5
+// against 21.8).
+//
+// More than one round at D 64 runs two workgroups per CU.  The append stays out of
+// that kernel, inside its 128 registers it spilled; its launch and the pair kernel
+// take 1.01 to 1.15 times less than the 64 x 128 tile that appends, 5 to 15 % less than
+// 128 x 64 from 768 keys on.
+//
+// One round at D 64 takes the half ring for few steps of 128 keys (3 to 5 % less than
+// the full ring; 16 heads of 1021 14.1 -> 13.2 us) and the full ring above, where the
+// deeper queue covers memory (4096 keys 5 to 26 % less, 141 heads of 12 on 9472 71 us
+// against 100): from 12 steps where no other tile reads the same keys (half / full 1.02
+// at 12, 1.06 at 14), 14 with a few (1.00 at 14, 1.03 at 18), 17 with ten (1.01 at 18).
+FaChoice fa_choice(int64_t BH, int S_q, int S_kv, int S_cache, int D, bool causal) {
+  FaChoice c;
+  const bool append = S_cache >= 0, odd64 = append && S_cache % 128 == 64;
+  const int q_tiles = (S_q + fa_bq(2) - 1) / fa_bq(2);
+  const int64_t fine = BH * q_tiles;
+  c.qg = fa_default_qg(BH, S_q, S_kv, D, causal);
+  if (c.qg == 2 && odd64 && (D == 128 || (fine <= 256 && S_kv <= 128))) c.qg = 4;
+  const bool inside = append && S_cache % fa_bkv(4) == 0;
+  if (D == 64 && fine > 256 && S_q > fa_bq(2) && S_q <= fa_bq(4) && S_kv <= (inside ? 256 : 128)) c.qg = 4;
+  if (D == 64 && fine > 256 && inside && BH * ((S_q + fa_bq(4) - 1) / fa_bq(4)) <= 256 && S_kv <= 704) c.qg = 4;
+  const int steps = (S_kv + fa_bkv(c.qg) - 1) / fa_bkv(c.qg);
+  c.splits = fa_splits(BH * ((S_q + fa_bq(c.qg) - 1) / fa_bq(c.qg)), steps, BH * S_q, D);
+  if (D == 64 && c.qg == 2) {
+    if (fine > 256) c.ring = FaRing::kPair;
+    else if ((steps + c.splits - 1) / c.splits <= (q_tiles == 1 ? 11 : q_tiles < 10 ? 13 : 16)) c.ring = FaRing::kHalf;
+  }
+  c.fused = append && S_cache % fa_bkv(c.qg) == 0 && c.ring != FaRing::kPair;
+  return c;
+}
+
+// Launch the flash-style kernel: a configuration's tile (enough key splits to reach
+// ~256 workgroups, each keeping >= 8 steps), or the built-in choice.
+int attention_fa(FaArgs a, int D, const FaChoice &choice, bool built_in, hipStream_t st, const AttModule *mod) {
+  const int qg = choice.qg;
   const int BQ = fa_bq(qg), BKV = fa_bkv(qg);
   a.q_tiles = (a.S_q + BQ - 1) / BQ;
   const int ntiles = (a.S_kv + BKV - 1) / BKV;
   const size_t rows = (size_t)a.BH * a.S_q;
   auto part_bytes = [&](int splits) { return splits > 1 ? (size_t)splits * rows * (D + 2) * sizeof(float) : 0; };
   const int base = split_count((int64_t)a.BH * a.q_tiles, ntiles, 8, 8);
-  a.splits = built_in ? std::max(base, fa_splits((int64_t)a.BH * a.q_tiles, ntiles, D)) : base;
+  a.splits = built_in ? choice.splits : base;
   if (int rc = grid_ok(a.BH, a.q_tiles, a.splits, "attention")) return rc;
   WorkspaceLease lease;  // held until the merge kernel is queued
   if (a.splits > 1) {
-    int rc = library_workspace(part_bytes(base), part_bytes(a.splits), st, lease);
+    int rc = library_workspace(part_bytes(std::min(base, a.splits)), part_bytes(a.splits), st, lease);
     if (rc) return rc;
-    if (lease.bytes < part_bytes(a.splits)) a.splits = base;  // the workspace can't grow now
+    if (lease.bytes < part_bytes(a.splits)) a.splits = std::min(base, a.splits);  // the workspace can't grow now
   }
   if (a.splits > 1) {
     a.part_o = static_cast<float *>(lease.ptr);
@@ -343,13 +390,11 @@ int attention_fa(FaArgs a, int D, int qg, bool built_in, hipStream_t st, const A
     if (fused) attention_fa_kernel<DPV, QGV, true><<<blocks, FA_THREADS, 0, st>>>(a);       \
     else attention_fa_kernel<DPV, QGV, false><<<blocks, FA_THREADS, 0, st>>>(a);            \
   } while (0)
-  if (built_in && D == 64 && qg == 2) {
-    if (!fa_pairs(a.BH, a.S_q, D, qg)) {
-      if (fused) attention_fa_half_kernel<true><<<blocks, FA_THREADS, 0, st>>>(a);
-      else attention_fa_half_kernel<false><<<blocks, FA_THREADS, 0, st>>>(a);
-    } else {
-      attention_fa_pair_kernel<<<blocks, FA_THREADS, 0, st>>>(a);
-    }
+  if (choice.ring == FaRing::kPair) {
+    attention_fa_pair_kernel<<<blocks, FA_THREADS, 0, st>>>(a);
+  } else if (choice.ring == FaRing::kHalf) {
+    if (fused) attention_fa_half_kernel<true><<<blocks, FA_THREADS, 0, st>>>(a);
+    else attention_fa_half_kernel<false><<<blocks, FA_THREADS, 0, st>>>(a);
   } else if (D == 128) {
     if (qg == 4) PK_FA_LAUNCH(128, 4);
     else PK_FA_LAUNCH(128, 2);
@@ -500,12 +545,13 @@ int attention_run(const uint16_t *Q, const uint16_t *K, const uint16_t *V, uint1
                             D, st);
   }
   if (mode >= 0) {
-    const int qg = mode ? mode : fa_default_qg(BH, S_q, S_kv, D, causal != 0);
+    const FaChoice choice = mode ? FaChoice{mode} : fa_choice(BH, S_q, S_kv, -1, D, causal != 0);
+    const int qg = choice.qg;
     if (scale > 0.f && fa_applicable(S_kv, S_kv, D, kv_rows, Q, K, V, O, nullptr, nullptr, nullptr, nullptr,
                                      fa_bkv(qg))) {
       FaArgs a{Q, K, V, nullptr, nullptr, nullptr, nullptr, O, nullptr, nullptr, BH, S_q, S_kv, S_kv, kv_rows,
                scale, causal, 1, 1};
-      return attention_fa(a, D, qg, mode == 0, st, mod);
+      return attention_fa(a, D, choice, mode == 0, st, mod);
     }
     if (mode) {
       set_error("attention: the flash kernel (%d x %d tiles) needs D 64 or 128, 16-byte aligned tensors and "
@@ -549,7 +595,8 @@ int fused_kv_append_attention(const uint16_t *Q, uint16_t *Kc, uint16_t *Vc, con
                INT32_MAX);
   const int S_kv = S_cache + S_q;
   if (S_q > 0 && scale > 0.f && mode >= 0) {
-    int qg = mode ? mode : fa_default_qg(BH, S_q, S_kv, D, causal != 0);
+    const FaChoice choice = mode ? FaChoice{mode, 1, FaRing::kFull, true}
+                                 : fa_choice(BH, S_q, S_kv, S_cache, D, causal != 0);
     // the append inside the attention kernel needs S_cache on a key step of the
     // tile; the decode kernel takes any, the pair kernel none
     auto fits = [&](int bkv) {
@@ -560,12 +607,11 @@ int fused_kv_append_attention(const uint16_t *Q, uint16_t *Kc, uint16_t *Vc, con
                                      cache_capacity, scale, causal, 1, 1},
                               D, st);
     }
-    if (!mode && D == 128 && qg == 2 && !fits(fa_bkv(2))) qg = 4;  // S_cache on a 64-key but not a 128-key step
-    if (fits(fa_bkv(qg)) && !(!mode && fa_pairs(BH, S_q, D, qg))) {
+    if (choice.fused && fits(fa_bkv(choice.qg))) {
       // the append happens inside the attention kernel
       FaArgs a{Q, Kc, Vc, Kn, Vn, Kc, Vc, O, nullptr, nullptr, (int)BH, S_q, S_kv, S_cache, cache_capacity,
                scale, causal, 1, 1};
-      return attention_fa(a, D, qg, mode == 0, st, mod);
+      return attention_fa(a, D, choice, mode == 0, st, mod);
     }
   }
   if (mode > 0) {
@@ -598,9 +644,13 @@ int pk_attention_plan(int BH, int S_q, int S_cache, int D, int append, int causa
     *out = pk_plan{PK_PLAN_DECODE, S_q, AD_U * 512 / D, s, 0};
     inside = append != 0;
   } else if (flash) {
-    const int qg = fa_default_qg(BH, S_q, S_kv, D, causal != 0);
-    *out = pk_plan{PK_PLAN_FLASH, fa_bq(qg), fa_bkv(qg), 1, (S_kv + fa_bkv(qg) - 1) / fa_bkv(qg)};
-    inside = append && S_cache % fa_bkv(qg) == 0 && !fa_pairs(BH, S_q, D, qg);
+    const FaChoice c = fa_choice(BH, S_q, S_kv, append ? S_cache : -1, D, causal != 0);
+    const int steps = (S_kv + fa_bkv(c.qg) - 1) / fa_bkv(c.qg);
+    *out = pk_plan{c.ring == FaRing::kPair   ? PK_PLAN_FLASH_PAIR
+                   : c.ring == FaRing::kHalf ? PK_PLAN_FLASH_HALF
+                                             : PK_PLAN_FLASH,
+                   fa_bq(c.qg), fa_bkv(c.qg), c.splits, (steps + c.splits - 1) / c.splits};
+    inside = c.fused;
   } else {
     *out = pk_plan{PK_PLAN_TILE, 0, 0, 1, 0};
   }

@@ -86,3 +86,40 @@ def test_flash_d64_rings(gpu, oracle, BH, Sq, Skv, causal):
     q, k, v = (synth.normal_bf16((1, BH, n, 64), 196 + i) for i, n in enumerate((Sq, Skv, Skv)))
     got = from_dev(kernels.attention_prefill(to_dev(q), to_dev(k), to_dev(v), None, causal))
     _check(oracle, got, q, k, v, causal)
+
+
+# each variant of the built-in choice by name, with key splits of 1, even and odd
+# counts, and splits past the last step (25 steps in 8, 10 in 8)
+@pytest.mark.parametrize("BH,Sq,Sc,D,append,kernel,block_m,splits,inside", [
+    (7, 38, 64, 64, True, "FLASH", 128, 1, True), (5, 64, 64, 64, True, "FLASH", 128, 1, True),
+    (260, 66, 100, 64, False, "FLASH", 128, 1, False), (260, 70, 128, 64, True, "FLASH", 128, 1, True),
+    (90, 33, 4096, 64, True, "FLASH", 64, 2, True), (90, 33, 4097, 64, True, "FLASH", 64, 2, False),
+    (25, 9, 2900, 64, False, "FLASH_HALF", 64, 8, False), (40, 9, 2900, 64, False, "FLASH_HALF", 64, 6, False),
+    (2, 20, 1920, 64, True, "FLASH_HALF", 64, 8, True), (3, 40, 16384, 64, True, "FLASH_HALF", 64, 16, True),
+    (2, 70, 12352, 64, True, "FLASH_HALF", 64, 12, False), (270, 40, 200, 64, True, "FLASH_PAIR", 64, 1, False),
+    (3, 130, 832, 128, True, "FLASH", 128, 8, True), (3, 40, 8256, 128, True, "FLASH", 128, 16, True),
+    (20, 9, 2900, 128, True, "FLASH", 64, 8, False), (6, 4, 128, 64, False, "FLASH_HALF", 64, 1, False),
+    (6, 4, 130, 64, False, "DECODE", 4, 1, False), (40, 2, 900, 128, True, "DECODE", 2, 4, True)])
+def test_every_variant(gpu, oracle, BH, Sq, Sc, D, append, kernel, block_m, splits, inside):
+    import ctypes as C
+
+    from polykernel_amd import _lib, kernels
+
+    plan, fused = _lib.Plan(), C.c_int()
+    _lib.check(_lib.load().pk_attention_plan(BH, Sq, Sc, D, int(append), 1, C.byref(plan), C.byref(fused)),
+               "pk_attention_plan")
+    assert (plan.kernel, plan.block_m, plan.splits, bool(fused.value)) == (getattr(_lib, "PLAN_" + kernel), block_m,
+                                                                           splits, inside)
+    keys = Sc + Sq if append else Sc
+    print(f"variant {kernel} BH{BH} Sq{Sq} Sc{Sc} D{D} append={append}", flush=True)
+    q, kn, vn = (synth.normal_bf16((1, BH, Sq, D), 200 + i) for i in range(3))
+    kc, vc = (synth.normal_bf16((1, BH, keys, D), 203 + i) for i in range(2))
+    if append:
+        dk, dv = to_dev(kc), to_dev(vc)
+        got = from_dev(kernels.fused_kv_append_attention(to_dev(q), to_dev(kn), to_dev(vn), dk, dv, Sc))
+        for cache, new, dev in ((kc, kn, dk), (vc, vn, dv)):
+            cache[:, :, Sc:] = new
+            assert np.array_equal(from_dev(dev), cache)
+    else:
+        got = from_dev(kernels.attention_prefill(to_dev(q), to_dev(kc), to_dev(vc), None, True))
+    _check(oracle, got, q, kc, vc, True)

@@ -123,3 +123,34 @@ def test_few_queries_on_short_keys(S_q, S_cache, D, append, decode):
     """Three and four queries on up to 128 keys of D 64: flash 5.0 us, decode 5.9 (96 heads, 4 keys)."""
     assert (attention_plan(96, S_q, S_cache, D, append)[0].kernel == _lib.PLAN_DECODE) == decode
 
+
+# us of the variant that was taken before / of this one
+@pytest.mark.parametrize("BH,S_q,S_cache,append,causal,kernel,block_m,splits,inside", [
+    (141, 12, 9472, True, True, "FLASH", 64, 1, True),         # half ring 100 / full 71
+    (43, 160, 6656, True, True, "FLASH", 64, 1, True),         # 70.3 / 54.0
+    (16, 1021, 1021, False, True, "FLASH_HALF", 64, 1, False),  # 14.1 full / 13.2
+    (32, 333, 1200, True, True, "FLASH_HALF", 64, 1, False),    # 12 steps, six tiles of a head read the same keys
+    (7, 1995, 1995, False, False, "FLASH_HALF", 64, 1, False),  # 32.0 in two / 22.1
+    (108, 99, 2816, False, False, "FLASH", 64, 1, False),       # 34.8 half / 27.8
+    (7, 37, 64, True, True, "FLASH", 128, 1, True),             # 10.1 append first / 7.5
+    (1, 12, 64, True, True, "FLASH", 128, 1, True),             # 7.2 / 6.4
+    (1, 12, 192, True, True, "FLASH_HALF", 64, 1, False),       # 128 x 64 appending is 1.06 times as long
+    (449, 68, 73, False, True, "FLASH", 128, 1, False),         # pair 16.0 / 13.2
+    (466, 74, 128, True, True, "FLASH", 128, 1, True),          # 26.1 / 22.6
+    (128, 256, 2048, True, True, "FLASH_PAIR", 64, 1, False), (40, 1024, 1024, False, False, "FLASH_PAIR", 64, 1, False),
+    (64, 512, 512, False, True, "FLASH", 128, 1, False),
+    (64, 500, 64, True, True, "FLASH", 128, 1, True), (64, 500, 65, True, True, "FLASH_PAIR", 64, 1, False)])  # 21.8 / 19.5
+def test_flash_takes_the_faster_variant_at_64(BH, S_q, S_cache, append, causal, kernel, block_m, splits, inside):
+    p, fused = attention_plan(BH, S_q, S_cache, 64, append, causal)
+    assert (p.kernel, p.block_m, p.splits, fused) == (getattr(_lib, "PLAN_" + kernel), block_m, splits, inside)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_flash_splits_stay_in_one_round(D):
+    for BH, S_q, S_cache in ((1, 8, 1 << 17), (8, 500, 0), (16, 7, 1000), (12, 29, 3200), (8, 1000, 24), (40, 64, 8192),
+                             (200, 33, 8192), (1, 5, 1 << 20)):
+        p, _ = attention_plan(BH, S_q, S_cache, D)
+        tiles = BH * -(-S_q // p.block_m)
+        assert p.splits == 1 or (tiles * p.splits <= 256 and 2 * p.splits <= -(-(S_cache + S_q) // p.block_n))
+    assert attention_plan(16, 7, 1000, 128)[0].splits > 1 and attention_plan(12, 29, 3200, 128)[0].splits > 1
+    assert attention_plan(8, 500, 0, 128)[0].splits == 1       # 15.9 in four / 12.7
