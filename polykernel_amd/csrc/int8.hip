@@ -612,6 +612,12 @@ static int check_workspace(size_t need, size_t ws_bytes) {
   return PK_ERR_WORKSPACE;
 }
 
+static int check_workspace_alignment(const I8sPlan &plan, const void *ws) {
+  if (!plan.v || plan.splits <= 1 || aligned16(ws)) return PK_OK;
+  set_error("int8 matmul: workspace must be 16-byte aligned");
+  return PK_ERR_WORKSPACE;
+}
+
 static int use_workspace(size_t need, void *&ws, size_t ws_bytes, hipStream_t st, WorkspaceLease &lease) {
   if (need == 0) return PK_OK;
   if (ws == nullptr) {
@@ -676,8 +682,10 @@ int int8_run(int epi, const uint16_t *A, const int8_t *W, const float *scale, ui
     auto base = [&] {
       return i8s_plan(M, N, K, nullptr, device_cus(), plan) ? i8s_workspace(plan, M, N) : generic_workspace(M, N, K, nullptr);
     };
-    if (ws)
+    if (ws) {
       if (int rc = check_workspace(base(), ws_bytes)) return rc;
+      if (int rc = check_workspace_alignment(plan, ws)) return rc;
+    }
     // a caller's scratch as it is (launch_matmul_int8_noalloc's static buffer
     // is the cap for all, so that calls with and without it split alike),
     // library scratch as far as it can be had
@@ -688,6 +696,7 @@ int int8_run(int epi, const uint16_t *A, const int8_t *W, const float *scale, ui
       return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
     };
     WorkspaceLease lease;
+    // unaligned scratch that was taken (the column-split kernel uses none) holds no partials
     const size_t part = choose(ws ? (aligned16(ws) ? ws_bytes : 0) : kInt8ScratchBytes);
     float *partial = static_cast<float *>(ws);
     if (part && !ws) {
@@ -713,10 +722,7 @@ int int8_run(int epi, const uint16_t *A, const int8_t *W, const float *scale, ui
   if (fast) {
     int rc = use_workspace(i8s_workspace(plan, M, N), ws, ws_bytes, st, lease);
     if (rc) return rc;
-    if (plan.splits > 1 && !aligned16(ws)) {
-      set_error("int8 matmul: workspace must be 16-byte aligned");
-      return PK_ERR_WORKSPACE;
-    }
+    if (int rc = check_workspace_alignment(plan, ws)) return rc;
     I8sArgs a{A, W, scale, static_cast<float *>(ws), C, R, tab, M, N, K,
               plan.splits, plan.split_steps, plan.slices * plan.splits};
     plan.v->fn[epi](dim3(plan.slices * plan.splits, plan.mblocks), st, a);

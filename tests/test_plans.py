@@ -154,3 +154,13 @@ def test_flash_splits_stay_in_one_round(D):
         assert p.splits == 1 or (tiles * p.splits <= 256 and 2 * p.splits <= -(-(S_cache + S_q) // p.block_n))
     assert attention_plan(16, 7, 1000, 128)[0].splits > 1 and attention_plan(12, 29, 3200, 128)[0].splits > 1
     assert attention_plan(8, 500, 0, 128)[0].splits == 1       # 15.9 in four / 12.7
+
+
+@pytest.mark.parametrize("M,N,Kd", [(16, 4096, 8192), (1, 4096, 4096), (16, 28672, 8192), (300, 4096, 4096)])
+def test_int8_refuses_unaligned_scratch_where_the_column_kernel_splits(M, N, Kd):
+    """Scratch that is refused stays refused whichever kernel the product takes
+    (nothing is launched: the addresses are made up)."""
+    lib, cfg, at = _lib.load(), _lib.Config(), 1 << 20
+    assert lib.pk_int8_default_config(M, N, Kd, cfg) == 0 and cfg.block_k < Kd
+    for ws, size in ((at + 8, 1 << 28), (at, 64)):
+        assert lib.pk_matmul_int8_ex(0, at, at, at, at, None, M, N, Kd, None, ws, size, None) == _lib.PK_ERR_WORKSPACE
