@@ -355,7 +355,9 @@ LaunchFn CodeObjectPanelLauncher(std::shared_ptr<ModuleTable> table) {
       return ModuleLaunch(mod->fns[0], tiles, 1, (unsigned)PK_PANEL_THREADS, p->stream, a, "pk_panel", error,
                           pk_panel_lds_bytes(p->K));
     }
-    // GEMM config: the row normalisation, then the plain GEMM
+    // GEMM config: the row normalisation, then the plain GEMM.  The config's operand
+    // checks hold whichever kernel forms the product: what is taken does not depend
+    // on the built-in choice for the shape.
     const bool dma = c.block_k == 32;
     if ((dma || c.vector_width == 8) && !Aligned16(p->W)) {
       error = "code-object GEMM config {" + autotune::ToString(c) + "} needs a 16-byte aligned W";

@@ -57,8 +57,12 @@ ROW_ROWS, ROW_COLS = 37, (512, 1024, 2048, 4096, 8192, 16384, 32768, 65536, 7000
 # RMSNorm -> MatMul: the whole-K panel (ragged M) and the RMSNorm-into-
 # workspace path followed by a GEMM (K 1536 and 2048); at K 64 the panel
 # (64 x 256), and the 64-deep GEMM configs whose block_k equals K: N % 8 != 0
-# (no panel) and more than 256 panel tiles (33 x 8)
-PANEL_SHAPES = ((40, 136, 768), (64, 256, 1536), (72, 264, 2048), (64, 256, 64), (40, 1001, 64), (1056, 512, 64))
+# (no panel) and more than 256 panel tiles (33 x 8).  The launcher forms the
+# product with the library's kernel where the built-in choice is no configuration,
+# so two of these shapes take a tile there and launch the object's own pk_gemm:
+# (1056, 512, 64) and, with N % 8 != 0, (72, 1001, 64)
+PANEL_SHAPES = ((40, 136, 768), (64, 256, 1536), (72, 264, 2048), (64, 256, 64), (40, 1001, 64), (72, 1001, 64),
+                (1056, 512, 64))
 
 
 def conformance_entries() -> list:

@@ -668,7 +668,10 @@ def test_conformance_code_objects_bit_identical(gpu, oracle):
     residual + RMSNorm and masked softmax; the RMSNorm -> MatMul panels and
     long-row path; attention), served from its code object, equals the
     linked kernel at the same configuration bit for bit (ragged M and N
-    tiles; null bias for the residual op included) and matches the oracle."""
+    tiles; null bias for the residual op included) and matches the oracle.
+    RMSNorm -> MatMul compares with the built-in choice instead: where that is
+    no configuration, both run the library's kernel behind the object's row
+    kernel, and elsewhere the object's pk_gemm."""
     import torch
 
     from polykernel_amd import emit

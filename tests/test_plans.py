@@ -57,6 +57,16 @@ def test_few_rows_take_the_faster_kernel(epi, M, N, Kd, plan):
     assert (p.kernel, p.block_m, p.block_n) == plan
 
 
+def test_conformance_objects_launch_their_own_gemm():
+    """A served RMSNorm -> MatMul call launches the object's pk_gemm only where the
+    built-in choice is a tile; the conformance set holds one such shape per staging."""
+    from polykernel_amd import emit
+
+    tiles = [s for s in emit.PANEL_SHAPES
+             if all(gemm_plan(*s, scratch=n).kernel == _lib.PLAN_TILE for n in (0, 64 << 20))]
+    assert {s[1] % 8 == 0 for s in tiles} == {True, False}
+
+
 @pytest.mark.parametrize("M,N,Kd,odd", [(1, 50257, 8, True), (32, 50257, 8, True), (33, 50257, 56, False),
                                         (33, 50257, 64, True), (64, 8191, 8, True), (65, 50257, 64, False)])
 def test_odd_rows_take_the_faster_kernel(M, N, Kd, odd):
