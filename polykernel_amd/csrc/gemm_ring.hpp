@@ -24,9 +24,10 @@
 // 8192, 2048] 22.6 / 34.2, [501, 2048, 8192] 28.9 / 73.8 (K split in 4), [777,
 // 12288, 4096] 73.6 / 87, [1024, 4096, 4096] 37.0 / 60.5, [128, 4096, 4096]
 // 15.2 / 38.9, [1278, 16128, 4032] 148 / 201.  Timing-only builds of the 128 x
-// 128 tile at [1024, 4096, 4096]: MFMA alone 25.7, loads alone 28.7 (26 TB/s
-// from L2), all 37.6, so the two overlap by about 60 %; 7.9 of it is launch,
-// first loads and epilogue.
+// 128 tile at [1024, 4096, 4096]: MFMA alone 25.7, loads alone 28.7, all 37.6, each
+// with 7.9 of launch, first loads and epilogue.  Without those the tiles' 537 MB
+// come at 26 TB/s, and half of the MFMA time runs beside them.  Counters: MFMA busy
+// on 37 % of the cycles there, 50 % at [777, 12288, 4096], no bank conflicts.
 //
 // Like the streaming kernel it can split K over workgroups (fp32 partials,
 // gemm_reduce_body, or int8_stream.hpp's reduction).  Needs K % 8 == 0, N % 8 == 0, 16-byte aligned A and B;

@@ -385,16 +385,16 @@ __device__ __forceinline__ void stream_body(const I8sArgs &g) {
 }
 
 // ---------------------------------------------------------------------------
-// The same stream with K split over the waves (up to 32 rows; what
-// launch_matmul_int8 and the decode chain run unless a configuration asks for
-// stream_body).  A workgroup owns a slice of 16*NT columns and one K split; its
+// The same stream with K split over the waves (the built-in choice up to 32 rows and
+// 100 MB of weights; above, and where a configuration asks for it, stream_body
+// runs).  A workgroup owns a slice of 16*NT columns and one K split; its
 // WK waves take the 64-row steps w, w + WK, ... of the split through private
 // rings, add their tiles in LDS and finish in place, so that a slice count
 // near the CU count needs no split partials and no second launch at all --
 // stream_body's waves split the slice by columns and leave 4-14 partials per
-// output to a reduction of 4-5 us.  Few waves and a short ring (2 waves of 2-3
-// stages) stream faster than many: the fewer rows of the matrix are in flight,
-// the more of them fall into open DRAM pages.  W and A stages, transpose reads
+// output to a reduction of 4-5 us.  Four waves and a short ring (2 stages
+// of the widest slices, 4 of the narrowest) stream faster than more: the fewer rows
+// of the matrix are in flight, the more of them fall into open DRAM pages.  W and A stages, transpose reads
 // and widening as in stream_body; K % 8 == 0 (the last step's missing rows are
 // zeroed in A's fragments), N % 16 == 0, 16-byte aligned operands.
 // ---------------------------------------------------------------------------

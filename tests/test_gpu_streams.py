@@ -12,6 +12,7 @@
 """
 from __future__ import annotations
 
+import ctypes as C
 import threading
 
 import numpy as np
@@ -51,6 +52,16 @@ def _run_thread(fn, iters, results, idx, errors, stream):
         errors.append(e)
 
 
+def _int8_splits(M=16, N=4096, Kd=8192):
+    """Splits of the kernel the call runs (default_config names a configuration,
+    and few rows run a kernel that is none)."""
+    from polykernel_amd import _lib
+
+    p = _lib.Plan()
+    _lib.check(_lib.load().pk_int8_plan(M, N, Kd, 16 << 20, C.byref(p)), "pk_int8_plan")
+    return p.splits
+
+
 def test_split_workspaces_concurrent_streams(gpu):
     import torch
 
@@ -58,6 +69,7 @@ def test_split_workspaces_concurrent_streams(gpu):
 
     cfg = rt.default_config("matmul_int8", 16, 4096, 8192)
     assert cfg["block_k"] < 8192, f"expected a split-K plan, got {cfg}"
+    assert _int8_splits() > 1
     i8 = [_int8_case(10 + j) for j in range(3)]
     att = [_att_case(20 + 3 * j) for j in range(3)]
     scale = 1.0 / np.sqrt(128)
@@ -90,6 +102,7 @@ def test_split_workspace_one_stream_two_threads(gpu):
 
     from polykernel_amd import kernels
 
+    assert _int8_splits() > 1
     cases = [_int8_case(40 + j) for j in range(4)]
     want = [from_dev(kernels.matmul_int8(*c)) for c in cases]
     torch.cuda.synchronize()
@@ -182,7 +195,7 @@ def test_release_workspace_and_per_thread_stream(gpu):
     from polykernel_amd import runtime as rt
 
     lib = _lib.load()
-    assert rt.default_config("matmul_int8", 16, 4096, 8192)["block_k"] < 8192
+    assert rt.default_config("matmul_int8", 16, 4096, 8192)["block_k"] < 8192 and _int8_splits() > 1
     a, wq, s = _int8_case(7)
     want = from_dev(kernels.matmul_int8(a, wq, s))
     for rnd in range(3):
