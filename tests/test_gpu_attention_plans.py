@@ -99,7 +99,7 @@ def test_flash_d64_rings(gpu, oracle, BH, Sq, Skv, causal):
     (2, 70, 12352, 64, True, "FLASH_HALF", 64, 12, False), (270, 40, 200, 64, True, "FLASH_PAIR", 64, 1, False),
     (3, 130, 832, 128, True, "FLASH", 128, 8, True), (3, 40, 8256, 128, True, "FLASH", 128, 16, True),
     (20, 9, 2900, 128, True, "FLASH", 64, 8, False), (6, 4, 128, 64, False, "FLASH_HALF", 64, 1, False),
-    (6, 4, 130, 64, False, "DECODE", 4, 1, False), (40, 2, 900, 128, True, "DECODE", 2, 4, True)])
+    (6, 4, 130, 64, False, "DECODE", 4, 1, False), (40, 2, 900, 128, True, "DECODE", 2, 2, True)])
 def test_every_variant(gpu, oracle, BH, Sq, Sc, D, append, kernel, block_m, splits, inside):
     import ctypes as C
 

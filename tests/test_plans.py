@@ -119,6 +119,7 @@ def attention_plan(BH, S_q, S_cache, D, append=True, causal=True):
     (160, 1, 4096, 64, False, 1),    # 38 in two rounds / 31
     (100, 4, 4096, 64, False, 2),    # 32 in 4 / 26
     (8, 1, 16384, 128, False, 16), (1, 1, 1 << 20, 128, False, 16),
+    (100, 1, 509, 128, True, 1), (100, 2, 1021, 64, True, 1),   # 10.2 in two / 8.6, 11.3 / 10.1
     (32, 1, 256, 128, True, 1), (32, 4, 2048, 128, True, 8), (1, 2, 8, 128, True, 1), (300, 1, 1 << 16, 64, True, 1)])
 def test_decode_splits(BH, S_q, S_cache, D, append, splits):
     p, fused = attention_plan(BH, S_q, S_cache, D, append)
