@@ -346,16 +346,23 @@ constexpr size_t kInt8ScratchBytes = size_t(16) << 20;
 // kernel, us of those / here.  Its fixed cost is 4.9 against 2.9 and 2.7, so it
 // needs weights to read: `work` bytes, once for each 64 rows, as the stream does
 // ([53, 1024, 56] 3.0 / 4.9, [44, 512, 368] 4.1 / 6.8, [39, 8192, 64] 3.5 / 5.0;
-// [224, 2800, 184] generic 5.3 / 6.1).  Up to 128 columns the stream has no wide
-// slice ([108, 128, 512] 17.1 / 7.6).  Few tiles over a long K are split in 8 at
-// most, the others in 16 and more ([35, 688, 27968] 23 / 30, [66, 48, 27144]
-// generic 13 / 29, [150, 192, 16384] 17 / 21).
+// [224, 2800, 184] generic 5.3 / 6.1), and at one or two k-steps rounds that are
+// nearly full at one ([160, 36848, 64] 10.9 / 17.1 in 1.1 rounds, [43, 30000, 64] 7.2 / 5.6 in
+// 0.9).  Up to 128 columns the stream has no wide slice ([108, 128, 512] 17.1 / 7.6).
+// Few tiles over a long K are split in 8 at most, the others in 16 and more ([35,
+// 688, 27968] 23 / 30, [66, 48, 27144] generic 13 / 29, [150, 192, 16384] 17 / 21; more
+// than 128 rows of up to 128 columns [556, 128, 8576] 20.3 / 16.0).  17000 products of whole
+// steps: 392 take over 4 % longer than in the other kernel, 172 would be shorter in this.
 bool i8_ring_pays(int M, int N, int K, const RingChoice &p) {
   const double work = (double)((M + 63) / 64) * N * K;
   if (K % I8S_KSTEP != 0)
     return p.units > 128 ? p.units > 180 || work > 1.4e6 : (double)M * N * K > 2e8 && (int64_t)M * N > 50000;
-  if (p.splits >= 8 && p.units <= 72 && K > (p.units <= 40 ? 4096 : 8192)) return false;
-  return N <= 128 || !((work <= 1.3e6 && K <= 256) || (work <= 3e6 && K <= 128));
+  const double fill = p.units / (256.0 * ((p.units + 255) / 256));
+  if (p.splits >= 8 && p.units <= 72 && K > (p.units <= 40 ? 4096 : 8192)) return N <= 128 && M > 128;
+  if (N <= 128 || K > 256) return true;
+  if (K <= 128)
+    return work > (K <= 64 ? 3.6e6 : 3e6) ? K > 64 || p.units <= 256 || fill >= 0.66 : fill > 0.88 && M <= 128;
+  return work > 1.3e6 || fill > 0.66 || (N > 1032 && (int64_t)M * N > 75000);
 }
 RingChoice i8_ring_plan(int M, int N, int K, size_t scratch) {
   if (M <= kI8RingRows) return RingChoice{};

@@ -87,6 +87,14 @@ def test_int8_takes_the_faster_kernel(M, N, Kd, kernel):
     assert int8_plan(M, N, Kd).kernel == kernel
 
 
+# one or two k-steps: rounds that are nearly full; up to 128 columns; few tiles over a long K
+@pytest.mark.parametrize("M,N,Kd,ring", [
+    (160, 36848, 64, False), (43, 30000, 64, True), (1529, 1984, 64, False), (300, 30000, 64, True),   # 10.9 / 17.1, 7.2 / 5.6
+    (556, 128, 8576, True), (120, 400, 23624, False), (60, 128, 8576, False)])                         # 20.3 / 16.0
+def test_int8_ring_at_short_k(M, N, Kd, ring):
+    assert (int8_plan(M, N, Kd).kernel == _lib.PLAN_RING) == ring
+
+
 # weights above 32 MB whose rows are a multiple of 1024 bytes: full rounds of workgroups
 @pytest.mark.parametrize("M,N,Kd", [(1, 5120, 16384), (1, 3072, 22784), (16, 8192, 8192), (8, 4096, 18944), (1, 20480, 4352),
                                     (16, 6144, 14592), (1, 12288, 7296)])
