@@ -238,13 +238,18 @@ int softmax_run(const RowArgs &a, const pk_config &c, hipStream_t st) {
 // Few short rows stay with the generic kernel too, whose 256 threads hold one
 // element of a row each, or a few, where a wave here has a chain of eight and
 // more: us in a replayed graph with a mask, generic / ragged, [64, 33] 2.6 / 3.8,
-// [1000, 33] 3.0 / 3.7, [2000, 65] 3.9 / 3.9; [512, 300] 3.5 / 3.7; [256, 700] 4.0 /
-// 4.4, [512, 1021] 5.8 / 5.6; [256, 1021] 4.7 / 5.2, [256, 1300] 6.0 / 5.4; [64, 2047] 6.2 / 3.9.
+// [1000, 33] 3.0 / 3.7, [2090, 23] 3.8 / 4.5, [2000, 65] 3.9 / 3.9; [512, 300] 3.5 / 3.7;
+// [256, 700] 4.0 / 4.4, [655, 555] 3.9 / 4.5, [512, 1021] 5.8 / 5.6; [256, 1021] 4.7 / 5.2,
+// [256, 1300] 6.0 / 5.4; [64, 2047] 6.2 / 3.9.
 bool softmax_few_rows(int rows, int cols) {
-  return rows <= (cols <= 256    ? 1536
+  return rows <= (cols <= 16     ? 1536
+                  : cols <= 64   ? 2200
+                  : cols <= 128  ? 1900
+                  : cols <= 256  ? 1600
                   : cols <= 505  ? 640
-                  : cols <= 700  ? 512
-                  : cols <= 1009 ? 320
+                  : cols <= 600  ? 800
+                  : cols <= 700  ? 640
+                  : cols <= 1150 ? 320
                   : cols <= 1280 ? 256
                                  : 0);
 }

@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 # waves or vectors per lane (498 ... 32754 columns), and row counts that leave
 # the last chunk of the tensor short or whole; up to 1280 columns with few rows
 # (the generic kernel) and with more (the ragged one)
-@pytest.mark.parametrize("rows,cols", [(1537, 1), (1539, 3), (1544, 9), (2001, 255), (643, 497), (645, 499), (517, 699),
+@pytest.mark.parametrize("rows,cols", [(1537, 1), (1539, 3), (1544, 9), (2203, 33), (1903, 101), (2001, 255),
+                                       (643, 497), (645, 499), (805, 555), (643, 699),
                                        (323, 1009), (325, 1011), (257, 1279), (1, 1), (5, 3), (8, 9), (3, 497), (6, 499), (7, 1009), (5, 1011), (4, 1521),
                                        (5, 1523), (9, 2033), (5, 2035), (3, 4081), (3, 4083), (5, 8177), (3, 8179),
                                        (3, 16369), (3, 16371), (3, 32753), (2, 32755), (97, 1021)])
@@ -34,7 +35,7 @@ def test_softmax_ragged_rows(gpu, oracle, rows, cols):
         assert rep.max_ulp <= 1 and (1 - rep.bit_exact) * want.size <= max(2, 0.02 * want.size), rep
 
 
-@pytest.mark.parametrize("rows", [9, 263])  # the generic kernel, the ragged one
+@pytest.mark.parametrize("rows", [9, 327])  # the generic kernel, the ragged one
 def test_softmax_ragged_neighbour_rows_do_not_mix(gpu, oracle, rows):
     """A row of infinities or NaN between ordinary rows, and a fully masked row:
     only that row's outputs are affected, although its neighbours read its elements."""

@@ -107,6 +107,7 @@ def test_int8_stream_fills_its_rounds(M, N, Kd):
 # us of the generic / the ragged kernel: 2.6 / 3.8, 3.0 / 3.7, 3.5 / 3.7, 4.0 / 4.4, 4.7 / 5.2, then the other way
 @pytest.mark.parametrize("rows,cols,ragged", [
     (64, 33, False), (1000, 33, False), (512, 300, False), (256, 700, False), (256, 1021, False), (4000, 33, True),
+    (2090, 23, False), (2400, 23, True), (655, 555, False), (900, 555, True),   # 3.8 / 4.5, 3.9 / 4.5
     (1000, 300, True), (512, 1021, True), (64, 2047, True), (1, 32753, True), (16336, 1021, True), (16336, 1024, False),
     (1, 32755, False)])
 def test_softmax_takes_the_faster_kernel(rows, cols, ragged):
