@@ -290,15 +290,16 @@ struct FaChoice {
 // the rows it reads back, within one round of 256 workgroups.  16 heads of 7 on
 // 1000 cached keys at D 128 19.5 -> 14.6 us, 12 of 29 on 3200 26.1 -> 20.6; D 64, 7
 // heads of 1995 22.1 unsplit, 32.0 in 2; 108 of 99 on 2816 27.8 and 39.8.  More than
-// 8 keep 8 steps each, since the merge reads them one after the other (4 heads of 16
-// on 8192 keys 18.3 us in 8, 19.8 in 16).  A configuration keeps split_count's.
+// 8 keep 5 steps each, since the merge reads them one after the other (D 64, 4 heads
+// of 16 on 8192 keys 18.3 us in 8, 19.8 in 16; D 128, 6 of 5 on 11328 29.2 and 24.4).
+// A configuration keeps split_count's.
 int fa_splits(int64_t tiles, int steps, int64_t rows, int D) {
   const double step_us = D == 128 ? 1.3 : 0.85, fill_us = D == 128 ? 0.37 : 0.39;
   const double row_us = D == 128 ? 0.25e-3 : 0.07e-3;
   int best = 1;
   double best_us = steps * (step_us + fill_us * tiles / 256);
   for (int s : {2, 3, 4, 6, 8, 12, 16}) {
-    if (tiles * s > 256 || (s > 8 ? 8 : 2) * s > steps) break;
+    if (tiles * s > 256 || (s <= 8 ? s >= steps : 5 * s > steps)) break;
     const double us = (steps + s - 1) / s * (step_us + fill_us * tiles * s / 256) + 2.7 + s * (0.1 + row_us * rows);
     if (us < best_us) {
       best_us = us;

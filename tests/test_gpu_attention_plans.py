@@ -96,7 +96,7 @@ def test_flash_d64_rings(gpu, oracle, BH, Sq, Skv, causal):
     (90, 33, 4096, 64, True, "FLASH", 64, 2, True), (90, 33, 4097, 64, True, "FLASH", 64, 2, False),
     (25, 9, 2900, 64, False, "FLASH_HALF", 64, 8, False), (40, 9, 2900, 64, False, "FLASH_HALF", 64, 6, False),
     (2, 20, 1920, 64, True, "FLASH_HALF", 64, 8, True), (3, 40, 16384, 64, True, "FLASH_HALF", 64, 16, True),
-    (2, 70, 12352, 64, True, "FLASH_HALF", 64, 12, False), (270, 40, 200, 64, True, "FLASH_PAIR", 64, 1, False),
+    (2, 70, 8256, 64, True, "FLASH_HALF", 64, 12, False), (270, 40, 200, 64, True, "FLASH_PAIR", 64, 1, False),
     (3, 130, 832, 128, True, "FLASH", 128, 8, True), (3, 40, 8256, 128, True, "FLASH", 128, 16, True),
     (20, 9, 2900, 128, True, "FLASH", 64, 8, False), (6, 4, 128, 64, False, "FLASH_HALF", 64, 1, False),
     (6, 4, 130, 64, False, "DECODE", 4, 1, False), (40, 2, 900, 128, True, "DECODE", 2, 2, True)])
