@@ -89,7 +89,8 @@ def test_flash_d64_rings(gpu, oracle, BH, Sq, Skv, causal):
 
 
 # each variant of the built-in choice by name, with key splits of 1, even and odd
-# counts, and splits past the last step (25 steps in 8, 10 in 8)
+# counts, and splits past the last step (25 steps in 8, 10 in 8) or batch (97 and 121
+# in 12)
 @pytest.mark.parametrize("BH,Sq,Sc,D,append,kernel,block_m,splits,inside", [
     (7, 38, 64, 64, True, "FLASH", 128, 1, True), (5, 64, 64, 64, True, "FLASH", 128, 1, True),
     (260, 66, 100, 64, False, "FLASH", 128, 1, False), (260, 70, 128, 64, True, "FLASH", 128, 1, True),
@@ -99,7 +100,8 @@ def test_flash_d64_rings(gpu, oracle, BH, Sq, Skv, causal):
     (2, 70, 8256, 64, True, "FLASH_HALF", 64, 12, False), (270, 40, 200, 64, True, "FLASH_PAIR", 64, 1, False),
     (3, 130, 832, 128, True, "FLASH", 128, 8, True), (3, 40, 8256, 128, True, "FLASH", 128, 16, True),
     (20, 9, 2900, 128, True, "FLASH", 64, 8, False), (6, 4, 128, 64, False, "FLASH_HALF", 64, 1, False),
-    (6, 4, 130, 64, False, "DECODE", 4, 1, False), (40, 2, 900, 128, True, "DECODE", 2, 2, True)])
+    (6, 4, 130, 64, False, "DECODE", 4, 1, False), (40, 2, 900, 128, True, "DECODE", 2, 2, True),
+    (2, 4, 3100, 128, True, "DECODE", 4, 12, True), (2, 4, 7740, 64, True, "DECODE", 4, 12, True)])
 def test_every_variant(gpu, oracle, BH, Sq, Sc, D, append, kernel, block_m, splits, inside):
     import ctypes as C
 
